@@ -800,19 +800,15 @@ static int cnab2_call(gd_cnab2_mats *M, int lmax, int mmax, int nr, int mode, co
             }
         }
     }
-    GD_TRY(zero_status(ctx, M->status));
     GD_TRY(gd_launch_cnab2_lmajor(ctx->stream, M->L.as<double>(), M->LU.as<double>(), M->lmax + 1, lmax, mmax, nr,
-                                  M->bw, M->dt, M->theta, mode, M->bc_rows, a, b, c, d, e, f, oa, ob,
-                                  M->status.as<int>()));
-    int st = 0;
-    GD_TRY(read_status(ctx, M->status, &st));
+                                  M->bw, M->dt, M->theta, mode, M->bc_rows, a, b, c, d, e, f, oa, ob));
     if (flags & GD_HOST) {
         double *ha = (mode == 2) ? const_cast<double *>(u_re) : o_re;
         double *hb = (mode == 2) ? const_cast<double *>(u_im) : o_im;
         GD_TRY(gd_from_device(ctx, ha, oa, sizeof(double) * n));
         GD_TRY(gd_from_device(ctx, hb, ob, sizeof(double) * n));
     }
-    GD_CHECK(!(st & 4), GD_ERR_MISSING_L, "Missing implicit matrix for l > %d", M->lmax);
+    GD_CHECK(mode == 1 || lmax <= M->lmax, GD_ERR_MISSING_L, "Missing implicit matrix for l > %d", M->lmax);
     return GD_OK;
 }
 

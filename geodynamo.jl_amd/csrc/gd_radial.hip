@@ -4,9 +4,9 @@
 //   * band solve (solve_banded!, linear_algebra.jl:59-88)
 //   * CNAB2 operator assembly per l (create_shtns_timestepping_matrices,
 //     timestep.jl:498-543)
-//   * rhs / solve / fused rhs+solve in the reference l-major layout, one
-//     wavefront per l with L_l and LU(S_l) in LDS (build_rhs_cnab2!,
-//     solve_implicit_step!, timestep.jl:610-730)
+//   * rhs / solve / fused rhs+solve in the reference l-major layout, column
+//     tiles of one l in LDS (build_rhs_cnab2!, solve_implicit_step!,
+//     timestep.jl:610-730)
 #include "gd_internal.hpp"
 #include "gd_radial.hpp"
 
@@ -126,103 +126,246 @@ int gd_cnab2_build(hipStream_t st, const double *d_lap, const double *d_rinv2, d
 }
 
 // ---------------------------------------------------------------- l-major CNAB2 (reference layout)
-// One block (64 lanes) per l; columns (m, re/im) of that l are spread over the
-// lanes; L_l and LU_l are staged in LDS.  mode: 0 rhs only, 1 solve only,
-// 2 fused rhs+solve in place on u.
-__global__ void __launch_bounds__(64) cnab2_lmajor_kernel(
-    const double *__restrict__ Lall, const double *__restrict__ LUall, int nl_mats, int lmax, int mmax, int n,
-    int bw, int nlm, double dt, double theta, int mode, int bc_rows, const double *u_re, const double *u_im,
-    const double *__restrict__ nl_re, const double *__restrict__ nl_im, const double *__restrict__ np_re,
-    const double *__restrict__ np_im, double *out_re, double *out_im, int *__restrict__ status)
+// mode: 0 rhs only, 1 solve only, 2 fused rhs + solve in place on u.
+//
+// One block per (l, 2^ctl columns (m, re/im) of that l).  Every row of the
+// block's columns is brought into LDS in one batch of coalesced loads (the
+// threads take rows in turn, columns fastest), the rhs -- a band stencil, no
+// recurrence -- is formed by all threads from that tile, and the two
+// substitutions run from LDS, one lane per column, with the row's
+// coefficients (uniform over the block: one l) as LDS broadcasts and the
+// next D rows read while D rows are computed.  Bound by HBM latency plus the
+// 2n dependent FP64 rows: at lmax=127, nr=65, bw=3 a lane that walked its
+// column through global memory (one wavefront per l) waited on memory at
+// every row, 306 us a launch (rhs 287, solve 324) against 10 us for the bytes
+// of both; rhs and solve calls together 673 -> 30 us.  The missing-l error
+// is decided from the sizes on the host, so no status word is cleared and
+// read back around the launch.
+struct CnabLArgs {
+    const double *L, *LU;
+    int nl_mats, lmax, mmax, n, nlm, bc_rows, ctl;
+    double inv_dt, lw;
+    const double *u[2], *nl[2], *np[2];
+    double *out[2];
+};
+constexpr int CNABL_THREADS = 512;
+constexpr int CNABL_UR = 9; // rows a thread loads in one batch: every row up to n = 72 at 64 columns
+
+static size_t cnabl_lds(int n, int bw, int mode, int ctl)
 {
-    extern __shared__ double sm[];
-    const int l = blockIdx.x;
     const int w = 2 * bw + 1;
+    return sizeof(double) * (size_t)n * (((mode == 2 ? 2 : 1) << ctl) + (mode == 2 ? 2 : 1) * w);
+}
+
+template <int BW, int MODE> __global__ void __launch_bounds__(CNABL_THREADS) cnab2_lmajor_kernel(CnabLArgs a)
+{
+    constexpr int W = 2 * BW + 1, UR = CNABL_UR, D = 4;
+    extern __shared__ double sm[];
+    const int l = a.lmax - (int)blockIdx.y; // the widest l first
+    const int n = a.n, nlm = a.nlm, mmax = a.mmax, ctl = a.ctl;
     const int ml = l < mmax ? l : mmax;
+    const int ncol = 2 * (ml + 1), c0 = (int)blockIdx.x << ctl;
+    // a missing l is an error of the rhs (timestep.jl:646), reported by the
+    // caller; solve_implicit_step! skips it (timestep.jl:709)
+    if (c0 >= ncol || l >= a.nl_mats) return;
     const int lm0 = l <= mmax ? l * (l + 1) / 2 : (mmax + 1) * (mmax + 2) / 2 + (l - mmax - 1) * (mmax + 1);
-    if (l >= nl_mats) {
-        // build_rhs_cnab2! errors on a missing l (timestep.jl:646);
-        // solve_implicit_step! skips it (timestep.jl:709)
-        if (mode != 1 && threadIdx.x == 0) atomicOr(status, 4);
-        return;
+    const int tid = threadIdx.x;
+    // rows 0 .. n-1 of the tile: T holds u (modes 0, 2) or the rhs (mode 1),
+    // X the system being solved; row i of the coefficients:
+    //   sL[i W + q] = L(i, i - BW + q)
+    //   sU[i W + q], q < BW: the L factor (i, i - BW + q); q = BW + p: U(i, i + 1 + p); q = 2 BW: 1 / U(i, i)
+    double *T = sm, *X = MODE == 2 ? T + ((size_t)n << ctl) : T;
+    double *sL = X + ((size_t)n << ctl), *sU = MODE == 2 ? sL + W * n : sL;
+    const int c = tid & ((1 << ctl) - 1), w0 = tid >> ctl, rs = CNABL_THREADS >> ctl; // column, first row, row step
+    const int cc = min(c0 + c, ncol - 1), ri = cc > ml, m = cc - (ri ? ml + 1 : 0);
+    const size_t base = (size_t)lm0 + m;
+    const double *u = a.u[ri] + base;
+    double nlv[UR], npv[UR];
+    auto nload = [&](int k0) {
+#pragma unroll
+        for (int k = 0; k < UR; ++k) {
+            const size_t o = (size_t)nlm * min(w0 + (k0 + k) * rs, n - 1);
+            nlv[k] = a.nl[ri][base + o];
+            npv[k] = a.np[ri][base + o];
+        }
+    };
+    for (int k0 = 0; k0 * rs < n; k0 += UR) {
+        double v[UR];
+#pragma unroll
+        for (int k = 0; k < UR; ++k) v[k] = u[(size_t)nlm * min(w0 + (k0 + k) * rs, n - 1)];
+        if (MODE != 1 && k0 == 0) nload(0); // in flight with the tile
+#pragma unroll
+        for (int k = 0; k < UR; ++k)
+            if (w0 + (k0 + k) * rs < n) T[((size_t)(w0 + (k0 + k) * rs) << ctl) + c] = v[k];
     }
-    double *sL = sm, *sLU = sm + w * n;
-    for (int q = threadIdx.x; q < w * n; q += 64) {
-        sL[q] = Lall[(size_t)l * w * n + q];
-        sLU[q] = LUall[(size_t)l * w * n + q];
+    const double *Lb = a.L + (size_t)l * W * n, *LUb = a.LU + (size_t)l * W * n;
+    for (int e = tid; e < W * n; e += CNABL_THREADS) {
+        const int i = e / W, q = e - i * W;
+        if (MODE != 1) {
+            const int j = i - BW + q;
+            sL[e] = (j >= 0 && j < n) ? Lb[BANDIDX(BW, BW + i - j, j)] : 0.0;
+        }
+        if (MODE != 0) {
+            const int j = q < BW ? i - BW + q : (q < 2 * BW ? i + 1 + q - BW : i);
+            const double v = (j >= 0 && j < n) ? LUb[BANDIDX(BW, BW + i - j, j)] : 0.0;
+            sU[e] = q == 2 * BW ? 1.0 / v : v;
+        }
     }
     __syncthreads();
-    const double inv_dt = 1.0 / dt, lw = 1.0 - theta;
-    const int ncol = 2 * (ml + 1);
-    for (int c = threadIdx.x; c < ncol; c += 64) {
-        const int reim = c / (ml + 1), m = c % (ml + 1);
-        const size_t base = (size_t)lm0 + m;
-        const double *u = reim ? u_im : u_re;
-        const double *nlv = reim ? nl_im : nl_re;
-        const double *npv = reim ? np_im : np_re;
-        double *o = reim ? out_im : out_re;
-        if (mode == 0 || mode == 2) {
-            // rhs, and for the fused mode the forward substitution on the fly;
-            // a window of original u keeps in-place updates safe.
-            double win[16];
-            for (int q = 0; q < 2 * bw + 1; ++q) {
-                int j = q - bw;
-                win[q] = (j >= 0 && j < n) ? u[base + (size_t)nlm * j] : 0.0;
-            }
-            for (int i = 0; i < n; ++i) {
-                double lin = 0.0;
-                if (lw != 0.0) {
-                    int j0 = i - bw < 0 ? 0 : i - bw, j1 = i + bw > n - 1 ? n - 1 : i + bw;
-                    for (int j = j0; j <= j1; ++j) lin += sL[BANDIDX(bw, bw + i - j, j)] * win[j - i + bw];
+    if (MODE != 1) {
+        for (int k0 = 0; k0 * rs < n; k0 += UR) {
+#pragma unroll
+            for (int k = 0; k < UR; ++k) {
+                const int i = w0 + (k0 + k) * rs;
+                if (i >= n) break;
+                const double *col = T + c;
+                double v = a.inv_dt * col[(size_t)i << ctl] + 1.5 * nlv[k] - 0.5 * npv[k];
+                if (a.lw != 0.0) {
+                    double lin = 0.0;
+#pragma unroll
+                    for (int q = 0; q < W; ++q) {
+                        const int j = i - BW + q;
+                        if (j >= 0 && j < n) lin += sL[i * W + q] * col[(size_t)j << ctl];
+                    }
+                    v += a.lw * lin;
                 }
-                const size_t oi = base + (size_t)nlm * i;
-                double v = inv_dt * win[bw] + 1.5 * nlv[oi] - 0.5 * npv[oi];
-                if (lw != 0.0) v += lw * lin;
-                if (bc_rows && (i == 0 || i == n - 1)) v = 0.0; // Dirichlet value
-                if (mode == 2) {
-                    double acc = 0.0;
-                    int j0 = i - bw < 0 ? 0 : i - bw;
-                    for (int j = j0; j < i; ++j) acc += sLU[BANDIDX(bw, bw + i - j, j)] * o[base + (size_t)nlm * j];
-                    v = v - acc;
-                }
-                // shift window before overwriting (o may alias u)
-                for (int q = 0; q < 2 * bw; ++q) win[q] = win[q + 1];
-                int jn = i + bw + 1;
-                win[2 * bw] = (jn < n) ? u[base + (size_t)nlm * jn] : 0.0;
-                o[oi] = v;
+                if (a.bc_rows && (i == 0 || i == n - 1)) v = 0.0; // Dirichlet value
+                if (MODE == 2) X[((size_t)i << ctl) + c] = v;
+                else if (c0 + c < ncol) a.out[ri][base + (size_t)nlm * i] = v;
             }
+            if ((k0 + UR) * rs < n) nload(k0 + UR);
         }
-        if (mode == 1 || mode == 2) {
-            const double *src = (mode == 1) ? u : o;
-            if (mode == 1) {
-                for (int i = 0; i < n; ++i) {
-                    double acc = 0.0;
-                    int j0 = i - bw < 0 ? 0 : i - bw;
-                    for (int j = j0; j < i; ++j) acc += sLU[BANDIDX(bw, bw + i - j, j)] * o[base + (size_t)nlm * j];
-                    o[base + (size_t)nlm * i] = src[base + (size_t)nlm * i] - acc;
-                }
+        if (MODE == 0) return;
+        __syncthreads();
+    }
+    if (tid < (1 << ctl)) {
+        double *x = X + tid;
+        struct Blk {
+            double v[D], f[D][BW], d[D];
+        } A, B;
+        double yw[BW]; // the BW rows solved last, nearest last
+#pragma unroll
+        for (int q = 0; q < BW; ++q) yw[q] = 0.0;
+        // forward: rows i0 .. i0 + D - 1 with the unit L
+        auto fload = [&](Blk &b, int i0) {
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                const int i = min(i0 + d, n - 1);
+                b.v[d] = x[(size_t)i << ctl];
+#pragma unroll
+                for (int q = 0; q < BW; ++q) b.f[d][q] = sU[i * W + q];
             }
-            for (int i = n - 1; i >= 0; --i) {
-                double acc = 0.0;
-                int j1 = i + bw > n - 1 ? n - 1 : i + bw;
-                for (int j = i + 1; j <= j1; ++j) acc += sLU[BANDIDX(bw, bw + i - j, j)] * o[base + (size_t)nlm * j];
-                o[base + (size_t)nlm * i] = (o[base + (size_t)nlm * i] - acc) / sLU[BANDIDX(bw, bw, i)];
+        };
+        auto fcomp = [&](const Blk &b, int i0) {
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                if (i0 + d >= n) break;
+                double v = b.v[d];
+#pragma unroll
+                for (int q = 0; q < BW; ++q) v -= b.f[d][q] * yw[q];
+#pragma unroll
+                for (int q = 0; q < BW - 1; ++q) yw[q] = yw[q + 1];
+                yw[BW - 1] = v;
+                x[(size_t)(i0 + d) << ctl] = v;
             }
+        };
+        fload(A, 0);
+        for (int i0 = 0; i0 < n; i0 += 2 * D) {
+            fload(B, i0 + D);
+            fcomp(A, i0);
+            fload(A, i0 + 2 * D);
+            fcomp(B, i0 + D);
+        }
+        // back: rows i0, i0 - 1, ... with U; yw nearest last as above
+#pragma unroll
+        for (int q = 0; q < BW; ++q) yw[q] = 0.0;
+        auto bload = [&](Blk &b, int i0) {
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                const int i = max(i0 - d, 0);
+                b.v[d] = x[(size_t)i << ctl];
+                b.d[d] = sU[i * W + 2 * BW];
+#pragma unroll
+                for (int q = 0; q < BW; ++q) b.f[d][q] = sU[i * W + BW + q];
+            }
+        };
+        auto bcomp = [&](const Blk &b, int i0) {
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                if (i0 - d < 0) break;
+                double v = b.v[d];
+#pragma unroll
+                for (int q = BW - 1; q >= 0; --q) v -= b.f[d][q] * yw[BW - 1 - q];
+                v *= b.d[d];
+#pragma unroll
+                for (int q = 0; q < BW - 1; ++q) yw[q] = yw[q + 1];
+                yw[BW - 1] = v;
+                x[(size_t)(i0 - d) << ctl] = v;
+            }
+        };
+        bload(A, n - 1);
+        for (int i0 = n - 1; i0 >= 0; i0 -= 2 * D) {
+            bload(B, i0 - D);
+            bcomp(A, i0);
+            bload(A, i0 - 2 * D);
+            bcomp(B, i0 - D);
         }
     }
+    __syncthreads();
+    if (c0 + c < ncol)
+        for (int i = w0; i < n; i += rs) a.out[ri][base + (size_t)nlm * i] = X[((size_t)i << ctl) + c];
+}
+
+template <int BW> static void cnabl_launch(hipStream_t st, const CnabLArgs &a, int mode)
+{
+    const size_t lds = cnabl_lds(a.n, BW, mode, a.ctl);
+    const dim3 grid((2 * (a.mmax + 1) + (1 << a.ctl) - 1) >> a.ctl, a.lmax + 1), block(CNABL_THREADS);
+    if (mode == 0) hipLaunchKernelGGL((cnab2_lmajor_kernel<BW, 0>), grid, block, lds, st, a);
+    else if (mode == 1) hipLaunchKernelGGL((cnab2_lmajor_kernel<BW, 1>), grid, block, lds, st, a);
+    else hipLaunchKernelGGL((cnab2_lmajor_kernel<BW, 2>), grid, block, lds, st, a);
 }
 
 int gd_launch_cnab2_lmajor(hipStream_t st, const double *L, const double *LU, int nl_mats, int lmax, int mmax,
                            int n, int bw, double dt, double theta, int mode, int bc_rows, const double *u_re,
                            const double *u_im, const double *nl_re, const double *nl_im, const double *np_re,
-                           const double *np_im, double *out_re, double *out_im, int *d_status)
+                           const double *np_im, double *out_re, double *out_im)
 {
-    int nlm = gd_nlm_of(lmax, mmax);
-    size_t lds = sizeof(double) * 2 * (2 * bw + 1) * n;
-    GD_CHECK(lds <= 64 * 1024 && bw <= 7, GD_ERR_ARG, "band too large (n=%d bw=%d)", n, bw);
-    hipLaunchKernelGGL(cnab2_lmajor_kernel, dim3(lmax + 1), dim3(64), lds, st, L, LU, nl_mats, lmax, mmax, n, bw,
-                       nlm, dt, theta, mode, bc_rows, u_re, u_im, nl_re, nl_im, np_re, np_im, out_re, out_im,
-                       d_status);
+    GD_CHECK(sizeof(double) * 2 * (2 * bw + 1) * n <= 64 * 1024 && bw >= 1 && bw <= 7, GD_ERR_ARG,
+             "band too large (n=%d bw=%d)", n, bw);
+    // columns per block: 64 (a whole wavefront of solves) while two blocks fit
+    // a CU's 160 KB, fewer for the long columns
+    int ctl = 6;
+    while (ctl > 2 && cnabl_lds(n, bw, mode, ctl) > 80 * 1024) --ctl;
+    GD_CHECK(cnabl_lds(n, bw, mode, ctl) <= 160 * 1024, GD_ERR_ARG, "band too large (n=%d bw=%d)", n, bw);
+    CnabLArgs a{};
+    a.L = L;
+    a.LU = LU;
+    a.nl_mats = nl_mats;
+    a.lmax = lmax;
+    a.mmax = mmax;
+    a.n = n;
+    a.nlm = gd_nlm_of(lmax, mmax);
+    a.bc_rows = bc_rows;
+    a.ctl = ctl;
+    a.inv_dt = 1.0 / dt;
+    a.lw = 1.0 - theta;
+    const double *in[6] = {u_re, u_im, nl_re, nl_im, np_re, np_im};
+    for (int k = 0; k < 2; ++k) {
+        a.u[k] = in[k];
+        a.nl[k] = in[2 + k];
+        a.np[k] = in[4 + k];
+    }
+    a.out[0] = out_re;
+    a.out[1] = out_im;
+    switch (bw) {
+    case 1: cnabl_launch<1>(st, a, mode); break;
+    case 2: cnabl_launch<2>(st, a, mode); break;
+    case 3: cnabl_launch<3>(st, a, mode); break;
+    case 4: cnabl_launch<4>(st, a, mode); break;
+    case 5: cnabl_launch<5>(st, a, mode); break;
+    case 6: cnabl_launch<6>(st, a, mode); break;
+    default: cnabl_launch<7>(st, a, mode); break;
+    }
     return gd_check_launch("cnab2_lmajor_kernel");
 }
 

@@ -12,7 +12,7 @@ int gd_cnab2_build(hipStream_t st, const double *d_lap, const double *d_rinv2, d
 int gd_launch_cnab2_lmajor(hipStream_t st, const double *L, const double *LU, int nl_mats, int lmax, int mmax,
                            int n, int bw, double dt, double theta, int mode, int bc_rows, const double *u_re,
                            const double *u_im, const double *nl_re, const double *nl_im, const double *np_re,
-                           const double *np_im, double *out_re, double *out_im, int *d_status);
+                           const double *np_im, double *out_re, double *out_im);
 int gd_launch_cnab2_step(hipStream_t st, const double *nuLap, const double *rinv2, const double *nus,
                          const double *LUt, const int *l_of_idx, int nl, int n, int bw, int nlm, double dt,
                          double theta, int bc_mask, const double *st_in, double *st_out, const double *nl_arr,

@@ -440,24 +440,24 @@ static int step_vjp(gd_step *s, const double *xs, bool boot, const double *lam_i
 // l-major (nlm, nr) planes of the five fields <-> m-major device planes
 static int planes_to_device(gd_step *s, const double *re, const double *im, double *dev)
 {
-    const int *map = s->sht.d_lmaj_of_idx.as<int>();
+    LmPlanes p;
     for (int f = 0; f < 5; ++f) {
         const size_t o = (size_t)f * s->fs;
-        GD_TRY(gd_launch_perm(s->ctx->stream, re + o, map, s->nlm, s->d.nr, dev + (2 * f) * s->fs));
-        GD_TRY(gd_launch_perm(s->ctx->stream, im + o, map, s->nlm, s->d.nr, dev + (2 * f + 1) * s->fs));
+        p.add(re + o, dev + (2 * f) * s->fs);
+        p.add(im + o, dev + (2 * f + 1) * s->fs);
     }
-    return GD_OK;
+    return gd_launch_to_m<double>(s->ctx->stream, s->d.lmax, s->d.mmax, s->d.nr, p, (size_t)s->nlm);
 }
 
 static int planes_from_device(gd_step *s, const double *dev, double *re, double *im)
 {
-    const int *map = s->sht.d_idx_of_lmaj.as<int>();
+    LmPlanes p;
     for (int f = 0; f < 5; ++f) {
         const size_t o = (size_t)f * s->fs;
-        GD_TRY(gd_launch_perm(s->ctx->stream, dev + (2 * f) * s->fs, map, s->nlm, s->d.nr, re + o));
-        GD_TRY(gd_launch_perm(s->ctx->stream, dev + (2 * f + 1) * s->fs, map, s->nlm, s->d.nr, im + o));
+        p.add(dev + (2 * f) * s->fs, re + o);
+        p.add(dev + (2 * f + 1) * s->fs, im + o);
     }
-    return GD_OK;
+    return gd_launch_from_m(s->ctx->stream, s->d.lmax, s->d.mmax, s->d.nr, p);
 }
 
 // host or device planes in (GD_HOST staged through buf), device planes out

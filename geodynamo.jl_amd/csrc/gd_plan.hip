@@ -73,8 +73,6 @@ int gd_sht_plan_build(gd_ctx *ctx, int lmax, int mmax, int nlat, int nlon, int p
     GD_TRY(upload(ctx, p->d_moff, p->maps.moff));
     GD_TRY(upload(ctx, p->d_ne, p->maps.ne));
     GD_TRY(upload(ctx, p->d_l_of_idx, p->maps.l_of_idx));
-    GD_TRY(upload(ctx, p->d_lmaj_of_idx, p->maps.lmaj_of_idx));
-    GD_TRY(upload(ctx, p->d_idx_of_lmaj, p->maps.idx_of_lmaj));
     GD_TRY(upload(ctx, p->d_m_of_idx, p->maps.m_of_idx));
     std::vector<double> xn(p->x.begin(), p->x.begin() + p->nlat2);
     GD_TRY(upload(ctx, p->d_x, xn));
@@ -119,7 +117,7 @@ int gd_sht_plan_build(gd_ctx *ctx, int lmax, int mmax, int nlat, int nlon, int p
 
 void gd_sht_plan_release(gd_sht_plan *p)
 {
-    DevBuf *bufs[] = {&p->d_moff, &p->d_ne, &p->d_l_of_idx, &p->d_lmaj_of_idx, &p->d_idx_of_lmaj, &p->d_x,
+    DevBuf *bufs[] = {&p->d_moff, &p->d_ne, &p->d_l_of_idx, &p->d_x,
                       &p->d_m_of_idx, &p->wone, &p->wq64,
                       &p->tab64, &p->tab32, &p->tw, &p->sinth, &p->costh, &p->wq, &p->syn, &p->fb,
                       &p->gb, &p->outm, &p->h_in0, &p->h_in1, &p->h_in2, &p->h_in3, &p->h_out0,
@@ -261,13 +259,15 @@ static int run_synth(gd_sht_plan *p, bool vec, const double *a_re, const double 
     GD_TRY(p->syn.ensure(sizeof(T) * (size_t)nr * cin * nlm));
     GD_TRY(p->fb.ensure(sizeof(T) * (size_t)p->nlat2 * nr * nm * nslot));
     T *syn = p->syn.as<T>();
+    // vector: S := pol (b) in columns 0,1; T := tor (a) in columns 2,3
+    LmPlanes cols;
     if (vec) {
-        // S := pol (b) in columns 0,1; T := tor (a) in columns 2,3
-        GD_TRY(gd_launch_pack<T>(st, b_re, b_im, p->d_lmaj_of_idx.as<int>(), nlm, nr, cin, 0, syn));
-        GD_TRY(gd_launch_pack<T>(st, a_re, a_im, p->d_lmaj_of_idx.as<int>(), nlm, nr, cin, 2, syn));
-    } else {
-        GD_TRY(gd_launch_pack<T>(st, a_re, a_im, p->d_lmaj_of_idx.as<int>(), nlm, nr, cin, 0, syn));
+        cols.add(b_re, syn);
+        cols.add(b_im, syn + nlm);
     }
+    cols.add(a_re, syn + (vec ? 2 : 0) * (size_t)nlm);
+    cols.add(a_im, syn + (vec ? 3 : 1) * (size_t)nlm);
+    GD_TRY(gd_launch_to_m<T>(st, p->lmax, p->mmax, nr, cols, (size_t)cin * nlm));
     if (adj) {
         hipLaunchKernelGGL((colscale_kernel<T>), dim3((nlm + 255) / 256, nr * cin), dim3(256), 0, st, syn,
                            p->d_l_of_idx.as<int>(), p->d_m_of_idx.as<int>(), nlm, vec ? 1 : 0);
@@ -362,6 +362,7 @@ static int run_analysis(gd_sht_plan *p, bool vec, const double *f0, const double
     a.mmax = p->mmax;
     double *om = p->outm.as<double>();
     const int maxgroup = (p->lmax + 2) / 2;
+    LmPlanes planes;
     if (vec) {
         a.tab0 = gd_sht_tab(p, 1);
         a.tab1 = gd_sht_tab(p, 2);
@@ -375,10 +376,10 @@ static int run_analysis(gd_sht_plan *p, bool vec, const double *f0, const double
             GD_TRY(gd_check_launch("cm_kernel"));
         }
         // o0 = tor, o1 = pol
-        GD_TRY(gd_launch_unpack(st, om + 2 * fs, p->d_idx_of_lmaj.as<int>(), nlm, nr, o0_re));
-        GD_TRY(gd_launch_unpack(st, om + 3 * fs, p->d_idx_of_lmaj.as<int>(), nlm, nr, o0_im));
-        GD_TRY(gd_launch_unpack(st, om, p->d_idx_of_lmaj.as<int>(), nlm, nr, o1_re));
-        GD_TRY(gd_launch_unpack(st, om + fs, p->d_idx_of_lmaj.as<int>(), nlm, nr, o1_im));
+        planes.add(om + 2 * fs, o0_re);
+        planes.add(om + 3 * fs, o0_im);
+        planes.add(om, o1_re);
+        planes.add(om + fs, o1_im);
     } else {
         a.tab0 = gd_sht_tab(p, 0);
         a.tab1 = nullptr;
@@ -390,10 +391,10 @@ static int run_analysis(gd_sht_plan *p, bool vec, const double *f0, const double
                                p->d_m_of_idx.as<int>(), nlm);
             GD_TRY(gd_check_launch("cm_kernel"));
         }
-        GD_TRY(gd_launch_unpack(st, om, p->d_idx_of_lmaj.as<int>(), nlm, nr, o0_re));
-        GD_TRY(gd_launch_unpack(st, om + fs, p->d_idx_of_lmaj.as<int>(), nlm, nr, o0_im));
+        planes.add(om, o0_re);
+        planes.add(om + fs, o0_im);
     }
-    return GD_OK;
+    return gd_launch_from_m(st, p->lmax, p->mmax, nr, planes);
 }
 
 // stage host arrays (GD_HOST) to device buffers

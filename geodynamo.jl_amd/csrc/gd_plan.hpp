@@ -10,7 +10,7 @@ struct gd_sht_plan {
     LmMaps maps;
     FftPlan fft;
     std::vector<double> x, w, theta; // host FP64 grid (cos theta, Gauss weights, colatitude)
-    DevBuf d_moff, d_ne, d_l_of_idx, d_lmaj_of_idx, d_idx_of_lmaj, d_x, d_m_of_idx;
+    DevBuf d_moff, d_ne, d_l_of_idx, d_x, d_m_of_idx;
     DevBuf tab64, tab32;             // [3][nlm][nlat2]: P, dP/dtheta, m P / sin
     DevBuf tw, sinth, costh, wq;     // in the plan's arithmetic type
     DevBuf wone, wq64;               // nlat/2 ones (plan type) and the weights 2 pi w_i / nlon in FP64

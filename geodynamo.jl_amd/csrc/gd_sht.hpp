@@ -90,11 +90,24 @@ template <typename T> int gd_launch_synth_vec(hipStream_t st, const SynthArgs &a
 template <typename T> int gd_launch_synth_scal(hipStream_t st, const SynthArgs &a);
 template <typename T> int gd_launch_ana(hipStream_t st, const AnaArgs &a, bool vec, int maxgroup);
 template <typename T> int gd_launch_ring(hipStream_t st, int mode, const RingArgs &a);
+// up to LM_MAXPLANES planes between the l-major layout of the interface
+// (level stride nlm) and the m-major device layout, one launch for all:
+// to_m writes element type T with dst_ls elements from level to level (nlm for
+// a plane, cin * nlm for a synthesis column); from_m is plane to plane
+constexpr int LM_MAXPLANES = 10;
+struct LmPlanes {
+    int n = 0;
+    const double *src[LM_MAXPLANES];
+    void *dst[LM_MAXPLANES];
+    void add(const double *s, void *d)
+    {
+        src[n] = s;
+        dst[n++] = d;
+    }
+};
 template <typename T>
-int gd_launch_pack(hipStream_t st, const double *re, const double *im, const int *lmaj_of_idx, int nlm, int nr,
-                   int cin, int c0, T *out);
-int gd_launch_unpack(hipStream_t st, const double *src, const int *idx_of_lmaj, int nlm, int nr, double *dst);
-int gd_launch_perm(hipStream_t st, const double *src, const int *map, int nlm, int nr, double *dst);
+int gd_launch_to_m(hipStream_t st, int lmax, int mmax, int nr, const LmPlanes &a, size_t dst_ls);
+int gd_launch_from_m(hipStream_t st, int lmax, int mmax, int nr, const LmPlanes &a);
 
 // ---- batched step launches (gd_sht.hip): one grid over several shells'
 // launches of the tangential step's kernels, all in one compile-time form.

@@ -801,22 +801,27 @@ extern "C" int gd_step_destroy(gd_step *s)
     return GD_OK;
 }
 
+static int planes_convert(gd_step *s, const LmPlanes &p, bool to_device)
+{
+    return to_device ? gd_launch_to_m<double>(s->ctx->stream, s->d.lmax, s->d.mmax, s->d.nr, p, (size_t)s->nlm)
+                     : gd_launch_from_m(s->ctx->stream, s->d.lmax, s->d.mmax, s->d.nr, p);
+}
+
 // l-major user layout <-> m-major device planes
 static int convert_state(gd_step *s, const double *re, const double *im, double *dev, bool to_device)
 {
-    const int nr = s->d.nr, nlm = s->nlm;
-    const int *map = to_device ? s->sht.d_lmaj_of_idx.as<int>() : s->sht.d_idx_of_lmaj.as<int>();
+    LmPlanes p;
     for (int f = 0; f < 5; ++f) {
         const size_t o = (size_t)f * s->fs;
         if (to_device) {
-            GD_TRY(gd_launch_perm(s->ctx->stream, re + o, map, nlm, nr, dev + (2 * f) * s->fs));
-            GD_TRY(gd_launch_perm(s->ctx->stream, im + o, map, nlm, nr, dev + (2 * f + 1) * s->fs));
+            p.add(re + o, dev + (2 * f) * s->fs);
+            p.add(im + o, dev + (2 * f + 1) * s->fs);
         } else {
-            GD_TRY(gd_launch_perm(s->ctx->stream, dev + (2 * f) * s->fs, map, nlm, nr, const_cast<double *>(re) + o));
-            GD_TRY(gd_launch_perm(s->ctx->stream, dev + (2 * f + 1) * s->fs, map, nlm, nr, const_cast<double *>(im) + o));
+            p.add(dev + (2 * f) * s->fs, const_cast<double *>(re) + o);
+            p.add(dev + (2 * f + 1) * s->fs, const_cast<double *>(im) + o);
         }
     }
-    return GD_OK;
+    return planes_convert(s, p, to_device);
 }
 
 extern "C" int gd_step_set_state(gd_step *s, const double *re, const double *im, int flags)
@@ -1098,9 +1103,10 @@ extern "C" int gd_step_set_composition(gd_step *s, const double *re, const doubl
         b = a + s->fs;
     }
     double *dst = s->cstate[s->step & 1].as<double>();
-    const int *map = s->sht.d_lmaj_of_idx.as<int>();
-    GD_TRY(gd_launch_perm(st, a, map, s->nlm, s->d.nr, dst + 8 * s->fs));
-    GD_TRY(gd_launch_perm(st, b, map, s->nlm, s->d.nr, dst + 9 * s->fs));
+    LmPlanes p;
+    p.add(a, dst + 8 * s->fs);
+    p.add(b, dst + 9 * s->fs);
+    GD_TRY(planes_convert(s, p, true));
     s->csyn_ok = false;
     if (flags & GD_HOST) GD_HIP(hipStreamSynchronize(st));
     return GD_OK;
@@ -1119,9 +1125,10 @@ extern "C" int gd_step_get_composition(gd_step *s, double *re, double *im, int f
         b = a + s->fs;
     }
     const double *src = s->cstate[s->step & 1].as<double>();
-    const int *map = s->sht.d_idx_of_lmaj.as<int>();
-    GD_TRY(gd_launch_perm(st, src + 8 * s->fs, map, s->nlm, s->d.nr, a));
-    GD_TRY(gd_launch_perm(st, src + 9 * s->fs, map, s->nlm, s->d.nr, b));
+    LmPlanes p;
+    p.add(src + 8 * s->fs, a);
+    p.add(src + 9 * s->fs, b);
+    GD_TRY(planes_convert(s, p, false));
     if (flags & GD_HOST) {
         GD_TRY(gd_from_device(s->ctx, re, a, sizeof(double) * s->fs));
         GD_TRY(gd_from_device(s->ctx, im, b, sizeof(double) * s->fs));
@@ -1146,14 +1153,16 @@ static int comp_planes(gd_step *s, double *buf, double *re, double *im, int flag
         }
     }
     if (to_device) {
-        const int *map = s->sht.d_lmaj_of_idx.as<int>();
-        GD_TRY(gd_launch_perm(st, a, map, s->nlm, s->d.nr, buf + 8 * s->fs));
-        GD_TRY(gd_launch_perm(st, b, map, s->nlm, s->d.nr, buf + 9 * s->fs));
+        LmPlanes p;
+        p.add(a, buf + 8 * s->fs);
+        p.add(b, buf + 9 * s->fs);
+        GD_TRY(planes_convert(s, p, true));
         if (flags & GD_HOST) GD_HIP(hipStreamSynchronize(st));
     } else {
-        const int *map = s->sht.d_idx_of_lmaj.as<int>();
-        GD_TRY(gd_launch_perm(st, buf + 8 * s->fs, map, s->nlm, s->d.nr, a));
-        GD_TRY(gd_launch_perm(st, buf + 9 * s->fs, map, s->nlm, s->d.nr, b));
+        LmPlanes p;
+        p.add(buf + 8 * s->fs, a);
+        p.add(buf + 9 * s->fs, b);
+        GD_TRY(planes_convert(s, p, false));
         if (flags & GD_HOST) {
             GD_TRY(gd_from_device(s->ctx, re, a, sizeof(double) * s->fs));
             GD_TRY(gd_from_device(s->ctx, im, b, sizeof(double) * s->fs));

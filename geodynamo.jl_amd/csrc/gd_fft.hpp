@@ -1,0 +1,196 @@
+// gd_fft.hpp -- register FFT butterflies and the compiled ring-FFT plans.
+//
+// A transform of length n = 2^a 3^b runs as two or three Stockham stages of
+// radix up to 18, each butterfly held in registers: stage s reads
+// x[j + r n/R], multiplies by the stage's twiddles and writes
+// (j / Ns) Ns R + j % Ns + r Ns (Ns: the product of the earlier radices).
+#pragma once
+#include "gd_internal.hpp"
+
+template <typename T> struct alignas(2 * sizeof(T)) C2 {
+    T x, y;
+};
+template <typename T> __device__ __forceinline__ C2<T> cadd(C2<T> a, C2<T> b) { return {a.x + b.x, a.y + b.y}; }
+template <typename T> __device__ __forceinline__ C2<T> csub(C2<T> a, C2<T> b) { return {a.x - b.x, a.y - b.y}; }
+template <typename T> __device__ __forceinline__ C2<T> cmul(C2<T> a, C2<T> b)
+{
+    return {a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x};
+}
+// multiply by i*dir
+template <typename T> __device__ __forceinline__ C2<T> cmuli(C2<T> a, int dir)
+{
+    return dir > 0 ? C2<T>{-a.y, a.x} : C2<T>{a.y, -a.x};
+}
+
+// cos(2 pi k / 144) and sin(2 pi k / 144), k = 0 .. 18: every twiddle inside a
+// radix that divides 144
+__host__ __device__ constexpr double cos144(int k)
+{
+    constexpr double c[19] = {
+        1.0, 0.9990482215818577624037, 0.996194698091745532295, 0.9914448613738104111446, 0.9848077530122080593667,
+        0.9762960071199333659709, 0.9659258262890682867497, 0.9537169507482269211438, 0.9396926207859083840541,
+        0.9238795325112867561282, 0.9063077870366499632426, 0.8870108331782217010546, 0.8660254037844386467637,
+        0.8433914458128857012729, 0.8191520442889917896845, 0.7933533402912351645798, 0.7660444431189780352024,
+        0.7372773368101240413843, 0.7071067811865475244008};
+    constexpr double s[19] = {
+        0.0, 0.0436193873653359997818, 0.0871557427476581735581, 0.1305261922200515915484,
+        0.1736481776669303488517, 0.2164396139381028797596, 0.2588190451025207623489, 0.3007057995042731216225,
+        0.3420201433256687330441, 0.3826834323650897717285, 0.422618261740699436187, 0.4617486132350339305629, 0.5,
+        0.5372996083468238318408, 0.573576436351046096108, 0.6087614290087206394161, 0.6427876096865393263226,
+        0.6755902076156602443483, 0.7071067811865475244008};
+    k %= 144;
+    if (k > 72) k = 144 - k;
+    return k > 54 ? -c[72 - k] : k > 36 ? -s[k - 36] : k > 18 ? s[36 - k] : c[k];
+}
+__host__ __device__ constexpr double sin144(int k) { return cos144(k + 108); }
+
+// a e^(DIR 2 pi i k / 144), k a constant once the caller's loop is unrolled
+template <int DIR, typename T> __device__ __forceinline__ C2<T> rot144(C2<T> a, int k)
+{
+    k %= 144;
+    if (k == 0) return a;
+    if (k == 36) return cmuli(a, DIR);
+    if (k == 72) return C2<T>{-a.x, -a.y};
+    if (k == 108) return cmuli(a, -DIR);
+    const T c = (T)cos144(k), s = (T)(DIR * sin144(k));
+    return C2<T>{a.x * c - a.y * s, a.x * s + a.y * c};
+}
+
+// in-register DFT of radix R (a divisor of 144): v[k] <- sum_n v[n] e^(DIR 2 pi i n k / R)
+template <int R, int DIR, typename T> __device__ __forceinline__ void dft(C2<T> *v)
+{
+    if constexpr (R == 2) {
+        const C2<T> t = v[0];
+        v[0] = cadd(t, v[1]);
+        v[1] = csub(t, v[1]);
+    } else if constexpr (R == 3) {
+        const T s3 = T(0.86602540378443864676);
+        const C2<T> t1 = cadd(v[1], v[2]), d = csub(v[1], v[2]);
+        const C2<T> t2 = {v[0].x - T(0.5) * t1.x, v[0].y - T(0.5) * t1.y};
+        const C2<T> t3 = cmuli(C2<T>{s3 * d.x, s3 * d.y}, DIR);
+        v[0] = cadd(v[0], t1);
+        v[1] = cadd(t2, t3);
+        v[2] = csub(t2, t3);
+    } else if constexpr (R == 4) {
+        const C2<T> a = cadd(v[0], v[2]), b = csub(v[0], v[2]), c = cadd(v[1], v[3]);
+        const C2<T> d = cmuli(csub(v[1], v[3]), DIR);
+        v[0] = cadd(a, c);
+        v[2] = csub(a, c);
+        v[1] = cadd(b, d);
+        v[3] = csub(b, d);
+    } else {
+        // R = A B: n = B n1 + n2, k = k1 + A k2
+        constexpr int A = R % 4 == 0 ? (R == 8 ? 2 : 4) : (R == 9 ? 3 : 2), B = R / A;
+        static_assert(144 % R == 0, "radix");
+        C2<T> u[R];
+#pragma unroll
+        for (int n2 = 0; n2 < B; ++n2) {
+            C2<T> w[A];
+#pragma unroll
+            for (int n1 = 0; n1 < A; ++n1) w[n1] = v[B * n1 + n2];
+            dft<A, DIR>(w);
+#pragma unroll
+            for (int k1 = 0; k1 < A; ++k1) u[n2 * A + k1] = rot144<DIR>(w[k1], 144 / R * n2 * k1);
+        }
+#pragma unroll
+        for (int k1 = 0; k1 < A; ++k1) {
+            C2<T> w[B];
+#pragma unroll
+            for (int n2 = 0; n2 < B; ++n2) w[n2] = u[n2 * A + k1];
+            dft<B, DIR>(w);
+#pragma unroll
+            for (int k2 = 0; k2 < B; ++k2) v[k1 + A * k2] = w[k2];
+        }
+    }
+}
+
+// ---- compiled plans: two stages where both radices are at most 18 (the least
+// largest radix), else three of at most 12
+struct FftStages {
+    int n = 0, r[3] = {1, 1, 1};
+};
+constexpr FftStages fft_stages(int n)
+{
+    constexpr int set[9] = {3, 4, 6, 8, 9, 12, 16, 18, 0};
+    FftStages f;
+    for (int a = 0; set[a]; ++a)
+        for (int b = a; set[b]; ++b)
+            if (set[a] * set[b] == n && (f.n == 0 || set[b] < f.r[1])) {
+                f.n = 2;
+                f.r[0] = set[a];
+                f.r[1] = set[b];
+            }
+    if (f.n) return f;
+    for (int a = 0; set[a]; ++a)
+        for (int b = a; set[b]; ++b)
+            for (int c = b; set[c] && set[c] <= 12; ++c)
+                if (set[a] * set[b] * set[c] == n && (f.n == 0 || set[c] < f.r[2])) {
+                    f.n = 3;
+                    f.r[0] = set[a];
+                    f.r[1] = set[b];
+                    f.r[2] = set[c];
+                }
+    return f;
+}
+
+// Twiddles of the stages after the first, e^(-2 pi i r k / (Ns R)) at
+// [offset + r Ns + k] (r < R, k < Ns), so that consecutive k are consecutive:
+// stage 1 at offset 0, stage 2 after it.
+constexpr int fft_tw_off(FftStages f, int s) { return s == 2 ? f.r[0] * f.r[1] : 0; }
+constexpr int fft_tw_len(FftStages f) { return f.r[0] * f.r[1] + (f.n == 3 ? f.r[0] * f.r[1] * f.r[2] : 0); }
+
+// LDS positions of the two exchanges (padded against bank conflicts): after
+// the first stage element e sits at e + (e / r0) P1, after the second of three
+// at e + (e / (r0 r1)) P2; LD is the stride from one transform to the next,
+// congruent to 2 (16-byte elements) or 4 (8-byte) modulo a bank row so that
+// lanes on different transforms fall on different banks.
+template <typename T, int N> struct FftLds {
+    static constexpr FftStages f = fft_stages(N);
+    static constexpr int P1 = f.r[0] % 2 == 0 ? 1 : 0;
+    static constexpr int P2 = f.n == 3 ? f.r[0] : 0;
+    static constexpr int S1 = N + N / f.r[0] * P1, S2 = N + (f.n == 3 ? f.r[2] * P2 : 0);
+    static constexpr int S = S1 > S2 ? S1 : S2;
+    static constexpr int M = sizeof(T) == 8 ? 8 : 16, W = sizeof(T) == 8 ? 2 : 4;
+    static constexpr int LD = S + (W - S % M + M) % M;
+};
+
+// butterfly j of stage s (1 or 2): its inputs from one transform's LDS row
+// with the twiddles applied, transformed in place of v
+template <typename T, int N, int S, int DIR>
+__device__ __forceinline__ void fft_lds_stage(const C2<T> *x, const C2<T> *tws, int j, C2<T> *v)
+{
+    using F = FftLds<T, N>;
+    constexpr FftStages f = F::f;
+    constexpr int R = f.r[S], Ns = S == 1 ? f.r[0] : f.r[0] * f.r[1], nb = N / R;
+    const C2<T> *tw = tws + fft_tw_off(f, S) + (nb == Ns ? j : j % Ns);
+    C2<T> w[R];
+#pragma unroll
+    for (int r = 1; r < R; ++r) w[r] = tw[r * Ns];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int p = S == 1 ? j + r * nb + (j / f.r[0] + r * (nb / f.r[0])) * F::P1 : j + r * (nb + F::P2);
+        v[r] = x[p];
+    }
+#pragma unroll
+    for (int r = 1; r < R; ++r) {
+        if (DIR > 0) w[r].y = -w[r].y;
+        v[r] = cmul(v[r], w[r]);
+    }
+    dft<R, DIR>(v);
+}
+
+// results of butterfly j of stage s into the next exchange
+template <typename T, int N, int S> __device__ __forceinline__ void fft_lds_put(C2<T> *x, int j, const C2<T> *v)
+{
+    using F = FftLds<T, N>;
+    constexpr FftStages f = F::f;
+    if constexpr (S == 0) {
+#pragma unroll
+        for (int r = 0; r < f.r[0]; ++r) x[j * (f.r[0] + F::P1) + r] = v[r];
+    } else {
+        static_assert(S == 1 && f.n == 3, "the second exchange of three stages");
+#pragma unroll
+        for (int r = 0; r < f.r[1]; ++r)
+            x[j / f.r[0] * (f.r[0] * f.r[1] + F::P2) + j % f.r[0] + r * f.r[0]] = v[r];
+    }
+}

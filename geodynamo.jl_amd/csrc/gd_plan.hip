@@ -92,6 +92,8 @@ int gd_sht_plan_build(gd_ctx *ctx, int lmax, int mmax, int nlat, int nlon, int p
         tw[2 * k] = std::cos(a);
         tw[2 * k + 1] = -std::sin(a);
     }
+    std::vector<double> tws;
+    gd_ring_stage_twiddles(nlon, tws);
     for (int i = 0; i < nlat; ++i) {
         s[i] = std::sin(p->theta[i]);
         c[i] = std::cos(p->theta[i]);
@@ -101,12 +103,14 @@ int gd_sht_plan_build(gd_ctx *ctx, int lmax, int mmax, int nlat, int nlon, int p
     if (prec == GD_PREC_FP64) {
         GD_TRY(upload(ctx, p->wone, std::vector<double>(p->nlat2, 1.0)));
         GD_TRY(upload(ctx, p->tw, tw));
+        if (!tws.empty()) GD_TRY(upload(ctx, p->tws, tws));
         GD_TRY(upload(ctx, p->sinth, s));
         GD_TRY(upload(ctx, p->costh, c));
         GD_TRY(upload(ctx, p->wq, wq));
     } else {
         GD_TRY(upload(ctx, p->wone, std::vector<float>(p->nlat2, 1.0f)));
         GD_TRY(upload(ctx, p->tw, std::vector<float>(tw.begin(), tw.end())));
+        if (!tws.empty()) GD_TRY(upload(ctx, p->tws, std::vector<float>(tws.begin(), tws.end())));
         GD_TRY(upload(ctx, p->sinth, std::vector<float>(s.begin(), s.end())));
         GD_TRY(upload(ctx, p->costh, std::vector<float>(c.begin(), c.end())));
         GD_TRY(upload(ctx, p->wq, std::vector<float>(wq.begin(), wq.end())));
@@ -119,7 +123,7 @@ void gd_sht_plan_release(gd_sht_plan *p)
 {
     DevBuf *bufs[] = {&p->d_moff, &p->d_ne, &p->d_l_of_idx, &p->d_x,
                       &p->d_m_of_idx, &p->wone, &p->wq64,
-                      &p->tab64, &p->tab32, &p->tw, &p->sinth, &p->costh, &p->wq, &p->syn, &p->fb,
+                      &p->tab64, &p->tab32, &p->tw, &p->tws, &p->sinth, &p->costh, &p->wq, &p->syn, &p->fb,
                       &p->gb, &p->outm, &p->h_in0, &p->h_in1, &p->h_in2, &p->h_in3, &p->h_out0,
                       &p->h_out1, &p->h_out2, &p->h_out3};
     for (DevBuf *b : bufs) b->release();
@@ -135,6 +139,7 @@ const void *gd_sht_tab(const gd_sht_plan *p, int t)
 void gd_sht_fill_ring(const gd_sht_plan *p, RingArgs &a, int nr)
 {
     a.tw = p->tw.p;
+    a.tws = p->tws.p;
     a.sinth = p->sinth.p;
     a.costh = p->costh.p;
     a.wq = p->wq.p;

@@ -63,6 +63,7 @@ struct RingArgs {
     const double *phys_in[2];
     double *phys_out[2];
     const void *tw;       // T2[nlon], e^{-2 pi i k / nlon}
+    const void *tws;      // T2, twiddles of the compiled plan's stages (null where nlon has none)
     const void *sinth, *costh, *wq; // T[nlat] sin, cos of colatitude; T[nlat2] 2 pi w / nlon
     int nlat, nlat2, nlon, nr, mmax;
     int nstages, radix[12];
@@ -90,6 +91,20 @@ template <typename T> int gd_launch_synth_vec(hipStream_t st, const SynthArgs &a
 template <typename T> int gd_launch_synth_scal(hipStream_t st, const SynthArgs &a);
 template <typename T> int gd_launch_ana(hipStream_t st, const AnaArgs &a, bool vec, int maxgroup);
 template <typename T> int gd_launch_ring(hipStream_t st, int mode, const RingArgs &a);
+// ring lengths with a compiled FFT plan (gd_fft.hpp): every 2^a 3^b from 48 to 768
+#define GD_RING_LENGTHS                                                                                          \
+    GD_RING_LEN(48) GD_RING_LEN(54) GD_RING_LEN(64) GD_RING_LEN(72) GD_RING_LEN(81) GD_RING_LEN(96)              \
+    GD_RING_LEN(108) GD_RING_LEN(128) GD_RING_LEN(144) GD_RING_LEN(162) GD_RING_LEN(192) GD_RING_LEN(216)        \
+    GD_RING_LEN(243) GD_RING_LEN(256) GD_RING_LEN(288) GD_RING_LEN(324) GD_RING_LEN(384) GD_RING_LEN(432)        \
+    GD_RING_LEN(486) GD_RING_LEN(512) GD_RING_LEN(576) GD_RING_LEN(648) GD_RING_LEN(729) GD_RING_LEN(768)
+bool gd_ring_compiled(int nlon);
+// stage twiddles of the compiled plan of nlon, e^{-i angle} as (re, im) pairs
+void gd_ring_stage_twiddles(int nlon, std::vector<double> &tw);
+// a boundary pass (RING_SYNTH, RING_ANALYSIS; 1 or 2 fields) by the compiled
+// plan of its ring length; false where there is none
+template <typename T> bool gd_launch_ring_plan(hipStream_t st, int mode, const RingArgs &a);
+template <> bool gd_launch_ring_plan<float>(hipStream_t st, int mode, const RingArgs &a);
+template <> bool gd_launch_ring_plan<double>(hipStream_t st, int mode, const RingArgs &a);
 // up to LM_MAXPLANES planes between the l-major layout of the interface
 // (level stride nlm) and the m-major device layout, one launch for all:
 // to_m writes element type T with dst_ls elements from level to level (nlm for

@@ -213,8 +213,8 @@ int launch_adj_chain_bw(hipStream_t st, const AdjChainArgs &c, int bw)
 // 4, 5 mu(u_pol) / (c_m l(l+1)); 6, 7 mu(u_tor) / (c_m l(l+1)); 8, 9 T / r;
 // 10, 11 mu(T) / c_m   (re, im each; l = 0 cotangent columns 0)
 constexpr int ADJ_COLS = 12;
-// Fourier records: u (0..7), the force cotangent (8..15), grad T (16..23),
-// the advection cotangent (24..27)
+// Fourier slots per record: u, the force cotangent and grad T (8 each), the
+// advection cotangent (4); products: two vector arrays
 constexpr int ADJ_NSLOT = 28;
 constexpr int ADJ_NSLOT_G = 16;
 
@@ -280,10 +280,10 @@ static int adj_work(gd_step *s, gd_adj_work **out)
     if (!s->adjw) {
         gd_adj_work *w = new gd_adj_work();
         const size_t esz = s->d.prec == GD_PREC_FP64 ? sizeof(double) : sizeof(float);
-        const size_t nm = s->d.mmax + 1, nr = s->d.nr;
         int rc = w->syn.ensure(esz * s->fs * ADJ_COLS);
-        if (rc == GD_OK) rc = w->fb.ensure(esz * (size_t)s->sht.nlat2 * nr * nm * ADJ_NSLOT);
-        if (rc == GD_OK) rc = w->gb.ensure(esz * nm * s->sht.nlat2 * nr * ADJ_NSLOT_G);
+        const size_t recs = (size_t)(s->d.mmax + 1) * s->d.nr * s->sht.nlat2;
+        if (rc == GD_OK) rc = w->fb.ensure(esz * recs * ADJ_NSLOT);
+        if (rc == GD_OK) rc = w->gb.ensure(esz * recs * ADJ_NSLOT_G);
         if (rc == GD_OK) rc = w->tmp.ensure(sizeof(double) * s->fs * 8);
         if (rc == GD_OK) rc = w->m_of_idx.ensure(sizeof(int) * s->nlm);
         if (rc == GD_OK &&
@@ -336,7 +336,10 @@ static int nonlinear_adjoint_T(gd_step *s, const double *xs, const double *mu, d
     a.out = w->fb.p;
     a.in = w->syn.p;
     a.cin = ADJ_COLS;
-    a.nslot = ADJ_NSLOT;
+    const size_t nm = p->mmax + 1, recs = nm * nr * p->nlat2;
+    a.dim = RecDim{1, nm, nm * nr}; // as the step: FB[i][level][m], GB[m][i][level]
+    a.plane = 8;
+    a.rstr = ADJ_NSLOT;
     // u and the force cotangent as full fields, grad T as a gradient field
     // (S = T/r only: its zero toroidal columns are not contracted)
     a.nf = 2;
@@ -344,25 +347,25 @@ static int nonlinear_adjoint_T(gd_step *s, const double *xs, const double *mu, d
     for (int k = 0; k < 20; ++k) a.colmap[k] = k < 10 ? k : -1;
     a.tab0 = gd_sht_tab(p, 1);
     a.tab1 = gd_sht_tab(p, 2);
-    a.slot0 = 0;
     GD_TRY(gd_launch_synth_vec<T>(st, a));
     a.nf = 1;
     for (int k = 0; k < 20; ++k) a.colmap[k] = k < 2 ? 10 + k : -1;
     a.tab0 = gd_sht_tab(p, 0);
     a.tab1 = nullptr;
-    a.slot0 = 24;
+    a.out = w->fb.as<T>() + 24;
     GD_TRY(gd_launch_synth_scal<T>(st, a));
     RingArgs r{};
     gd_sht_fill_ring(p, r, nr);
     r.fb = w->fb.p;
     r.gb = w->gb.p;
-    r.nslot_f = ADJ_NSLOT;
-    r.nslot_g = ADJ_NSLOT_G;
     r.nfield = 7;
-    static const int fn[7] = {0, 2, 8, 10, 16, 18, 24}, fsou[7] = {4, 6, 12, 14, 20, 22, 26};
-    for (int F = 0; F < 7; ++F) {
-        r.fn_off[F] = fn[F];
-        r.fs_off[F] = fsou[F];
+    r.fdim = a.dim;
+    r.gdim = RecDim{(size_t)p->nlat2 * nr, 1, (size_t)nr};
+    r.fstr = ADJ_NSLOT;
+    for (int F = 0; F < 7; ++F) r.foff[F] = 4 * F;
+    for (int P = 0; P < 4; ++P) {
+        r.goff[P] = gd_comp_off(P, 4, recs);
+        r.gstr[P] = gd_comp_str(P, 4);
     }
     r.ro = s->d.Pm / s->d.E;
     r.coriolis_index = s->d.coriolis_index;
@@ -370,8 +373,8 @@ static int nonlinear_adjoint_T(gd_step *s, const double *xs, const double *mu, d
     AnaArgs g{};
     g.mm = p->prec == GD_PREC_BF16X3;
     g.gb = w->gb.p;
-    g.nslot_g = ADJ_NSLOT_G;
-    g.gslot0 = 0;
+    g.plane = 8 * recs;
+    g.dim = r.gdim;
     g.nf = 2;
     g.moff = p->d_moff.as<int>();
     g.ne = p->d_ne.as<int>();
@@ -755,8 +758,9 @@ extern "C" int gd_adjoint_misfit(gd_adjoint *a, int kind, int level, const doubl
                        p->d_l_of_idx.as<int>(), rinv2, radial, nlm, nr, a->mcol.as<double>());
     GD_TRY(gd_check_launch("misfit_pack_kernel"));
     const int nm = p->mmax + 1;
-    GD_TRY(p->fb.ensure(sizeof(double) * (size_t)p->nlat2 * nm * 4));
-    GD_TRY(p->gb.ensure(sizeof(double) * (size_t)nm * p->nlat2 * 4));
+    const RecDim dim = gd_rec_dim(1, p->nlat2, true);
+    GD_TRY(p->fb.ensure(sizeof(double) * nm * dim.m * 4));
+    GD_TRY(p->gb.ensure(sizeof(double) * nm * dim.m * 4));
     SynthArgs sa{};
     sa.in = a->mcol.p;
     sa.cin = 2;
@@ -769,17 +773,16 @@ extern "C" int gd_adjoint_misfit(gd_adjoint *a, int kind, int level, const doubl
     sa.nlm = nlm;
     sa.mmax = p->mmax;
     sa.out = p->fb.p;
-    sa.nslot = 4;
-    sa.slot0 = 0;
+    sa.dim = dim;
+    sa.rstr = 4;
     sa.tab0 = gd_sht_tab(p, 0);
     GD_TRY(gd_launch_synth_scal<double>(st, sa));
     RingArgs rg{};
     gd_sht_fill_ring(p, rg, 1);
     rg.fb = p->fb.p;
-    rg.nslot_f = 4;
     rg.nfield = 1;
-    rg.fn_off[0] = 0;
-    rg.fs_off[0] = 2;
+    rg.fstr = 4;
+    rg.fdim = dim;
     rg.phys_out[0] = a->mgrid.as<double>();
     GD_TRY(gd_launch_ring<double>(st, RING_SYNTH, rg));
     GD_TRY(gd_from_device(s->ctx, a->hgrid.data(), a->mgrid.p, sizeof(double) * nlat * nlon));
@@ -804,14 +807,14 @@ extern "C" int gd_adjoint_misfit(gd_adjoint *a, int kind, int level, const doubl
     gd_sht_fill_ring(p, ra, 1);
     ra.wq = a->ones.p;
     ra.gb = p->gb.p;
-    ra.nslot_g = 4;
+    ra.gstr[0] = 4;
+    ra.gdim = dim;
     ra.nfield = 1;
     ra.phys_in[0] = a->mgrid.as<double>();
     GD_TRY(gd_launch_ring<double>(st, RING_ANALYSIS, ra));
     AnaArgs g{};
     g.gb = p->gb.p;
-    g.nslot_g = 4;
-    g.gslot0 = 0;
+    g.dim = dim;
     g.nf = 1;
     g.moff = p->d_moff.as<int>();
     g.ne = p->d_ne.as<int>();

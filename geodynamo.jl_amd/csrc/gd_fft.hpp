@@ -6,6 +6,7 @@
 // (j / Ns) Ns R + j % Ns + r Ns (Ns: the product of the earlier radices).
 #pragma once
 #include "gd_internal.hpp"
+#include "gd_sht.hpp"
 
 template <typename T> struct alignas(2 * sizeof(T)) C2 {
     T x, y;
@@ -132,40 +133,88 @@ constexpr FftStages fft_stages(int n)
                 }
     return f;
 }
+// the stage order of a direction: inverse transforms (dir > 0) start with the
+// largest radix divisible by 3 and forward ones end with it, so that on a
+// dealiased grid (nm <= n / 3) whole inputs of the first, and whole outputs of
+// the last, radix fall into the unused middle third of the orders
+constexpr FftStages fft_stages(int n, int dir)
+{
+    FftStages f = fft_stages(n), g = f;
+    int t = 0;
+    for (int s = 0; s < f.n; ++s)
+        if (f.r[s] % 3 == 0 && (f.r[t] % 3 != 0 || f.r[s] > f.r[t])) t = s;
+    int k = 0;
+    g.r[k++] = f.r[t];
+    for (int s = 0; s < f.n; ++s)
+        if (s != t) g.r[k++] = f.r[s];
+    if (dir < 0)
+        for (int s = 0; 2 * s < f.n; ++s) {
+            const int x = g.r[s];
+            g.r[s] = g.r[f.n - 1 - s];
+            g.r[f.n - 1 - s] = x;
+        }
+    return g;
+}
+
+// Elements k = r n / R .. (r + 1) n / R - 1 of a packed Hermitian spectrum:
+// used ones are k < nm (order k) and n - k < nm (order n - k), nm <= n / 2, and
+// nm <= n / 3 with DEAL
+enum { PART_LOW = 0, PART_HIGH = 1, PART_NONE = 2, PART_BOTH = 3 };
+constexpr int fft_part(int r, int R, bool deal)
+{
+    if (deal && 3 * r >= R && 3 * (r + 1) <= 2 * R) return PART_NONE;
+    return 2 * (r + 1) <= R ? PART_LOW : 2 * r >= R ? PART_HIGH : PART_BOTH;
+}
 
 // Twiddles of the stages after the first, e^(-2 pi i r k / (Ns R)) at
 // [offset + r Ns + k] (r < R, k < Ns), so that consecutive k are consecutive:
-// stage 1 at offset 0, stage 2 after it.
-constexpr int fft_tw_off(FftStages f, int s) { return s == 2 ? f.r[0] * f.r[1] : 0; }
+// stage 1 at offset 0, stage 2 after it, the forward order's after the inverse's.
 constexpr int fft_tw_len(FftStages f) { return f.r[0] * f.r[1] + (f.n == 3 ? f.r[0] * f.r[1] * f.r[2] : 0); }
+constexpr int fft_tw_off(int n, int dir, int s)
+{
+    const FftStages f = fft_stages(n, dir);
+    return (dir < 0 ? fft_tw_len(fft_stages(n, 1)) : 0) + (s == 2 ? f.r[0] * f.r[1] : 0);
+}
 
 // LDS positions of the two exchanges (padded against bank conflicts): after
 // the first stage element e sits at e + (e / r0) P1, after the second of three
-// at e + (e / (r0 r1)) P2; LD is the stride from one transform to the next,
-// congruent to 2 (16-byte elements) or 4 (8-byte) modulo a bank row so that
-// lanes on different transforms fall on different banks.
-template <typename T, int N> struct FftLds {
-    static constexpr FftStages f = fft_stages(N);
+// at e + (e / (r0 r1)) P2; ld(w) is the stride from one transform to the next,
+// congruent to w modulo a bank row of M elements: lanes on 16 (8-byte) or 8
+// (16-byte elements) consecutive transforms fall on different banks with
+// w = 1, lanes on four of them and neighbouring elements with w = M / 4.
+template <typename T, int N, int DIR> struct FftLds {
+    static constexpr FftStages f = fft_stages(N, DIR);
     static constexpr int P1 = f.r[0] % 2 == 0 ? 1 : 0;
     static constexpr int P2 = f.n == 3 ? f.r[0] : 0;
     static constexpr int S1 = N + N / f.r[0] * P1, S2 = N + (f.n == 3 ? f.r[2] * P2 : 0);
     static constexpr int S = S1 > S2 ? S1 : S2;
-    static constexpr int M = sizeof(T) == 8 ? 8 : 16, W = sizeof(T) == 8 ? 2 : 4;
-    static constexpr int LD = S + (W - S % M + M) % M;
+};
+template <typename T, int N> struct FftRow { // both directions
+    static constexpr int S = FftLds<T, N, 1>::S > FftLds<T, N, -1>::S ? FftLds<T, N, 1>::S : FftLds<T, N, -1>::S;
+    static constexpr int M = sizeof(T) == 8 ? 8 : 16;
+    static constexpr int ld(int w) { return S + (w - S % M + M) % M; }
 };
 
-// butterfly j of stage s (1 or 2): its inputs from one transform's LDS row
-// with the twiddles applied, transformed in place of v
+// twiddles of butterfly j of stage s (1 or 2); loaded before the barrier that
+// makes the stage's inputs visible, so that their latency is hidden by it
 template <typename T, int N, int S, int DIR>
-__device__ __forceinline__ void fft_lds_stage(const C2<T> *x, const C2<T> *tws, int j, C2<T> *v)
+__device__ __forceinline__ void fft_tw_load(const C2<T> *tws, int j, C2<T> *w)
 {
-    using F = FftLds<T, N>;
-    constexpr FftStages f = F::f;
+    constexpr FftStages f = fft_stages(N, DIR);
     constexpr int R = f.r[S], Ns = S == 1 ? f.r[0] : f.r[0] * f.r[1], nb = N / R;
-    const C2<T> *tw = tws + fft_tw_off(f, S) + (nb == Ns ? j : j % Ns);
-    C2<T> w[R];
+    const C2<T> *tw = tws + fft_tw_off(N, DIR, S) + (nb == Ns ? j : j % Ns);
 #pragma unroll
     for (int r = 1; r < R; ++r) w[r] = tw[r * Ns];
+}
+
+// butterfly j of stage s: its inputs from one transform's LDS row, times the
+// twiddles, transformed
+template <typename T, int N, int S, int DIR>
+__device__ __forceinline__ void fft_lds_stage(const C2<T> *x, const C2<T> *w, int j, C2<T> *v)
+{
+    using F = FftLds<T, N, DIR>;
+    constexpr FftStages f = F::f;
+    constexpr int R = f.r[S], nb = N / R;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const int p = S == 1 ? j + r * nb + (j / f.r[0] + r * (nb / f.r[0])) * F::P1 : j + r * (nb + F::P2);
@@ -173,16 +222,17 @@ __device__ __forceinline__ void fft_lds_stage(const C2<T> *x, const C2<T> *tws, 
     }
 #pragma unroll
     for (int r = 1; r < R; ++r) {
-        if (DIR > 0) w[r].y = -w[r].y;
-        v[r] = cmul(v[r], w[r]);
+        const C2<T> t = DIR > 0 ? C2<T>{w[r].x, -w[r].y} : w[r];
+        v[r] = cmul(v[r], t);
     }
     dft<R, DIR>(v);
 }
 
 // results of butterfly j of stage s into the next exchange
-template <typename T, int N, int S> __device__ __forceinline__ void fft_lds_put(C2<T> *x, int j, const C2<T> *v)
+template <typename T, int N, int S, int DIR>
+__device__ __forceinline__ void fft_lds_put(C2<T> *x, int j, const C2<T> *v)
 {
-    using F = FftLds<T, N>;
+    using F = FftLds<T, N, DIR>;
     constexpr FftStages f = F::f;
     if constexpr (S == 0) {
 #pragma unroll
@@ -193,4 +243,79 @@ template <typename T, int N, int S> __device__ __forceinline__ void fft_lds_put(
         for (int r = 0; r < f.r[1]; ++r)
             x[j / f.r[0] * (f.r[0] * f.r[1] + F::P2) + j % f.r[0] + r * f.r[0]] = v[r];
     }
+}
+
+// every butterfly of stage S (1 or 2) of ROWS transforms, in place in LDS (LD
+// elements from row to row), by NTHR threads: waits for the inputs and leaves
+// the results to the caller's (or the next stage's) barrier; the last stage
+// leaves them in natural order (with DEAL only those of used orders)
+template <typename T, int N, int S, int DIR, int ROWS, int NTHR, int LD, bool DEAL>
+__device__ __forceinline__ void fft_rows_stage(C2<T> *buf, const C2<T> *tws)
+{
+    constexpr FftStages f = fft_stages(N, DIR);
+    constexpr int R = f.r[S], nb = N / R, total = ROWS * nb, IT = (total + NTHR - 1) / NTHR;
+    C2<T> v[IT][R], w[R];
+    fft_tw_load<T, N, S, DIR>(tws, (int)threadIdx.x % nb, w);
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+        const int g = threadIdx.x + it * NTHR;
+        if (it > 0 && NTHR % nb != 0) fft_tw_load<T, N, S, DIR>(tws, g % nb, w);
+        if (total % NTHR == 0 || g < total) fft_lds_stage<T, N, S, DIR>(buf + g / nb * LD, w, g % nb, v[it]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+        const int g = threadIdx.x + it * NTHR;
+        if (total % NTHR == 0 || g < total) {
+            C2<T> *x = buf + g / nb * LD;
+            if constexpr (S == f.n - 1) {
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+                    if (fft_part(r, R, DEAL) != PART_NONE) x[g % nb + r * nb] = v[it][r];
+            } else {
+                fft_lds_put<T, N, S, DIR>(x, g % nb, v[it]);
+            }
+        }
+    }
+}
+
+// First stage of an inverse transform: butterfly j's inputs from the Fourier
+// slots of one component, order m's at rec + m * mstr (T elements), packed as
+// Z = X + iY of the north (X) and south (Y) rings: X_m + i Y_m at m, and
+// conj(X_m) + i conj(Y_m) at n - m (the imaginary parts of order 0 are not
+// read).  Unused orders read order 0.
+template <typename T, int N, bool DEAL>
+__device__ __forceinline__ void fft_pack_stage(const T *rec, unsigned mstr, int nm, int j, C2<T> *v)
+{
+    constexpr int R = fft_stages(N, 1).r[0], nb = N / R;
+    RingRec<T> z[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int part = fft_part(r, R, DEAL), k = j + r * nb;
+        if (part == PART_NONE) continue;
+        const int m = part == PART_LOW || (part == PART_BOTH && 2 * k < N) ? k : N - k;
+        z[r] = *reinterpret_cast<const RingRec<T> *>(rec + (m < nm ? (unsigned)m : 0u) * mstr);
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int part = fft_part(r, R, DEAL), k = j + r * nb;
+        v[r] = C2<T>{T(0), T(0)};
+        if (part == PART_NONE) continue;
+        const bool low = part == PART_LOW || (part == PART_BOTH && 2 * k < N);
+        const int m = low ? k : N - k;
+        const T s = r == 0 && j == 0 ? T(0) : low ? T(1) : T(-1);
+        if (m < nm) v[r] = C2<T>{z[r].v[0] - s * z[r].v[3], s * z[r].v[1] + z[r].v[2]};
+    }
+    dft<R, 1>(v);
+}
+
+// The Fourier slots of order m from a transform's natural-order row: split Z
+// into north X and south Y, G+- = (X +- Y) c
+template <typename T> __device__ __forceinline__ RingRec<T> fft_split(const C2<T> *b, int n, int m, T c)
+{
+    const C2<T> Z = b[m], Zc = b[m ? n - m : 0];
+    const C2<T> X = C2<T>{T(0.5) * (Z.x + Zc.x), T(0.5) * (Z.y - Zc.y)};
+    const C2<T> Y = C2<T>{T(0.5) * (Z.y + Zc.y), T(0.5) * (Zc.x - Z.x)};
+    return RingRec<T>{{(X.x + Y.x) * c, (X.y + Y.y) * c, (X.x - Y.x) * c, (X.y - Y.y) * c}};
 }

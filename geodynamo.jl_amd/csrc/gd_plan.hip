@@ -262,7 +262,8 @@ static int run_synth(gd_sht_plan *p, bool vec, const double *a_re, const double 
     const int nlm = p->nlm, nm = p->mmax + 1;
     const int cin = vec ? 4 : 2, nslot = vec ? 8 : 4;
     GD_TRY(p->syn.ensure(sizeof(T) * (size_t)nr * cin * nlm));
-    GD_TRY(p->fb.ensure(sizeof(T) * (size_t)p->nlat2 * nr * nm * nslot));
+    const RecDim dim = gd_rec_dim(nr, p->nlat2, sizeof(T) == 8);
+    GD_TRY(p->fb.ensure(sizeof(T) * nm * dim.m * nslot));
     T *syn = p->syn.as<T>();
     // vector: S := pol (b) in columns 0,1; T := tor (a) in columns 2,3
     LmPlanes cols;
@@ -291,8 +292,9 @@ static int run_synth(gd_sht_plan *p, bool vec, const double *a_re, const double 
     s.nlm = nlm;
     s.mmax = p->mmax;
     s.out = p->fb.p;
-    s.nslot = nslot;
-    s.slot0 = 0;
+    s.plane = 0;
+    s.rstr = nslot;
+    s.dim = dim;
     if (vec) {
         s.tab0 = gd_sht_tab(p, 1);
         s.tab1 = gd_sht_tab(p, 2);
@@ -305,21 +307,12 @@ static int run_synth(gd_sht_plan *p, bool vec, const double *a_re, const double 
     RingArgs r{};
     gd_sht_fill_ring(p, r, nr);
     r.fb = p->fb.p;
-    r.nslot_f = nslot;
-    if (vec) {
-        r.nfield = 2;
-        r.fn_off[0] = 0;
-        r.fs_off[0] = 4;
-        r.fn_off[1] = 2;
-        r.fs_off[1] = 6;
-        r.phys_out[0] = o0;
-        r.phys_out[1] = o1;
-    } else {
-        r.nfield = 1;
-        r.fn_off[0] = 0;
-        r.fs_off[0] = 2;
-        r.phys_out[0] = o0;
-    }
+    r.nfield = vec ? 2 : 1;
+    for (int F = 0; F < r.nfield; ++F) r.foff[F] = 4 * F;
+    r.fstr = nslot;
+    r.fdim = dim;
+    r.phys_out[0] = o0;
+    r.phys_out[1] = o1;
     GD_TRY(gd_launch_ring<T>(st, RING_SYNTH, r));
     if (adj) {
         const size_t n = (size_t)p->nlat * p->nlon * nr;
@@ -340,14 +333,19 @@ static int run_analysis(gd_sht_plan *p, bool vec, const double *f0, const double
     hipStream_t st = p->ctx->stream;
     const int nlm = p->nlm, nm = p->mmax + 1;
     const int nslot = vec ? 8 : 4;
-    GD_TRY(p->gb.ensure(sizeof(T) * (size_t)nm * p->nlat2 * nr * nslot));
+    const RecDim dim = gd_rec_dim(nr, p->nlat2, sizeof(T) == 8);
+    GD_TRY(p->gb.ensure(sizeof(T) * nm * dim.m * nslot));
     const size_t fs = (size_t)nr * nlm;
     GD_TRY(p->outm.ensure(sizeof(double) * fs * 2 * (vec ? 2 : 1)));
     RingArgs r{};
     gd_sht_fill_ring(p, r, nr);
     r.gb = p->gb.p;
-    r.nslot_g = nslot;
     r.nfield = vec ? 2 : 1;
+    for (int F = 0; F < r.nfield; ++F) {
+        r.goff[F] = 4 * F;
+        r.gstr[F] = nslot;
+    }
+    r.gdim = dim;
     r.phys_in[0] = f0;
     r.phys_in[1] = f1;
     if (adj) r.wq = p->wone.p;
@@ -355,8 +353,8 @@ static int run_analysis(gd_sht_plan *p, bool vec, const double *f0, const double
     AnaArgs a{};
     a.mm = p->prec == GD_PREC_BF16X3;
     a.gb = p->gb.p;
-    a.nslot_g = nslot;
-    a.gslot0 = 0;
+    a.plane = 0;
+    a.dim = dim;
     a.nf = 1;
     a.moff = p->d_moff.as<int>();
     a.ne = p->d_ne.as<int>();

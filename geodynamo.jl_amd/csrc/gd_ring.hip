@@ -1,11 +1,13 @@
 // gd_ring.hip -- longitude FFTs of a northern ring and its southern mirror as
-// one complex FFT (Stockham, radices 2,3,4,6,8, in LDS); RING_STEP also
-// evaluates the pointwise nonlinear products between the inverse and forward
-// FFTs, so physical-space values never leave LDS.  The boundary passes of the
-// compiled ring lengths are in gd_ring_io.hpp.
+// one complex FFT; the step modes also evaluate the pointwise nonlinear
+// products between the inverse and forward FFTs, so physical-space values
+// never leave LDS.  The ring lengths with a compiled plan are in
+// gd_ring_io.hpp (boundary passes) and gd_ring_step.hpp (step modes); here are
+// the dispatch and the runtime plan (Stockham, radices 2,3,4,6,8, in LDS) of
+// any other 2^a 3^b, and compiled plans of that form for the tangential modes'
+// most used lengths.
 #include <cmath>
 #include <cstdint>
-#include <cstdlib>
 
 #include "gd_fft.hpp"
 #include "gd_sht.hpp"
@@ -250,37 +252,25 @@ __device__ __forceinline__ void fft_ct(C2<T> *buf, const C2<T> *tw, int nfft)
     }
 }
 
-// One block per (northern node i, level r).
-// NC > 0: the ring length is the compile-time constant NC (nlon); NC = 0 uses
-// the runtime plan.
-// (i, r): the block's northern node and level (the launch's own grid, or its
-// share of a batched launch)
+// One block per (northern node i, level r) (the launch's own grid, or its share
+// of a batched launch).  NC > 0: the ring length is the compile-time constant
+// NC (nlon); NC = 0 uses the runtime plan.
 template <typename T, int MODE, int NC, class AT> __device__ __forceinline__ void ring_body(const AT &a, int i, int r)
 {
-    extern __shared__ char smem_raw[];
+    extern __shared__ __align__(16) char smem_raw[];
     const int n = NC > 0 ? NC : a.nlon, nm = a.mmax + 1;
     const int ld = ring_ld(n);
     C2<T> *tw = reinterpret_cast<C2<T> *>(smem_raw);
     C2<T> *buf = tw + n;
     __shared__ int srad[12];
-    __shared__ int sfn[16], sfs[16];
-    // The boundary layouts (RING_SYNTH writes, RING_ANALYSIS reads) are
-    // colatitude-fastest: a 128-byte line holds 16 consecutive rings of one
-    // (longitude, level).  Consecutive blocks go to different XCDs (block b to
-    // XCD b mod 8, each with its own L2), so those modes renumber the blocks
-    // for each XCD to take a contiguous range of (level, ring) and a line's
-    // pieces meet in one L2.  The step modes read and write ring-contiguous
-    // records and keep the plain order.
+    __shared__ size_t sfo[16];
     const int tid = threadIdx.x;
     constexpr int nthr = RING_THREADS;
     const int is = a.nlat - 1 - i; // southern mirror
     const C2<T> *twg = static_cast<const C2<T> *>(a.tw);
     for (int k = tid; k < n; k += nthr) tw[k] = twg[k];
     if (tid < 12) srad[tid] = a.radix[tid];
-    if (tid < 16) {
-        sfn[tid] = a.fn_off[tid];
-        sfs[tid] = a.fs_off[tid];
-    }
+    if (tid < 16) sfo[tid] = a.foff[tid];
     __syncthreads();
     // fields in / products out: compile-time for the step modes
     constexpr int NFC = MODE == RING_STEP ? 15 : MODE == RING_STEP_TANG ? 4 : MODE == RING_STEP_TANG_C ? 6
@@ -291,29 +281,26 @@ template <typename T, int MODE, int NC, class AT> __device__ __forceinline__ voi
 
     if (MODE != RING_ANALYSIS) {
         // Hermitian spectra of the north (X) and south (Y) rings packed as Z = X + iY
-        const T *src = static_cast<const T *>(a.fb) + ((size_t)i * a.nr + r) * nm * a.nslot_f;
-        // fixed trip count, fully unrolled: every thread's global loads are in
-        // flight together before the LDS stores consume them.  With a
-        // compile-time ring length the first MAXU iterations (enough for the
-        // nm <= n/3 orders of the dealiased grids) load unconditionally,
-        // clamped to the last element: a guarded load becomes a branch whose
-        // join waits for it.  Larger nm take the guarded iterations after.
+        // fixed trip count, fully unrolled: every thread's loads are in flight
+        // together before the LDS stores consume them.  With a compile-time ring
+        // length the first MAXU iterations (enough for the nm <= n/3 orders of
+        // the dealiased grids) load unconditionally, clamped to the last element:
+        // a guarded load becomes a branch whose join waits for it.  Larger nm
+        // take the guarded iterations after.
         constexpr int MAXI = 8;
         constexpr int MAXU0 = (NC > 0 && NFC > 0) ? (NFC * (NC / 3) + nthr - 1) / nthr : 0;
         constexpr int MAXU = MAXU0 < MAXI ? MAXU0 : MAXI;
         const int ne = NF * nm;
-        T xr[MAXI], xi[MAXI], yr[MAXI], yi[MAXI];
+        const size_t rec0 = r * a.fdim.l + i * a.fdim.i;
+        RingRec<T> z[MAXI];
 #pragma unroll
         for (int it = 0; it < MAXI; ++it) {
             const int e0 = tid + it * nthr;
             if (it < MAXU || e0 < ne) {
                 const int e = e0 < ne ? e0 : ne - 1;
                 const int F = e % NF, m = e / NF;
-                const T *s = src + (size_t)m * a.nslot_f;
-                xr[it] = s[sfn[F]];
-                xi[it] = s[sfn[F] + 1];
-                yr[it] = s[sfs[F]];
-                yi[it] = s[sfs[F] + 1];
+                z[it] = *reinterpret_cast<const RingRec<T> *>(static_cast<const T *>(a.fb) + sfo[F] +
+                                                              (m * a.fdim.m + rec0) * a.fstr);
             }
         }
 #pragma unroll
@@ -321,11 +308,12 @@ template <typename T, int MODE, int NC, class AT> __device__ __forceinline__ voi
             const int e = tid + it * nthr;
             if (e < NF * nm) {
                 const int F = e % NF, m = e / NF;
+                const T *v = z[it].v;
                 if (m == 0) {
-                    buf[F * ld] = C2<T>{xr[it], yr[it]};
+                    buf[F * ld] = C2<T>{v[0], v[2]};
                 } else {
-                    buf[F * ld + sk(m)] = C2<T>{xr[it] - yi[it], xi[it] + yr[it]};
-                    buf[F * ld + sk(n - m)] = C2<T>{xr[it] + yi[it], yr[it] - xi[it]};
+                    buf[F * ld + sk(m)] = C2<T>{v[0] - v[3], v[1] + v[2]};
+                    buf[F * ld + sk(n - m)] = C2<T>{v[0] + v[3], v[2] - v[1]};
                 }
             }
         }
@@ -489,39 +477,23 @@ template <typename T, int MODE, int NC, class AT> __device__ __forceinline__ voi
     const T c = static_cast<const T *>(a.wq)[i];
     T *gb = static_cast<T *>(a.gb);
     const int NPn = NPC ? NPC : NP;
-    // products np1.. go to their own records in gb2 (the scalar analysis then
-    // reads only its own slots); np1 = 0: every product in gb
-    const int np1 = a.gb2 ? a.np1 : NPn;
     for (int e = tid; e < NPn * nm; e += nthr) {
         const int P = e % NPn, m = e / NPn;
-        const C2<T> Z = buf[P * ld + sk(m)];
-        C2<T> X, Y;
-        if (m == 0) {
-            X = C2<T>{Z.x, T(0)};
-            Y = C2<T>{Z.y, T(0)};
-        } else {
-            const C2<T> Zc = buf[P * ld + sk(n - m)];
-            X = C2<T>{T(0.5) * (Z.x + Zc.x), T(0.5) * (Z.y - Zc.y)};
-            Y = C2<T>{T(0.5) * (Z.y + Zc.y), T(0.5) * (Zc.x - Z.x)};
-        }
-        const size_t rec = ((size_t)m * a.nlat2 + i) * a.nr + r;
-        T *d = P < np1 ? gb + rec * a.nslot_g + 4 * P : static_cast<T *>(a.gb2) + rec * a.nslot_g2 + 4 * (P - np1);
-        d[0] = (X.x + Y.x) * c;
-        d[1] = (X.y + Y.y) * c;
-        d[2] = (X.x - Y.x) * c;
-        d[3] = (X.y - Y.y) * c;
+        const C2<T> Z = buf[P * ld + sk(m)], Zc = buf[P * ld + sk(m ? n - m : 0)];
+        const C2<T> X = C2<T>{T(0.5) * (Z.x + Zc.x), T(0.5) * (Z.y - Zc.y)};
+        const C2<T> Y = C2<T>{T(0.5) * (Z.y + Zc.y), T(0.5) * (Zc.x - Z.x)};
+        const size_t rec = m * a.gdim.m + r * a.gdim.l + i * a.gdim.i;
+        *reinterpret_cast<RingRec<T> *>(gb + a.goff[P] + rec * a.gstr[P]) =
+            RingRec<T>{{(X.x + Y.x) * c, (X.y + Y.y) * c, (X.x - Y.x) * c, (X.y - Y.y) * c}};
     }
 }
 
+// consecutive nodes of one level on one XCD: their slots, and in the boundary
+// layouts their grid values, share cache lines
 template <typename T, int MODE, int NC> __global__ void __launch_bounds__(256) ring_kernel(RingArgs a)
 {
-    int i = blockIdx.x, r = blockIdx.y;
-    if (MODE == RING_SYNTH || MODE == RING_ANALYSIS) {
-        const int L = xcd_logical(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
-        i = L % gridDim.x;
-        r = L / gridDim.x;
-    }
-    ring_body<T, MODE, NC>(a, i, r);
+    const int L = xcd_logical(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
+    ring_body<T, MODE, NC>(a, L % gridDim.x, L / gridDim.x);
 }
 
 // The boundary passes (RING_SYNTH: Fourier -> physical rings, RING_ANALYSIS:
@@ -533,17 +505,17 @@ template <typename T, int MODE, int NC> __global__ void __launch_bounds__(256) r
 // (and their southern mirrors); the RG * NF transforms of the block share the
 // twiddles and one batched FFT.  Each transform gets the operations of the
 // one-ring form.
-template <typename T, int MODE, int NC, int RG>
+template <typename T, int MODE, int RG>
 __device__ __forceinline__ void ring_io_body(const RingArgs &a, int g, int r)
 {
     static_assert(MODE == RING_SYNTH || MODE == RING_ANALYSIS, "boundary passes only");
-    extern __shared__ char smem_raw[];
-    const int n = NC > 0 ? NC : a.nlon, nm = a.mmax + 1;
+    extern __shared__ __align__(16) char smem_raw[];
+    const int n = a.nlon, nm = a.mmax + 1;
     const int ld = ring_ld(n);
     C2<T> *tw = reinterpret_cast<C2<T> *>(smem_raw);
     C2<T> *buf = tw + n;
     __shared__ int srad[12];
-    __shared__ int sfn[16], sfs[16];
+    __shared__ size_t sfo[16];
     const int tid = threadIdx.x;
     constexpr int nthr = RING_THREADS;
     const int NF = a.nfield;
@@ -552,39 +524,35 @@ __device__ __forceinline__ void ring_io_body(const RingArgs &a, int g, int r)
     const C2<T> *twg = static_cast<const C2<T> *>(a.tw);
     for (int k = tid; k < n; k += nthr) tw[k] = twg[k];
     if (tid < 12) srad[tid] = a.radix[tid];
-    if (tid < 16) {
-        sfn[tid] = a.fn_off[tid];
-        sfs[tid] = a.fs_off[tid];
-    }
+    if (tid < 16) sfo[tid] = a.foff[tid];
     __syncthreads();
     if (MODE == RING_SYNTH) {
         // Hermitian spectra of the north (X) and south (Y) rings packed as Z = X + iY
         for (int e0 = 0; e0 < NT * nm; e0 += 8 * nthr) {
-            T xr[8], xi[8], yr[8], yi[8];
+            C2<T> xn[8], xs[8];
             // loads of 8 elements in flight before their stores; unconditional
             // (clamped to the last element): a guarded load becomes a branch
             // whose join waits for it
 #pragma unroll
             for (int it = 0; it < 8; ++it) {
                 const int e = min(e0 + tid + it * nthr, NT * nm - 1);
-                const int F = e % NF, m = (e / NF) % nm, q = e / (NF * nm);
-                const T *s = static_cast<const T *>(a.fb) + (((size_t)(i0 + q) * a.nr + r) * nm + m) * a.nslot_f;
-                xr[it] = s[sfn[F]];
-                xi[it] = s[sfn[F] + 1];
-                yr[it] = s[sfs[F]];
-                yi[it] = s[sfs[F] + 1];
+                const int F = e % NF, q = (e / NF) % nq, m = e / NT;
+                const C2<T> *p = reinterpret_cast<const C2<T> *>(
+                    static_cast<const T *>(a.fb) + sfo[F] + (m * a.fdim.m + r * a.fdim.l + (i0 + q) * a.fdim.i) * a.fstr);
+                xn[it] = p[0];
+                xs[it] = p[1];
             }
 #pragma unroll
             for (int it = 0; it < 8; ++it) {
                 const int e = e0 + tid + it * nthr;
                 if (e < NT * nm) {
-                    const int F = e % NF, m = (e / NF) % nm, q = e / (NF * nm);
+                    const int F = e % NF, q = (e / NF) % nq, m = e / NT;
                     C2<T> *b = buf + (q * NF + F) * ld;
                     if (m == 0) {
-                        b[0] = C2<T>{xr[it], yr[it]};
+                        b[0] = C2<T>{xn[it].x, xs[it].x};
                     } else {
-                        b[sk(m)] = C2<T>{xr[it] - yi[it], xi[it] + yr[it]};
-                        b[sk(n - m)] = C2<T>{xr[it] + yi[it], yr[it] - xi[it]};
+                        b[sk(m)] = C2<T>{xn[it].x - xs[it].y, xn[it].y + xs[it].x};
+                        b[sk(n - m)] = C2<T>{xn[it].x + xs[it].y, xs[it].x - xn[it].y};
                     }
                 }
             }
@@ -592,8 +560,7 @@ __device__ __forceinline__ void ring_io_body(const RingArgs &a, int g, int r)
         for (int k = nm + tid; k <= n - nm; k += nthr)
             for (int t = 0; t < NT; ++t) buf[t * ld + sk(k)] = C2<T>{T(0), T(0)};
         __syncthreads();
-        if constexpr (NC > 0) fft_ct<T, NC, +1, 0>(buf, tw, NT);
-        else fft_batch<T>(buf, tw, NT, n, ld, srad, a.nstages, +1);
+        fft_batch<T>(buf, tw, NT, n, ld, srad, a.nstages, +1);
         for (int e = tid; e < n * nq; e += nthr) {
             const int q = e % nq, j = e / nq, i = i0 + q, is = a.nlat - 1 - i;
             for (int F = 0; F < NF; ++F) {
@@ -634,12 +601,11 @@ __device__ __forceinline__ void ring_io_body(const RingArgs &a, int g, int r)
         }
     }
     __syncthreads();
-    if constexpr (NC > 0) fft_ct<T, NC, -1, 0>(buf, tw, NT);
-    else fft_batch<T>(buf, tw, NT, n, ld, srad, a.nstages, -1);
+    fft_batch<T>(buf, tw, NT, n, ld, srad, a.nstages, -1);
     // split Z into north X and south Y, form G+- = (X +- Y) * 2 pi w_i / n
     T *gb = static_cast<T *>(a.gb);
     for (int e = tid; e < NT * nm; e += nthr) {
-        const int F = e % NF, m = (e / NF) % nm, q = e / (NF * nm), i = i0 + q;
+        const int F = e % NF, q = (e / NF) % nq, m = e / NT, i = i0 + q;
         const T c = static_cast<const T *>(a.wq)[i];
         const C2<T> *b = buf + (q * NF + F) * ld;
         const C2<T> Z = b[sk(m)];
@@ -652,8 +618,8 @@ __device__ __forceinline__ void ring_io_body(const RingArgs &a, int g, int r)
             X = C2<T>{T(0.5) * (Z.x + Zc.x), T(0.5) * (Z.y - Zc.y)};
             Y = C2<T>{T(0.5) * (Z.y + Zc.y), T(0.5) * (Zc.x - Z.x)};
         }
-        const size_t rec = ((size_t)m * a.nlat2 + i) * a.nr + r;
-        T *d = gb + rec * a.nslot_g + 4 * F;
+        const size_t rec = m * a.gdim.m + r * a.gdim.l + i * a.gdim.i;
+        T *d = gb + a.goff[F] + rec * a.gstr[F];
         d[0] = (X.x + Y.x) * c;
         d[1] = (X.y + Y.y) * c;
         d[2] = (X.x - Y.x) * c;
@@ -662,10 +628,10 @@ __device__ __forceinline__ void ring_io_body(const RingArgs &a, int g, int r)
 }
 
 // blocks (ring group, level) in XCD-aware order, as the one-ring boundary form
-template <typename T, int MODE, int NC, int RG> __global__ void __launch_bounds__(256) ring_io_kernel(RingArgs a)
+template <typename T, int MODE, int RG> __global__ void __launch_bounds__(256) ring_io_kernel(RingArgs a)
 {
     const int L = xcd_logical(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
-    ring_io_body<T, MODE, NC, RG>(a, L % gridDim.x, L / gridDim.x);
+    ring_io_body<T, MODE, RG>(a, L % gridDim.x, L / gridDim.x);
 }
 
 // one grid over the ring passes of several shells (step modes): a shell's
@@ -674,15 +640,22 @@ template <typename T, int MODE, int NC> __global__ void __launch_bounds__(256) r
 {
     const int sh = b.shell_of_block[blockIdx.x];
     if (sh == BATCH_PAD) return;
-    const int loc = blockIdx.x - b.block_off[sh];
     const auto &a = batch_args(b, sh);
-    ring_body<T, MODE, NC>(a, loc % a.nlat2, loc / a.nlat2);
+    const int L = xcd_logical(blockIdx.x - b.block_off[sh], b.block_cnt[sh]);
+    ring_body<T, MODE, NC>(a, L % a.nlat2, L / a.nlat2);
 }
 } // namespace
 
 template <typename T, int MODE, int NC> static void ring_launch(hipStream_t st, dim3 grid, size_t lds, const RingArgs &a)
 {
     hipLaunchKernelGGL((ring_kernel<T, MODE, NC>), grid, dim3(RING_THREADS), lds, st, a);
+}
+
+// lengths whose tangential modes run ring_kernel's own compiled plan (the
+// measured choice: gd_ring_step.hpp)
+static bool ring_short(int nlon)
+{
+    return nlon == 48 || nlon == 96 || nlon == 144 || nlon == 192 || nlon == 288 || nlon == 384;
 }
 
 template <typename T, int MODE> static void ring_dispatch(hipStream_t st, dim3 grid, size_t lds, const RingArgs &a)
@@ -694,7 +667,6 @@ template <typename T, int MODE> static void ring_dispatch(hipStream_t st, dim3 g
     case 192: ring_launch<T, MODE, 192>(st, grid, lds, a); break;
     case 288: ring_launch<T, MODE, 288>(st, grid, lds, a); break;
     case 384: ring_launch<T, MODE, 384>(st, grid, lds, a); break;
-    case 768: ring_launch<T, MODE, 768>(st, grid, lds, a); break;
     default: ring_launch<T, MODE, 0>(st, grid, lds, a); break;
     }
 }
@@ -723,6 +695,9 @@ int gd_ring_tang_batchable(const RingArgs &a, bool fp64)
     GD_TRY(ring_check(RING_STEP_TANG, a, &nf));
     GD_CHECK((fp64 ? 16 : 8) * ((size_t)ring_ld(a.nlon) * nf + a.nlon) <= 160 * 1024, GD_ERR_ARG,
              "ring batch: nlon=%d needs too much LDS", a.nlon);
+    // the batched compiled plan takes dealiased grids (others run their own step)
+    GD_CHECK(ring_short(a.nlon) || !gd_ring_compiled(a.nlon) || (3 * (a.mmax + 1) <= a.nlon && gd_offsets_fit(a)),
+             GD_ERR_ARG, "ring batch: nlon=%d mmax=%d", a.nlon, a.mmax);
     return GD_OK;
 }
 
@@ -753,16 +728,18 @@ void gd_ring_stage_twiddles(int nlon, std::vector<double> &tw)
 {
     tw.clear();
     if (!gd_ring_compiled(nlon)) return;
-    const FftStages f = fft_stages(nlon);
-    tw.resize((size_t)2 * fft_tw_len(f));
-    for (int s = 1, Ns = f.r[0]; s < f.n; Ns *= f.r[s], ++s)
-        for (int r = 0; r < f.r[s]; ++r)
-            for (int k = 0; k < Ns; ++k) {
-                const double ang = 2.0 * M_PI * (double)(r * k) / (double)(Ns * f.r[s]);
-                double *o = tw.data() + 2 * (size_t)(fft_tw_off(f, s) + r * Ns + k);
-                o[0] = std::cos(ang);
-                o[1] = -std::sin(ang);
-            }
+    tw.resize((size_t)2 * (fft_tw_len(fft_stages(nlon, 1)) + fft_tw_len(fft_stages(nlon, -1))));
+    for (int dir : {1, -1}) {
+        const FftStages f = fft_stages(nlon, dir);
+        for (int s = 1, Ns = f.r[0]; s < f.n; Ns *= f.r[s], ++s)
+            for (int r = 0; r < f.r[s]; ++r)
+                for (int k = 0; k < Ns; ++k) {
+                    const double ang = 2.0 * M_PI * (double)(r * k) / (double)(Ns * f.r[s]);
+                    double *o = tw.data() + 2 * (size_t)(fft_tw_off(nlon, dir, s) + r * Ns + k);
+                    o[0] = std::cos(ang);
+                    o[1] = -std::sin(ang);
+                }
+    }
 }
 
 template <typename T> int gd_launch_ring(hipStream_t st, int mode, const RingArgs &a)
@@ -772,10 +749,6 @@ template <typename T> int gd_launch_ring(hipStream_t st, int mode, const RingArg
     if (mode == RING_SYNTH || mode == RING_ANALYSIS) {
         // the boundary passes take one scalar or one (theta, phi) pair: phys_in / phys_out [0], [1]
         GD_CHECK(nf <= 2, GD_ERR_ARG, "ring: %d fields in a boundary pass", nf);
-        // the compiled plans read and write the records in pairs and fours
-        GD_CHECK(a.nslot_f % 4 == 0 && a.nslot_g % 4 == 0 && a.fn_off[0] % 2 == 0 && a.fs_off[0] % 2 == 0 &&
-                     a.fn_off[1] % 2 == 0 && a.fs_off[1] % 2 == 0,
-                 GD_ERR_ARG, "ring: record slots not in pairs");
         if (gd_launch_ring_plan<T>(st, mode, a)) return gd_check_launch("ring_plan_kernel");
         const int rg = ring_io_rg<T>(a, nf);
         if (rg > 1) {
@@ -783,8 +756,8 @@ template <typename T> int gd_launch_ring(hipStream_t st, int mode, const RingArg
             const dim3 grid((a.nlat2 + rg - 1) / rg, a.nr);
 #define GD_RIO(MODE)                                                                                                  \
     {                                                                                                                 \
-        if (rg == 4) hipLaunchKernelGGL((ring_io_kernel<T, MODE, 0, 4>), grid, dim3(RING_THREADS), lds, st, a);       \
-        else hipLaunchKernelGGL((ring_io_kernel<T, MODE, 0, 2>), grid, dim3(RING_THREADS), lds, st, a);               \
+        if (rg == 4) hipLaunchKernelGGL((ring_io_kernel<T, MODE, 4>), grid, dim3(RING_THREADS), lds, st, a);       \
+        else hipLaunchKernelGGL((ring_io_kernel<T, MODE, 2>), grid, dim3(RING_THREADS), lds, st, a);               \
     }
             if (mode == RING_SYNTH) GD_RIO(RING_SYNTH) else GD_RIO(RING_ANALYSIS)
 #undef GD_RIO
@@ -794,19 +767,24 @@ template <typename T> int gd_launch_ring(hipStream_t st, int mode, const RingArg
     size_t lds = sizeof(C2<T>) * ((size_t)ring_ld(a.nlon) * nf + a.nlon);
     GD_CHECK(lds <= 160 * 1024, GD_ERR_ARG, "ring: LDS %zu too large", lds);
     dim3 grid(a.nlat2, a.nr);
+    if ((!ring_short(a.nlon) || (mode == RING_STEP && !(sizeof(T) == 4 && a.nlon == 384))) && gd_launch_ring_step_plan<T>(st, mode, a))
+        return gd_check_launch("ring_step_plan_kernel");
     switch (mode) {
     case RING_SYNTH: ring_launch<T, RING_SYNTH, 0>(st, grid, lds, a); break;
     case RING_ANALYSIS: ring_launch<T, RING_ANALYSIS, 0>(st, grid, lds, a); break;
     case RING_STEP_TANG: ring_dispatch<T, RING_STEP_TANG>(st, grid, lds, a); break;
     case RING_STEP_TANG_C: ring_dispatch<T, RING_STEP_TANG_C>(st, grid, lds, a); break;
     case RING_ADJ_TANG: ring_dispatch<T, RING_ADJ_TANG>(st, grid, lds, a); break;
-    default: ring_dispatch<T, RING_STEP>(st, grid, lds, a); break;
+    default:
+        if (sizeof(T) == 4 && a.nlon == 384) ring_launch<float, RING_STEP, 384>(st, grid, lds, a);
+        else ring_launch<T, RING_STEP, 0>(st, grid, lds, a);
+        break;
     }
     return gd_check_launch("ring_kernel");
 }
 
 // The tangential step's ring pass in one grid over several shells of one
-// ring length (the compile-time FFT plan of nlon where there is one)
+// ring length
 template <typename T, int NC>
 static void ring_batch_launch(hipStream_t st, const BatchRef<RingArgs> &b, int nblocks, size_t lds)
 {
@@ -816,6 +794,8 @@ static void ring_batch_launch(hipStream_t st, const BatchRef<RingArgs> &b, int n
 template <typename T> int gd_launch_ring_tang_batch(hipStream_t st, const BatchRef<RingArgs> &b, int nblocks, int nlon)
 {
     if (nblocks <= 0) return GD_OK;
+    if (!ring_short(nlon) && gd_launch_ring_tang_batch_plan<T>(st, b, nblocks, nlon))
+        return gd_check_launch("ring_step_batch_kernel");
     const size_t lds = sizeof(C2<T>) * ((size_t)ring_ld(nlon) * 4 + nlon);
     GD_CHECK(lds <= 160 * 1024, GD_ERR_ARG, "ring batch: LDS %zu too large", lds);
     switch (nlon) {
@@ -825,7 +805,6 @@ template <typename T> int gd_launch_ring_tang_batch(hipStream_t st, const BatchR
     case 192: ring_batch_launch<T, 192>(st, b, nblocks, lds); break;
     case 288: ring_batch_launch<T, 288>(st, b, nblocks, lds); break;
     case 384: ring_batch_launch<T, 384>(st, b, nblocks, lds); break;
-    case 768: ring_batch_launch<T, 768>(st, b, nblocks, lds); break;
     default: ring_batch_launch<T, 0>(st, b, nblocks, lds); break;
     }
     return gd_check_launch("ring_batch_kernel");

@@ -7,8 +7,6 @@
 //                    (l-m) even / odd partial sums over the northern nodes;
 //                    the epilogue forms north/south rings and, for vector
 //                    fields, v_theta = dP S + i Q T, v_phi = i Q S - dP T
-//  ana_kernel        the transpose contraction over the northern nodes with
-//                    G+- = Gn +- Gs, epilogue S = X_t - i Y_p, T = -i Y_t - X_p
 //  lm_tile_kernel    l-major <-> m-major planes
 #include <cmath>
 #include <cstdint>
@@ -78,21 +76,11 @@ int gd_launch_plm(hipStream_t st, const double *x, const int *moff, int lmax, in
 
 // ====================================================================== Legendre GEMMs
 namespace {
-constexpr int KT = 16; // K tile staged in LDS
 constexpr int TM = 32; // rows per tile (two 16-row MFMA blocks)
 
 template <typename T> using acc_t = typename Acc4<T>::type;
 
 template <typename T> __device__ __forceinline__ T shfl_xor3(T v) { return __shfl_xor(v, 3); }
-
-// XCD-aware block order.  Workgroup b of a launch goes to XCD b % 8, and each
-// XCD has its own L2; the blocks of one order m share their Legendre table
-// tile (and their spectral / Fourier inputs), so the logical index is built
-// so that consecutive logical blocks run on one XCD: XCD x takes the x-th
-// contiguous range of the logical order.  The m dimension is ordered
-// 0, mmax, 1, mmax-1, ... so that equal ranges carry equal work (the degree
-// count of m falls linearly with m).  (xcd_logical: gd_internal.hpp)
-__device__ __forceinline__ int paired_m(int k, int nm) { return (k & 1) ? nm - 1 - (k >> 1) : (k >> 1); }
 
 // 16-byte vector of T (stores of the staged output tiles)
 template <typename T> struct Vec16;
@@ -101,8 +89,8 @@ template <> struct Vec16<double> { using type = double2; };
 
 // Tile shape of a synthesis block: NF fields, VC virtual columns per level
 // (vector: S_re S_im T_re T_im per field, scalar: re im), NW waves of 16
-// columns each, NTILE = 16 NW columns = LT levels; RS output slots per
-// (node, level) record.
+// columns each, NTILE = 16 NW columns = LT levels; PL output planes of PS
+// slots per (node, level) record.
 // NG gradient fields (vector only: S alone, T = 0) follow the NF full fields
 // with 2 columns each: both components come from the S columns, so the zero
 // T columns are not contracted.  A full field's 4 columns must start at a
@@ -115,7 +103,8 @@ template <bool VEC, int NF, int NW, int NG = 0> struct SynthTile {
     static constexpr int GC = VC * PAIR;                        // columns per group
     static constexpr int NTILE = 16 * NW;
     static constexpr int LT = NTILE / GC * PAIR;
-    static constexpr int RS = VEC ? 8 * (NF + NG) : 4 * NF;
+    static constexpr int PL = NF + NG, PS = VEC ? 8 : 4; // output planes, slots per record
+    static constexpr int RS = PL * PS;
     static constexpr int NT = VEC ? 2 : 1; // tables: (dP, mP/sin) or P
     // virtual column -> (level within the tile, column within the level)
     __device__ static void decode(int vcol, int &lv, int &fv)
@@ -284,9 +273,8 @@ template <typename T, bool VEC, int NF, int NW, int KC, int NG = 0> constexpr si
     return 128 + sizeof(T) * (pipe > tile ? pipe : tile);
 }
 
-// The block's output tile -- TM nodes x LT levels, RS contiguous slots of each
-// (node, level, m) record -- is staged in LDS and stored as 16-byte vectors,
-// one record run after another.
+// The block's output tile -- per plane and level the records of TM consecutive
+// nodes -- is staged in LDS and stored as 16-byte vectors of those runs.
 // blk, nblk: the block's index and the block count of this synthesis (the
 // launch's own, or its share of a batched launch over several shells)
 template <typename T, bool VEC, int NF, int NW, int KC, bool VL, int NG, int MM, class AT>
@@ -319,7 +307,8 @@ __device__ __forceinline__ void synth_body(const AT &a, int blk, int nblk)
     synth_pipeline<T, VEC, NF, NW, KC, VL, NG, MM>(a, in, tab0, tab1, sA, scol, m, i0, r0, accE, accO);
     __syncthreads(); // the tile below reuses the pipeline's LDS
 
-    T *tile = sA; // [node][level][slot]
+    T *tile = sA; // [plane][level][node][slot]
+    auto rec = [&](int pl, int il, int lv_) { return tile + ((pl * LT + lv_) * TM + il) * TL::PS; };
     const int vcol = wave * 16 + (lane & 15);
     int lv, fv;
     TL::decode(vcol, lv, fv);
@@ -329,7 +318,7 @@ __device__ __forceinline__ void synth_body(const AT &a, int blk, int nblk)
         for (int v = 0; v < 4; ++v) {
             const int il = rb * 16 + acc_row<T>(lane, v);
             T on, os;
-            int srel;
+            int pl, srel;
             if constexpr (VEC) {
                 // north / south parity combination: dP flips sign once more than P, Q
                 const T dPn = accE[0][rb][v] + accO[0][rb][v], dPs = accO[0][rb][v] - accE[0][rb][v];
@@ -340,10 +329,10 @@ __device__ __forceinline__ void synth_body(const AT &a, int blk, int nblk)
                     // gradient field: theta = dP S, phi = i Q S (Q S_re -> phi_im,
                     // -Q S_im -> phi_re); the values of the full form with T = 0
                     const int gq = fv - 4 * NF, q2 = gq & 1;
-                    T *tg = tile + (il * LT + lv) * RS + 8 * (NF + (gq >> 1));
+                    T *tg = rec(NF + (gq >> 1), il, lv);
                     tg[q2] = dPn;
-                    tg[4 + q2] = dPs;
-                    tg[q2 ? 2 : 3] = q2 ? -Qn : Qn;
+                    tg[2 + q2] = dPs;
+                    tg[q2 ? 4 : 5] = q2 ? -Qn : Qn;
                     tg[q2 ? 6 : 7] = q2 ? -Qs : Qs;
                     continue;
                 }
@@ -360,15 +349,17 @@ __device__ __forceinline__ void synth_body(const AT &a, int blk, int nblk)
                     on = Qxn - dPn;
                     os = Qxs - dPs;
                 }
-                srel = 8 * (fv >> 2) + q; // + 4 for south
+                pl = fv >> 2;
+                srel = 4 * (q >> 1) + (q & 1); // + 2 for south
             } else {
                 on = accE[0][rb][v] + accO[0][rb][v];
                 os = accE[0][rb][v] - accO[0][rb][v];
-                srel = 4 * (fv >> 1) + (fv & 1); // + 2 for south
+                pl = fv >> 1;
+                srel = fv & 1; // + 2 for south
             }
-            T *t = tile + (il * LT + lv) * RS + srel;
+            T *t = rec(pl, il, lv) + srel;
             t[0] = on;
-            t[VEC ? 4 : 2] = os;
+            t[2] = os;
         }
     }
     __syncthreads();
@@ -378,12 +369,26 @@ __device__ __forceinline__ void synth_body(const AT &a, int blk, int nblk)
     T *out = static_cast<T *>(a.out);
     for (int t = tid; t < NV; t += 64 * NW) {
         const int e = t * EV;
-        const int rec = e / RS, so = e - rec * RS;
-        const int il = rec / LT, l2 = rec - il * LT;
+        // lanes along the records' runs: consecutive nodes of a (field, level), or
+        // the fields and levels side by side
+        int pl, l2, il, so;
+        if (a.dim.i == 1) {
+            const int run = e / (TM * TL::PS), w = e - run * (TM * TL::PS);
+            pl = run / LT;
+            l2 = run - pl * LT;
+            il = w / TL::PS;
+            so = w - il * TL::PS;
+        } else {
+            const int run = e / RS, w = e - run * RS;
+            il = run / LT;
+            l2 = run - il * LT;
+            pl = w / TL::PS;
+            so = w - pl * TL::PS;
+        }
         const int i = i0 + il, r = r0 + l2;
         if (i < a.nlat2 && r < a.nr) {
-            T *dst = out + (((size_t)i * a.nr + r) * nm + m) * a.nslot + a.slot0 + so;
-            *reinterpret_cast<V *>(dst) = *reinterpret_cast<const V *>(tile + e);
+            T *dst = out + pl * a.plane + (m * a.dim.m + r * a.dim.l + i * a.dim.i) * a.rstr + so;
+            *reinterpret_cast<V *>(dst) = *reinterpret_cast<const V *>(rec(pl, il, l2) + so);
         }
     }
 }
@@ -401,454 +406,6 @@ __global__ void __launch_bounds__(64 * NW) synth_batch_kernel(BatchRef<SynthArgs
     const int sh = b.shell_of_block[blockIdx.x];
     if (sh == BATCH_PAD) return;
     synth_body<T, VEC, NF, NW, KC, VL, NG, MM>(batch_args(b, sh), blockIdx.x - b.block_off[sh], b.block_cnt[sh]);
-}
-
-// ---------------------------------------------------------------- analysis
-template <typename T, bool VEC, int NF> __global__ void __launch_bounds__(64 * NF) ana_kernel(AnaArgs a)
-{
-    constexpr int NT = VEC ? 2 : 1;
-    extern __shared__ __align__(16) char smem_raw[];
-    constexpr int VC = VEC ? 4 * NF : 2 * NF;
-    constexpr int NTILE = 16 * NF;
-    constexpr int LT = NTILE / VC;
-    static_assert(NTILE * (TM + 1) <= 2 * NT * KT * (TM + NTILE), "analysis tile exceeds the pipeline LDS");
-    T *sA = reinterpret_cast<T *>(smem_raw);
-    T *sB = sA + 2 * NT * KT * TM; // A and B are double-buffered
-    const int gx = (a.maxgroup + TM - 1) / TM, gy = (a.nr + LT - 1) / LT, nmz = a.mmax + 1;
-    const int L = xcd_logical(blockIdx.x, gx * gy * 2 * nmz);
-    const int bx = L % gx, by = (L / gx) % gy, bz = L / (gx * gy);
-    const int m = paired_m(bz >> 1, nmz), p = bz & 1;
-    const int K = a.moff[m + 1] - a.moff[m], ne = a.ne[m];
-    const int Kp = p ? K - ne : ne;
-    const int kbase = a.moff[m] + (p ? ne : 0);
-    const int row0 = bx * TM, r0 = by * LT;
-    if (row0 >= Kp) return; // uniform over the block
-    const int tid = threadIdx.x, nthr = blockDim.x, wave = tid >> 6, lane = tid & 63;
-    const T *gb = static_cast<const T *>(a.gb);
-    const T *tab0 = static_cast<const T *>(a.tab0), *tab1 = static_cast<const T *>(a.tab1);
-    acc_t<T> acc[NT][2];
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int rb = 0; rb < 2; ++rb) acc[t][rb] = acc_t<T>{0, 0, 0, 0};
-
-    // software-pipelined K loop over the northern nodes (see synth_pipeline)
-    constexpr int RA = (NT * KT * TM + 64 * NF - 1) / (64 * NF);
-    constexpr int RB = NT * KT * 16 / 64;
-    constexpr int sAsz = NT * KT * TM, sBsz = NT * KT * NTILE;
-    const int nC = (a.nlat2 + KT - 1) / KT;
-    T ra[RA], rb[RB];
-    auto gload = [&](int c) {
-        const int k0 = c * KT;
-#pragma unroll
-        for (int q = 0; q < RA; ++q) {
-            const int e = tid + q * nthr;
-            T v = T(0);
-            if (e < sAsz) {
-                const int kk = e % KT, i = (e / KT) % TM, t = e / (KT * TM);
-                const int row = row0 + i;
-                if (row < Kp && k0 + kk < a.nlat2) v = (t == 0 ? tab0 : tab1)[(size_t)(kbase + row) * a.nlat2 + k0 + kk];
-            }
-            ra[q] = v;
-        }
-#pragma unroll
-        for (int q = 0; q < RB; ++q) {
-            const int e = tid + q * nthr;
-            T v = T(0);
-            if (e < sBsz) {
-                const int vv = e % NTILE, kk = (e / NTILE) % KT, t = e / (NTILE * KT);
-                const int lv = vv / VC, fv = vv - lv * VC, r = r0 + lv;
-                int comp, reim, pm;
-                if (VEC) {
-                    const int V = fv >> 2, q4 = fv & 3;
-                    comp = 2 * V + (q4 >> 1);
-                    reim = q4 & 1;
-                    // dP has southern sign -(-1)^(l+m): even group uses G-, odd G+; Q the reverse
-                    pm = (t == 0) ? (p == 0 ? 1 : 0) : p;
-                } else {
-                    comp = fv >> 1;
-                    reim = fv & 1;
-                    pm = p;
-                }
-                if (r < a.nr && k0 + kk < a.nlat2)
-                    v = gb[(((size_t)m * a.nlat2 + k0 + kk) * a.nr + r) * a.nslot_g + a.gslot0 + 4 * comp + 2 * pm + reim];
-            }
-            rb[q] = v;
-        }
-    };
-    auto sstore = [&](int b) {
-        T *A = sA + b * sAsz, *B = sB + b * sBsz;
-#pragma unroll
-        for (int q = 0; q < RA; ++q) {
-            const int e = tid + q * nthr;
-            if (e < sAsz) {
-                const int kk = e % KT, i = (e / KT) % TM, t = e / (KT * TM);
-                A[(t * KT + kk) * TM + i] = ra[q];
-            }
-        }
-#pragma unroll
-        for (int q = 0; q < RB; ++q) {
-            const int e = tid + q * nthr;
-            if (e < sBsz) B[e] = rb[q];
-        }
-    };
-    if (nC > 0) gload(0);
-    for (int c = 0; c < nC; ++c) {
-        sstore(c & 1);
-        __syncthreads();
-        if (c + 1 < nC) gload(c + 1);
-        const T *A = sA + (c & 1) * sAsz, *B = sB + (c & 1) * sBsz;
-#pragma unroll
-        for (int ks = 0; ks < KT; ks += 4) {
-#pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                const T b = B[(t * KT + ks + (lane >> 4)) * NTILE + wave * 16 + (lane & 15)];
-#pragma unroll
-                for (int rb_ = 0; rb_ < 2; ++rb_) {
-                    const T av = A[(t * KT + ks + (lane >> 4)) * TM + rb_ * 16 + (lane & 15)];
-                    acc[t][rb_] = mfma16x16x4(av, b, acc[t][rb_]);
-                }
-            }
-        }
-    }
-
-    // stage the (row x column) tile in LDS, padded against bank conflicts,
-    // then store each output column's rows (consecutive idx) contiguously
-    __syncthreads(); // the tile reuses the pipeline's LDS
-    constexpr int TMP = TM + 1;
-    T *tile = sA; // [column][row]
-    const int vcol = wave * 16 + (lane & 15);
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int row = rb * 16 + acc_row<T>(lane, v);
-            T o;
-            if constexpr (VEC) {
-                const T X = acc[0][rb][v], Y = acc[1][rb][v];
-                const T Yx = shfl_xor3(Y);
-                const int q = lane & 3;
-                if (q == 0) o = X + Yx;       // S_re
-                else if (q == 1) o = X - Yx;  // S_im
-                else if (q == 2) o = Yx - X;  // T_re
-                else o = -Yx - X;             // T_im
-            } else {
-                o = acc[0][rb][v];
-            }
-            tile[vcol * TMP + row] = o;
-        }
-    }
-    __syncthreads();
-    const size_t fs = (size_t)a.nr * a.nlm;
-    for (int t = tid; t < NTILE * TM; t += nthr) {
-        const int col = t / TM, row = t - col * TM;
-        const int lv = col / VC, fv = col - lv * VC, r = r0 + lv;
-        const int grow = row0 + row;
-        if (grow < Kp && r < a.nr) {
-            int outk, reim;
-            if constexpr (VEC) {
-                outk = 2 * (fv >> 2) + ((fv & 3) >> 1);
-                reim = fv & 1;
-            } else {
-                outk = fv >> 1;
-                reim = fv & 1;
-            }
-            double val = (double)tile[col * TMP + row];
-            const int idx = kbase + grow;
-            const int l = a.l_of_idx[idx];
-            const int sc = outk == 0 ? a.scale[0] : outk == 1 ? a.scale[1] : outk == 2 ? a.scale[2] : a.scale[3];
-            double *op = outk == 0 ? a.out[0] : outk == 1 ? a.out[1] : outk == 2 ? a.out[2] : a.out[3];
-            if (sc == 0) val = (l > 0) ? val / ((double)l * (double)(l + 1)) : 0.0;
-            else if (sc == 2) val = -val;
-            if (m == 0 && reim) val = 0.0; // imag(m=0) := 0 (shtnskit_field_functions.jl:432-435)
-            op[(size_t)reim * fs + (size_t)r * a.nlm + idx] = val;
-        }
-    }
-}
-// Analysis, table-resident form: one block of 4 waves per (row tile of TM
-// degrees, m, parity).  The block's table tile -- NT tables x TM degrees x all
-// KN (>= nlat/2, zero-padded) northern nodes -- is read from HBM once, in one
-// batch of loads, into LDS ([t][node][degree], padded rows).  The waves then
-// take the level tiles in turn (wave w: tiles w, w+4, ...); a wave keeps the
-// Fourier operand G of its tile in registers, one element per lane and
-// 4-node step, and reloads each register for its next tile as soon as the
-// MFMA that used it has issued, so the next tile's loads overlap this tile's
-// MFMAs.  STAGE: results go through a per-wave LDS tile and each output
-// column's consecutive idx are stored contiguously.
-// waves per analysis block (8 was measured slower at lmax 127 for FP32, 41 ->
-// 48 us: a wave's next-tile operand prefetch then spans fewer tiles; for FP64
-// it would exceed the register budget of a 512-thread block)
-template <typename T> constexpr int ana_waves() { return 4; }
-template <typename T, bool VEC, int NF, int KN, int MM, class AT>
-__device__ __forceinline__ void ana_res_body(const AT &a, int blk, int nblk)
-{
-    static_assert(!MM || sizeof(T) == 4, "the BF16x3 contraction takes FP32 operands");
-    constexpr int ANA_WAVES = ana_waves<T>();
-    constexpr int NT = VEC ? 2 : 1;
-    constexpr int VC = VEC ? 4 * NF : 2 * NF;
-    constexpr int LT = 16 / VC; // levels per wave tile (16 columns)
-    constexpr int KS = KN / 4;
-    constexpr int TMP = TM + 1; // output staging row stride
-    constexpr bool STAGE = sizeof(T) == 4;
-    constexpr int NA = NT * TM * KN / (64 * ANA_WAVES);
-    static_assert(NT * TM * KN % (64 * ANA_WAVES) == 0, "table tile must split evenly over the block");
-    static_assert(KN % 16 == 0, "nodes come in 16-node MFMA groups");
-    extern __shared__ __align__(16) char smem_raw[];
-    T *sA = reinterpret_cast<T *>(smem_raw);    // [t][node][TMA]
-    T *stg = sA + NT * KN * TMA;                 // [wave][16][TMP] when STAGE
-    __shared__ double sinv[TM];                  // 1 / (l(l+1)) of the tile's rows (0 at l = 0)
-    const int gx = (a.maxgroup + TM - 1) / TM, nmz = a.mmax + 1;
-    const int L = xcd_logical(blk, nblk);
-    const int bx = L % gx, bz = L / gx;
-    const int m = paired_m(bz >> 1, nmz), p = bz & 1;
-    const int K = a.moff[m + 1] - a.moff[m], ne = a.ne[m];
-    const int Kp = p ? K - ne : ne;
-    const int kbase = a.moff[m] + (p ? ne : 0);
-    const int row0 = bx * TM;
-    if (row0 >= Kp) return; // uniform over the block
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const T *gb = static_cast<const T *>(a.gb);
-    const T *tab0 = static_cast<const T *>(a.tab0), *tab1 = static_cast<const T *>(a.tab1);
-    const int k0 = a.k0, nk = a.nk; // this launch's node chunk
-    const bool accum = a.accum != 0;
-
-    if (tid < TM) {
-        const int l = row0 + tid < Kp ? a.l_of_idx[kbase + row0 + tid] : 0;
-        sinv[tid] = l > 0 ? 1.0 / ((double)l * (double)(l + 1)) : 0.0;
-    }
-    // table tile: all loads in flight together, then into LDS
-    // 16-byte loads of EV consecutive nodes where every table row is 16-byte
-    // aligned (nlat/2 a multiple of EV, the chunk start a multiple of 16)
-    constexpr int EV = 16 / (int)sizeof(T);
-    constexpr int NAV = (NT * TM * KN / EV + 64 * ANA_WAVES - 1) / (64 * ANA_WAVES);
-    using VT = typename Vec16<T>::type;
-    const bool vl = a.nlat2 % EV == 0 && nk % EV == 0 && ((uintptr_t)tab0 % 16) == 0 &&
-                    (NT == 1 || ((uintptr_t)tab1 % 16) == 0);
-    if (vl) {
-        VT ra[NAV];
-#pragma unroll
-        for (int q = 0; q < NAV; ++q) {
-            const int e = tid + q * 64 * ANA_WAVES;
-            const int t = e / (TM * KN / EV), rem = e - t * (TM * KN / EV);
-            const int i = rem / (KN / EV), k = (rem - i * (KN / EV)) * EV;
-            VT v;
-            T *pv = reinterpret_cast<T *>(&v);
-#pragma unroll
-            for (int u = 0; u < EV; ++u) pv[u] = T(0);
-            if (e < NT * TM * KN / EV && row0 + i < Kp && k < nk)
-                v = *reinterpret_cast<const VT *>((t == 0 ? tab0 : tab1) + (size_t)(kbase + row0 + i) * a.nlat2 + k0 + k);
-            ra[q] = v;
-        }
-#pragma unroll
-        for (int q = 0; q < NAV; ++q) {
-            const int e = tid + q * 64 * ANA_WAVES;
-            const int t = e / (TM * KN / EV), rem = e - t * (TM * KN / EV);
-            const int i = rem / (KN / EV), k = (rem - i * (KN / EV)) * EV;
-            const T *pv = reinterpret_cast<const T *>(&ra[q]);
-            if (e < NT * TM * KN / EV)
-#pragma unroll
-                for (int u = 0; u < EV; ++u) sA[(t * KN + k + u) * TMA + i] = pv[u];
-        }
-    } else {
-        T ra[NA];
-#pragma unroll
-        for (int q = 0; q < NA; ++q) {
-            const int e = tid + q * 64 * ANA_WAVES;
-            const int t = e / (TM * KN), rem = e - t * (TM * KN);
-            const int i = rem / KN, k = rem - i * KN;
-            T v = T(0);
-            if (row0 + i < Kp && k < nk) v = (t == 0 ? tab0 : tab1)[(size_t)(kbase + row0 + i) * a.nlat2 + k0 + k];
-            ra[q] = v;
-        }
-#pragma unroll
-        for (int q = 0; q < NA; ++q) {
-            const int e = tid + q * 64 * ANA_WAVES;
-            const int t = e / (TM * KN), rem = e - t * (TM * KN);
-            const int i = rem / KN, k = rem - i * KN;
-            sA[(t * KN + k) * TMA + i] = ra[q];
-        }
-    }
-
-    // this lane's column of a wave tile, and its G slot for table t
-    const int c = lane & 15, kq = lane >> 4;
-    const int lv = c / VC, fv = c - lv * VC;
-    int slot[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        int comp, reim, pm;
-        if constexpr (VEC) {
-            const int V = fv >> 2, q4 = fv & 3;
-            comp = 2 * V + (q4 >> 1);
-            reim = q4 & 1;
-            // dP has southern sign -(-1)^(l+m): even group uses G-, odd G+; Q the reverse
-            pm = (t == 0) ? (p == 0 ? 1 : 0) : p;
-        } else {
-            comp = fv >> 1;
-            reim = fv & 1;
-            pm = p;
-        }
-        slot[t] = a.gslot0 + 4 * comp + 2 * pm + reim;
-    }
-    const int ntiles = (a.nr + LT - 1) / LT;
-    const int niter = (ntiles + ANA_WAVES - 1) / ANA_WAVES;
-    // node of MFMA step ks for this lane: within each group of 16 nodes, lane
-    // group kq takes nodes 4kq .. 4kq+3 over 4 steps (A is indexed the same way)
-    auto node = [&](int ks) { return (ks >> 2) * 16 + 4 * kq + (ks & 3); };
-    const size_t nstride = (size_t)a.nr * a.nslot_g; // one node further in GB
-    const T *gm = gb + (size_t)m * a.nlat2 * nstride;
-    // Unconditional at clamped indices (a guarded load becomes a branch, and
-    // after branches that may skip loads the compiler waits for all of them
-    // at the next use): a node past the chunk meets table rows that are zero
-    // in LDS, and a level past nr (or a tile past the last) belongs to an
-    // output column that is never stored.
-    auto gload = [&](int tile, int t, int ks) {
-        const int r = min(tile * LT + lv, a.nr - 1), k = min(node(ks), nk - 1);
-        return gm[(size_t)(k0 + k) * nstride + (size_t)r * a.nslot_g + slot[t]];
-    };
-    T b[NT][KS];
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-        for (int t = 0; t < NT; ++t) b[t][ks] = gload(wave, t, ks);
-    __syncthreads(); // table tile in LDS
-
-    const size_t fs = (size_t)a.nr * a.nlm;
-    T *wst = stg + wave * 16 * TMP;
-    for (int it = 0; it < niter; ++it) {
-        const int tile = it * ANA_WAVES + wave, next = tile + ANA_WAVES;
-        acc_t<T> acc[NT][2];
-#pragma unroll
-        for (int t = 0; t < NT; ++t) acc[t][0] = acc[t][1] = acc_t<T>{0, 0, 0, 0};
-        if constexpr (MM) {
-            // BF16x3: each 16-node group (4 steps, lane group kq on nodes 4kq+j)
-            // as one split-precision 16x16x16 BF16 contraction
-#pragma unroll
-            for (int h = 0; h < KS / 4; ++h) {
-#pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    const Bf16Pair bp = bf16_split4(b[t][4 * h], b[t][4 * h + 1], b[t][4 * h + 2], b[t][4 * h + 3]);
-#pragma unroll
-                    for (int rb = 0; rb < 2; ++rb) {
-                        const T *A0 = sA + (t * KN + 16 * h + 4 * kq) * TMA + rb * 16 + c;
-                        const Bf16Pair ap = bf16_split4(A0[0], A0[TMA], A0[2 * TMA], A0[3 * TMA]);
-                        acc[t][rb] = mfma_bf16x3(ap, bp, acc[t][rb]);
-                    }
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) b[t][4 * h + j] = gload(next, t, 4 * h + j);
-                }
-            }
-        } else {
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-#pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    const T *Ak = sA + (t * KN + node(ks)) * TMA;
-                    acc[t][0] = mfma16x16x4(Ak[c], b[t][ks], acc[t][0]);
-                    acc[t][1] = mfma16x16x4(Ak[16 + c], b[t][ks], acc[t][1]);
-                    b[t][ks] = gload(next, t, ks);
-                }
-            }
-        }
-        if (tile >= ntiles) continue; // uniform over the wave
-        const int r = tile * LT + lv;
-#pragma unroll
-        for (int rb = 0; rb < 2; ++rb) {
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int row = rb * 16 + acc_row<T>(lane, v);
-                T o;
-                if constexpr (VEC) {
-                    const T X = acc[0][rb][v], Y = acc[1][rb][v];
-                    const T Yx = shfl_xor3(Y);
-                    const int q = lane & 3;
-                    if (q == 0) o = X + Yx;       // S_re
-                    else if (q == 1) o = X - Yx;  // S_im
-                    else if (q == 2) o = Yx - X;  // T_re
-                    else o = -Yx - X;             // T_im
-                } else {
-                    o = acc[0][rb][v];
-                }
-                if constexpr (STAGE) {
-                    wst[c * TMP + row] = o;
-                } else {
-                    const int grow = row0 + row;
-                    if (grow < Kp && r < a.nr) {
-                        int outk, reim;
-                        if constexpr (VEC) {
-                            outk = 2 * (fv >> 2) + ((fv & 3) >> 1);
-                            reim = fv & 1;
-                        } else {
-                            outk = fv >> 1;
-                            reim = fv & 1;
-                        }
-                        double val = (double)o;
-                        const int idx = kbase + grow;
-                        const int sc = a.scale[outk];
-                        if (sc == 0) val *= sinv[row];
-                        else if (sc == 2) val = -val;
-                        if (m == 0 && reim) val = 0.0; // imag(m=0) := 0 (shtnskit_field_functions.jl:432-435)
-                        double *dst = a.out[outk] + (size_t)reim * fs + (size_t)r * a.nlm + idx;
-                        *dst = accum ? *dst + val : val;
-                    }
-                }
-            }
-        }
-        if constexpr (STAGE) {
-            // the wave reads back what its own lanes wrote: LDS executes one
-            // wave's accesses in order; the fence keeps the compiler from
-            // reordering them
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-#pragma unroll
-            for (int q = 0; q < 16 * TM / 64; ++q) {
-                const int e = lane + 64 * q;
-                const int col = e / TM, row = e - col * TM;
-                const int lv2 = col / VC, fv2 = col - lv2 * VC, r2 = tile * LT + lv2;
-                const int grow = row0 + row;
-                if (grow < Kp && r2 < a.nr) {
-                    int outk, reim;
-                    if constexpr (VEC) {
-                        outk = 2 * (fv2 >> 2) + ((fv2 & 3) >> 1);
-                        reim = fv2 & 1;
-                    } else {
-                        outk = fv2 >> 1;
-                        reim = fv2 & 1;
-                    }
-                    double val = (double)wst[col * TMP + row];
-                    const int idx = kbase + grow;
-                    const int sc = a.scale[outk];
-                    if (sc == 0) val *= sinv[row];
-                    else if (sc == 2) val = -val;
-                    if (m == 0 && reim) val = 0.0; // imag(m=0) := 0 (shtnskit_field_functions.jl:432-435)
-                    double *dst = a.out[outk] + (size_t)reim * fs + (size_t)r2 * a.nlm + idx;
-                    *dst = accum ? *dst + val : val;
-                }
-            }
-            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-        }
-    }
-}
-
-template <typename T, bool VEC, int NF, int KN, int MM = 0>
-__global__ void __launch_bounds__(64 * ana_waves<T>()) ana_res_kernel(AnaArgs a)
-{
-    ana_res_body<T, VEC, NF, KN, MM>(a, blockIdx.x, gridDim.x);
-}
-
-// one grid over the analyses of several shells (a batched step)
-template <typename T, bool VEC, int NF, int KN, int MM = 0>
-__global__ void __launch_bounds__(64 * ana_waves<T>()) ana_res_batch_kernel(BatchRef<AnaArgs> b)
-{
-    const int sh = b.shell_of_block[blockIdx.x];
-    if (sh == BATCH_PAD) return;
-    ana_res_body<T, VEC, NF, KN, MM>(batch_args(b, sh), blockIdx.x - b.block_off[sh], b.block_cnt[sh]);
-}
-
-template <typename T, bool VEC, int NF, int KN> constexpr size_t ana_res_lds()
-{
-    constexpr int NT = VEC ? 2 : 1;
-    return sizeof(T) * ((size_t)NT * KN * TMA + (sizeof(T) == 4 ? (size_t)ana_waves<T>() * 16 * (TM + 1) : 0));
 }
 
 } // namespace
@@ -879,21 +436,9 @@ static void launch_synth(hipStream_t st, const SynthArgs &a)
     launch_synth_mm<T, VEC, NF, NW, KC, NG, 0>(st, a);
 }
 
-// The staged tile is stored in 16-byte vectors: record stride and first slot
-// must be multiples of 4 elements.
-static int synth_check(const SynthArgs &a, const char *what)
-{
-    GD_CHECK(a.nslot % 4 == 0 && a.slot0 % 4 == 0, GD_ERR_ARG, "%s: nslot=%d slot0=%d not multiples of 4", what,
-             a.nslot, a.slot0);
-    return GD_OK;
-}
-
 template <typename T> int gd_launch_synth_vec(hipStream_t st, const SynthArgs &a)
 {
     GD_CHECK(!a.mm || sizeof(T) == 4, GD_ERR_ARG, "synth_vec: the BF16x3 contraction takes FP32 operands");
-    GD_TRY(synth_check(a, "synth_vec"));
-    GD_CHECK(a.slot0 + 8 * (a.nf + a.ng) <= a.nslot, GD_ERR_ARG, "synth_vec: slots %d+%d exceed %d", a.slot0,
-             8 * (a.nf + a.ng), a.nslot);
     // one full field with 1 or 2 gradient fields: 6 columns per level (two
     // levels per 12-column group, 3 waves = 8 levels) or 8 (4 waves = 8 levels)
     if (a.ng == 1 && a.nf == 1) launch_synth<T, true, 1, 3, 16, 1>(st, a);
@@ -911,80 +456,10 @@ template <typename T> int gd_launch_synth_vec(hipStream_t st, const SynthArgs &a
 template <typename T> int gd_launch_synth_scal(hipStream_t st, const SynthArgs &a)
 {
     GD_CHECK(!a.mm || sizeof(T) == 4, GD_ERR_ARG, "synth_scal: the BF16x3 contraction takes FP32 operands");
-    GD_TRY(synth_check(a, "synth_scal"));
-    GD_CHECK(a.slot0 + 4 * a.nf <= a.nslot, GD_ERR_ARG, "synth_scal: slots %d+%d exceed %d", a.slot0, 4 * a.nf, a.nslot);
     if (a.nf == 5) launch_synth<T, false, 5, 5, 16>(st, a);
     else if (a.nf == 1) launch_synth<T, false, 1, 1, 16>(st, a);
     else GD_CHECK(false, GD_ERR_ARG, "synth_scal: nf=%d (1 or 5)", a.nf);
     return gd_check_launch("synth_kernel<scal>");
-}
-
-// grid rows cover the largest parity group (maxgroup = ceil((lmax+1)/2))
-// table-resident analysis for nlat/2 <= KN; false when no instance applies
-// nodes in chunks of at most KN: the first launch stores, the others add (the
-// sum over nodes is linear; the per-row factors, signs and imag(m=0) := 0
-// apply to every partial alike)
-template <typename T, bool VEC, int NF, int KN, int MM = 0> static bool try_ana_res(hipStream_t st, const AnaArgs &a0)
-{
-    constexpr size_t lds = ana_res_lds<T, VEC, NF, KN>();
-    if (lds > 64 * 1024) return false;
-    const int gx = (a0.maxgroup + TM - 1) / TM;
-    const int nchunk = (a0.nlat2 + KN - 1) / KN;
-    for (int c = 0; c < nchunk; ++c) {
-        AnaArgs a = a0;
-        a.k0 = c * KN;
-        a.nk = min(KN, a0.nlat2 - a.k0);
-        a.accum = c > 0;
-        hipLaunchKernelGGL((ana_res_kernel<T, VEC, NF, KN, MM>), dim3(gx * 2 * (a.mmax + 1)),
-                           dim3(64 * ana_waves<T>()), lds, st, a);
-    }
-    return true;
-}
-
-template <typename T, bool VEC, int NF, int MM> static bool ana_res_mm(hipStream_t st, const AnaArgs &a)
-{
-    if (a.nlat2 <= 32) return try_ana_res<T, VEC, NF, 32, MM>(st, a);
-    if (a.nlat2 <= 48) return try_ana_res<T, VEC, NF, 48, MM>(st, a);
-    if (a.nlat2 <= 96) return try_ana_res<T, VEC, NF, 96, MM>(st, a);
-    if constexpr (sizeof(T) == 4) // the FP64 operand registers of a 128-node tile would spill
-        if (a.nlat2 <= 128) return try_ana_res<T, VEC, NF, 128, MM>(st, a);
-    return try_ana_res<T, VEC, NF, 96, MM>(st, a); // node chunks of 96
-}
-
-template <typename T, bool VEC, int NF> static bool ana_res(hipStream_t st, const AnaArgs &a)
-{
-    if constexpr (sizeof(T) == 4)
-        if (a.mm) return ana_res_mm<T, VEC, NF, 1>(st, a);
-    return ana_res_mm<T, VEC, NF, 0>(st, a);
-}
-
-template <typename T> static int launch_ana(hipStream_t st, const AnaArgs &a, bool vec, int maxgroup)
-{
-    if (vec && a.nf == 2 && ana_res<T, true, 2>(st, a)) return gd_check_launch("ana_res_kernel<vec>");
-    if (vec && a.nf == 1 && ana_res<T, true, 1>(st, a)) return gd_check_launch("ana_res_kernel<vec>");
-    if (!vec && a.nf == 1 && ana_res<T, false, 1>(st, a)) return gd_check_launch("ana_res_kernel<scal>");
-    if (!vec && a.nf == 2 && ana_res<T, false, 2>(st, a)) return gd_check_launch("ana_res_kernel<scal>");
-    // streaming form (large nlat, or LDS beyond 64 KB)
-    GD_CHECK(!a.mm, GD_ERR_ARG, "ana: the BF16x3 contraction has no streaming form (nlat/2=%d)", a.nlat2);
-    const int VC = vec ? 4 * a.nf : 2 * a.nf;
-    const int LT = 16 * a.nf / VC;
-    dim3 grid(((maxgroup + TM - 1) / TM) * ((a.nr + LT - 1) / LT) * 2 * (a.mmax + 1));
-    const int NT = vec ? 2 : 1;
-    size_t lds = sizeof(T) * 2 * (NT * KT * TM + NT * KT * 16 * a.nf);
-    if (vec && a.nf == 2) hipLaunchKernelGGL((ana_kernel<T, true, 2>), grid, dim3(128), lds, st, a);
-    else if (vec && a.nf == 1) hipLaunchKernelGGL((ana_kernel<T, true, 1>), grid, dim3(64), lds, st, a);
-    else if (!vec && a.nf == 1) hipLaunchKernelGGL((ana_kernel<T, false, 1>), grid, dim3(64), lds, st, a);
-    else GD_CHECK(false, GD_ERR_ARG, "ana: nf=%d", a.nf);
-    return gd_check_launch(vec ? "ana_kernel<vec>" : "ana_kernel<scal>");
-}
-
-template <typename T> int gd_launch_ana(hipStream_t st, const AnaArgs &a, bool vec, int maxgroup)
-{
-    GD_CHECK(!a.mm || sizeof(T) == 4, GD_ERR_ARG, "ana: the BF16x3 contraction takes FP32 operands");
-    GD_CHECK(a.nf >= 1 && a.nf <= (vec ? 2 : 5), GD_ERR_ARG, "ana: nf=%d", a.nf);
-    AnaArgs b = a;
-    b.maxgroup = maxgroup;
-    return launch_ana<T>(st, b, vec, maxgroup);
 }
 
 // ---------------------------------------------------------------- batched step launches
@@ -1053,65 +528,11 @@ template int gd_launch_synth_tang_tile<double>(hipStream_t, const SynthArgs &, i
 // its own launch, and the 16-byte table form (VL) that the batched kernel has
 int gd_synth_tang_batchable(const SynthArgs &a)
 {
-    GD_TRY(synth_check(a, "synth batch"));
-    GD_CHECK(a.nf == 1 && a.ng == 1 && a.slot0 + 16 <= a.nslot, GD_ERR_ARG, "synth batch: nf=%d ng=%d slots %d/%d",
-             a.nf, a.ng, a.slot0, a.nslot);
+    GD_CHECK(a.nf == 1 && a.ng == 1, GD_ERR_ARG, "synth batch: nf=%d ng=%d", a.nf, a.ng);
     GD_CHECK(a.nlat2 % 4 == 0 && (uintptr_t)a.tab0 % 16 == 0 && (uintptr_t)a.tab1 % 16 == 0, GD_ERR_ARG,
              "synth batch: nlat/2=%d needs 16-byte table rows", a.nlat2);
     return GD_OK;
 }
-
-// node tile of the table-resident analysis for nlat/2 (0: not in one chunk)
-int gd_ana_kn(int nlat2, bool fp64)
-{
-    if (nlat2 <= 32) return 32;
-    if (nlat2 <= 48) return 48;
-    if (nlat2 <= 96) return 96;
-    if (!fp64 && nlat2 <= 128) return 128;
-    return 0;
-}
-
-int gd_ana_blocks(const AnaArgs &a) { return ((a.maxgroup + TM - 1) / TM) * 2 * (a.mmax + 1); }
-
-template <typename T, bool VEC, int KN, int MM>
-static void ana_batch_launch(hipStream_t st, const BatchRef<AnaArgs> &b, int nblocks)
-{
-    constexpr size_t lds = ana_res_lds<T, VEC, 1, KN>();
-    hipLaunchKernelGGL((ana_res_batch_kernel<T, VEC, 1, KN, MM>), dim3(nblocks), dim3(64 * ana_waves<T>()), lds, st, b);
-}
-
-template <typename T, bool VEC, int KN> static void ana_batch_mm(hipStream_t st, const BatchRef<AnaArgs> &b, int nblocks, int mm)
-{
-    if constexpr (sizeof(T) == 4) {
-        if (mm) {
-            ana_batch_launch<T, VEC, KN, 1>(st, b, nblocks);
-            return;
-        }
-    }
-    ana_batch_launch<T, VEC, KN, 0>(st, b, nblocks);
-}
-
-template <typename T>
-int gd_launch_ana_batch(hipStream_t st, const BatchRef<AnaArgs> &b, int nblocks, bool vec, int kn, int mm)
-{
-    GD_CHECK(!mm || sizeof(T) == 4, GD_ERR_ARG, "ana batch: the BF16x3 contraction takes FP32 operands");
-    if (nblocks <= 0) return GD_OK;
-    switch (kn) {
-    case 32: vec ? ana_batch_mm<T, true, 32>(st, b, nblocks, mm) : ana_batch_mm<T, false, 32>(st, b, nblocks, mm); break;
-    case 48: vec ? ana_batch_mm<T, true, 48>(st, b, nblocks, mm) : ana_batch_mm<T, false, 48>(st, b, nblocks, mm); break;
-    case 96: vec ? ana_batch_mm<T, true, 96>(st, b, nblocks, mm) : ana_batch_mm<T, false, 96>(st, b, nblocks, mm); break;
-    case 128:
-        if constexpr (sizeof(T) == 4) {
-            vec ? ana_batch_mm<T, true, 128>(st, b, nblocks, mm) : ana_batch_mm<T, false, 128>(st, b, nblocks, mm);
-            break;
-        }
-        [[fallthrough]];
-    default: GD_CHECK(false, GD_ERR_ARG, "ana batch: node tile %d", kn);
-    }
-    return gd_check_launch("ana_res_batch_kernel");
-}
-template int gd_launch_ana_batch<float>(hipStream_t, const BatchRef<AnaArgs> &, int, bool, int, int);
-template int gd_launch_ana_batch<double>(hipStream_t, const BatchRef<AnaArgs> &, int, bool, int, int);
 
 // ====================================================================== l-major <-> m-major planes
 // One block moves a 32 x 32 (m, l) tile of one (plane, level) through LDS: in
@@ -1224,7 +645,5 @@ template int gd_launch_synth_vec<float>(hipStream_t, const SynthArgs &);
 template int gd_launch_synth_vec<double>(hipStream_t, const SynthArgs &);
 template int gd_launch_synth_scal<float>(hipStream_t, const SynthArgs &);
 template int gd_launch_synth_scal<double>(hipStream_t, const SynthArgs &);
-template int gd_launch_ana<float>(hipStream_t, const AnaArgs &, bool, int);
-template int gd_launch_ana<double>(hipStream_t, const AnaArgs &, bool, int);
 template int gd_launch_to_m<float>(hipStream_t, int, int, int, const LmPlanes &, size_t);
 template int gd_launch_to_m<double>(hipStream_t, int, int, int, const LmPlanes &, size_t);

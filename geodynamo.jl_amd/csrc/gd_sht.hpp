@@ -9,12 +9,47 @@
 // t = 0 P, 1 dP/dtheta, 2 m P / sin(theta).  Southern values follow from the
 // parity P(pi-theta) = (-1)^(l+m) P(theta) (dP flips sign once more).
 //
-// Fourier layouts (complex of the real longitude transform, m = 0..mmax):
-//   FB[i][level][m][slot]  synthesis output, north and south rings of node i
-//   GB[m][i][level][slot]  analysis input G+ = Gn + Gs, G- = Gn - Gs, already
-//                          weighted by 2 pi w_i / nlon
+// Fourier arrays (complex of the real longitude transform, m = 0..mmax), a
+// record per (m, level, node i):
+//   FB  synthesis output, north and south rings of node i: a component's four
+//       slots are (north re, im, south re, im); a scalar field has one
+//       component, a vector field two (theta, phi), 8 contiguous slots
+//   GB  analysis input, a component's four slots (G+ re, im, G- re, im) of
+//       G+ = Gn + Gs, G- = Gn - Gs, already weighted by 2 pi w_i / nlon
+// The record order is the caller's (RecDim).  The stand-alone transforms keep
+// one field's records as [m][level][i]: a Legendre block (one m) and the
+// boundary ring passes (a few consecutive nodes of one level) both move whole
+// pieces of 64 bytes and more.  The step, whose ring pass takes one node and
+// level with every field, keeps FB as [i][level][m] with the fields' slots side
+// by side (its reads are contiguous) and GB as [m][i][level].
 #pragma once
 #include "gd_internal.hpp"
+
+// a component's four slots of one record
+template <typename T> struct alignas(16) RingRec {
+    T v[4];
+};
+// record (m, lev, i) is at index m * m + lev * l + i * i (strides in records)
+struct RecDim {
+    size_t m, l, i;
+};
+// the stand-alone transforms' [m][level][i], strides padded so that a vector
+// field's levels and orders are an odd number of 128-byte lines apart, and the
+// records it spans
+inline RecDim gd_rec_dim(int nr, int nlat2, bool fp64)
+{
+    const size_t line = fp64 ? 2 : 4; // records of a vector field's line
+    size_t l = (nlat2 + line - 1) / line * line;
+    if (l / line % 2 == 0) l += line;
+    return RecDim{nr * l + (nr % 2 ? 0 : line), l, 1};
+}
+// planes of products: nv tangential components in pairs, one vector array of
+// recs records each, then the scalars
+__host__ __device__ inline size_t gd_comp_off(int c, int nv, size_t recs)
+{
+    return c < nv ? 8 * recs * (c / 2) + 4 * (c % 2) : 4 * recs * c;
+}
+__host__ __device__ inline int gd_comp_str(int c, int nv) { return c < nv ? 8 : 4; }
 
 struct SynthArgs {
     const void *in;       // T*, [col][idx], col = level*cin + c
@@ -25,26 +60,30 @@ struct SynthArgs {
     const void *tab1;     // vector: Q = m P / sin
     const int *moff, *ne;
     int nlat2, nr, nlm, mmax;
-    void *out;            // T*, FB
-    int nslot, slot0;     // vector field f -> slot0 + 8f + 4h + (2c + reim); scalar -> slot0 + 4f + 2h + reim
+    void *out;            // T*, FB: field f's record at out + f * plane + rstr * index
+    size_t plane;         // elements from one field to the next
+    int rstr;             // elements from record to record
+    RecDim dim;
     int ng;               // vector: gradient fields (S only, T = 0) after the nf full ones; colmap
                           // then lists 4 nf + 2 ng columns (S_re S_im per gradient field)
     int mm;               // 1: BF16x3 split-precision contraction (FP32 operands), 0: native MFMA
 };
 
 struct AnaArgs {
-    const void *gb;       // T*, GB
-    int nslot_g, gslot0;  // component k of field f: gslot0 + 4*(comp index) + 2*pm + reim
+    const void *gb;       // T*, GB: field f's record at gb + f * plane + index * (4 or 8)
+    size_t plane;         // elements from one field to the next
+    RecDim dim;
     int nf;               // vector fields (components 2V, 2V+1) or scalar fields
     const void *tab0, *tab1;
     const int *moff, *ne, *l_of_idx;
     int nlat2, nr, nlm, mmax;
-    int maxgroup;         // largest parity group, ceil((lmax+1)/2); set by gd_launch_ana
+    int maxgroup;         // largest parity group, ceil((lmax+1)/2); set by gd_ana_plan
     // outputs, FP64 m-major [reim][level][idx]; vector field V: out[2V] gets S, out[2V+1] gets T
     double *out[4];
     int scale[4];         // 0: /l(l+1) (0 at l=0), 1: x1, 2: x(-1)
-    // table-resident analysis in node chunks (set by its launcher): nodes
-    // k0 .. k0 + nk - 1, accum = 1 adds to out instead of storing
+    int tw;               // level tiles per wave; set by gd_ana_plan
+    // node chunk (set by the launcher): nodes k0 .. k0 + nk - 1, accum = 1 adds
+    // to out instead of storing
     int k0, nk, accum;
     int mm;               // 1: BF16x3 split-precision contraction (FP32 operands), 0: native MFMA
 };
@@ -52,14 +91,12 @@ struct AnaArgs {
 struct RingArgs {
     const void *fb;       // T*
     void *gb;             // T*
-    int nslot_f, nslot_g;
-    // optional second analysis input: products np1 .. (the scalar analysis's)
-    // in their own records GB2[m][i][level][nslot_g2]; gb2 = null keeps every
-    // product in GB
-    void *gb2;
-    int nslot_g2, np1;
     int nfield;           // real fields to synthesise (SYNTH/STEP) or analyse (ANALYSIS)
-    int fn_off[16], fs_off[16]; // FB slot (re) of north / south spectra of each field
+    // a real field's four slots of a record: fb + foff + index * fstr (16-byte
+    // aligned), a product's: gb + goff + index * gstr
+    size_t foff[16], goff[5];
+    RecDim fdim, gdim;
+    int fstr, gstr[5];
     const double *phys_in[2];
     double *phys_out[2];
     const void *tw;       // T2[nlon], e^{-2 pi i k / nlon}
@@ -85,6 +122,15 @@ struct RingArgs {
 enum { RING_SYNTH = 0, RING_ANALYSIS = 1, RING_STEP = 2, RING_STEP_TANG = 3, RING_STEP_TANG_C = 4,
        RING_ADJ_TANG = 5 };
 
+// XCD-aware block order.  Workgroup b of a launch goes to XCD b % 8, and each
+// XCD has its own L2; the blocks of one order m share their Legendre table
+// tile (and their spectral / Fourier inputs), so the logical index is built
+// so that consecutive logical blocks run on one XCD: XCD x takes the x-th
+// contiguous range of the logical order.  The m dimension is ordered
+// 0, mmax, 1, mmax-1, ... so that equal ranges carry equal work (the degree
+// count of m falls linearly with m).
+__device__ __forceinline__ int paired_m(int k, int nm) { return (k & 1) ? nm - 1 - (k >> 1) : (k >> 1); }
+
 int gd_launch_plm(hipStream_t st, const double *x, const int *moff, int lmax, int mmax, int nlat2, double *tab64,
                   float *tab32, int nlm);
 template <typename T> int gd_launch_synth_vec(hipStream_t st, const SynthArgs &a);
@@ -98,6 +144,12 @@ template <typename T> int gd_launch_ring(hipStream_t st, int mode, const RingArg
     GD_RING_LEN(243) GD_RING_LEN(256) GD_RING_LEN(288) GD_RING_LEN(324) GD_RING_LEN(384) GD_RING_LEN(432)        \
     GD_RING_LEN(486) GD_RING_LEN(512) GD_RING_LEN(576) GD_RING_LEN(648) GD_RING_LEN(729) GD_RING_LEN(768)
 bool gd_ring_compiled(int nlon);
+// offsets along m fit 32 bits (the compiled plans' addresses)
+inline bool gd_offsets_fit(const RingArgs &a)
+{
+    const size_t lim = (size_t)1 << 31, nm = a.mmax + 1;
+    return nm * a.fdim.m * a.fstr < lim && nm * a.gdim.m * 8 < lim;
+}
 // stage twiddles of the compiled plan of nlon, e^{-i angle} as (re, im) pairs
 void gd_ring_stage_twiddles(int nlon, std::vector<double> &tw);
 // a boundary pass (RING_SYNTH, RING_ANALYSIS; 1 or 2 fields) by the compiled
@@ -105,6 +157,14 @@ void gd_ring_stage_twiddles(int nlon, std::vector<double> &tw);
 template <typename T> bool gd_launch_ring_plan(hipStream_t st, int mode, const RingArgs &a);
 template <> bool gd_launch_ring_plan<float>(hipStream_t st, int mode, const RingArgs &a);
 template <> bool gd_launch_ring_plan<double>(hipStream_t st, int mode, const RingArgs &a);
+// a step mode by the compiled plan of its ring length, and the tangential
+// step's batched launch; false where there is none
+template <typename T> bool gd_launch_ring_step_plan(hipStream_t st, int mode, const RingArgs &a);
+template <> bool gd_launch_ring_step_plan<float>(hipStream_t st, int mode, const RingArgs &a);
+template <> bool gd_launch_ring_step_plan<double>(hipStream_t st, int mode, const RingArgs &a);
+template <typename T> bool gd_launch_ring_tang_batch_plan(hipStream_t st, const BatchRef<RingArgs> &b, int nblocks, int nlon);
+template <> bool gd_launch_ring_tang_batch_plan<float>(hipStream_t st, const BatchRef<RingArgs> &b, int nblocks, int nlon);
+template <> bool gd_launch_ring_tang_batch_plan<double>(hipStream_t st, const BatchRef<RingArgs> &b, int nblocks, int nlon);
 // up to LM_MAXPLANES planes between the l-major layout of the interface
 // (level stride nlm) and the m-major device layout, one launch for all:
 // to_m writes element type T with dst_ls elements from level to level (nlm for
@@ -127,8 +187,8 @@ int gd_launch_from_m(hipStream_t st, int lmax, int mmax, int nr, const LmPlanes 
 // ---- batched step launches (gd_sht.hip): one grid over several shells'
 // launches of the tangential step's kernels, all in one compile-time form.
 // Block counts of one shell: gd_synth_tang_blocks (tile 0, 1, or 2 = FP32
-// only), nlat/2 * nr for the ring, gd_ana_blocks (args with maxgroup set) for
-// the analyses, whose node tile gd_ana_kn gives (0: several node chunks, not
+// only), nlat/2 * nr for the ring, gd_ana_blocks (args with gd_ana_plan done)
+// for the analyses, whose node tile gd_ana_kn gives (0: several node chunks, not
 // batched).
 int gd_synth_tang_blocks(const SynthArgs &a, int tile);
 bool gd_synth_tile_ok(int tile, bool fp64);
@@ -139,6 +199,7 @@ template <typename T> int gd_launch_ring_tang_batch(hipStream_t st, const BatchR
 int gd_synth_tang_batchable(const SynthArgs &a);
 int gd_ring_tang_batchable(const RingArgs &a, bool fp64);
 int gd_ana_kn(int nlat2, bool fp64);
-int gd_ana_blocks(const AnaArgs &a);
+void gd_ana_plan(AnaArgs &a, bool vec, int maxgroup);
+int gd_ana_blocks(const AnaArgs &a, bool vec);
 template <typename T>
 int gd_launch_ana_batch(hipStream_t st, const BatchRef<AnaArgs> &b, int nblocks, bool vec, int kn, int mm);

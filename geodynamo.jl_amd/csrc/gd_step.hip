@@ -207,19 +207,21 @@ static void base_args(gd_step *s, SynthArgs &a, RingArgs &r, AnaArgs &g)
     a.cin = SYNV_COLS;
     a.tab0 = gd_sht_tab(p, 1);
     a.tab1 = gd_sht_tab(p, 2);
-    a.slot0 = 0;
     r = RingArgs{};
     gd_sht_fill_ring(p, r, nr);
+    const size_t nm = p->mmax + 1;
+    a.dim = r.fdim = RecDim{1, nm, nm * nr};             // FB[i][level][m]
+    r.gdim = RecDim{(size_t)p->nlat2 * nr, 1, (size_t)nr}; // GB[m][i][level]
+    a.plane = 8;
     r.fb = s->fb.p;
     r.gb = s->gb.p;
-    // the scalar analysis's products in records of their own, so that neither
-    // analysis reads the other's slots (cache lines hold whole records)
-    r.gb2 = s->gb2.p;
     r.ro = s->d.Pm / s->d.E;
     r.coriolis_index = s->d.coriolis_index;
     g = AnaArgs{};
     g.mm = p->prec == GD_PREC_BF16X3;
     g.gb = s->gb.p;
+    g.plane = 8 * nm * r.gdim.m;
+    g.dim = r.gdim;
     g.moff = p->d_moff.as<int>();
     g.ne = p->d_ne.as<int>();
     g.l_of_idx = p->d_l_of_idx.as<int>();
@@ -227,12 +229,31 @@ static void base_args(gd_step *s, SynthArgs &a, RingArgs &r, AnaArgs &g)
     g.nr = nr;
     g.nlm = nlm;
     g.mmax = p->mmax;
-    g.maxgroup = (p->lmax + 2) / 2;
+}
+
+// The fields of a ring pass side by side in FB's records of 4 nf slots, and its
+// np products (npv of them tangential components): vector and scalar products
+// in arrays of their own so that neither analysis reads the other's slots
+static void ring_slots(gd_step *s, SynthArgs &a, RingArgs &r, int nf, int np, int npv)
+{
+    r.nfield = nf;
+    r.fstr = a.rstr = 4 * nf;
+    for (int F = 0; F < nf; ++F) r.foff[F] = 4 * F;
+    for (int P = 0; P < np; ++P) {
+        r.goff[P] = gd_comp_off(P, npv, (s->sht.mmax + 1) * r.gdim.m);
+        r.gstr[P] = gd_comp_str(P, npv);
+    }
+}
+
+static const void *scalar_products(const gd_step *s, size_t off)
+{
+    if (s->d.prec == GD_PREC_FP64) return s->gb.as<double>() + off;
+    return s->gb.as<float>() + off;
 }
 
 // The tangential step's arguments: u (S = u_pol, T = u_tor) and grad T
-// (S = T/r) only; FB records of 16 slots, 24 with the composition's gradient
-// (S = C/r) in slots 16..23.  gv: the vector analysis of the force, gs: the
+// (S = T/r) only, and with the composition its gradient (S = C/r): FB
+// records of 16 or 24 slots.  gv: the vector analysis of the force, gs: the
 // scalar analysis of -u.grad T (and -u.grad C), into nl_out; *mode: the ring
 // pass's form.
 static void tang_args(gd_step *s, double *nl_out, SynthArgs &a, RingArgs &r, AnaArgs &gv, AnaArgs &gs, int *mode)
@@ -241,8 +262,6 @@ static void tang_args(gd_step *s, double *nl_out, SynthArgs &a, RingArgs &r, Ana
     const size_t fs = s->fs;
     AnaArgs g;
     base_args(s, a, r, g);
-    const int nslot = s->comp ? 24 : 16;
-    a.nslot = nslot;
     if (s->synth_grad) {
         // u as a full field, grad T (and grad C) as gradient fields: their
         // zero toroidal columns are not contracted
@@ -255,26 +274,16 @@ static void tang_args(gd_step *s, double *nl_out, SynthArgs &a, RingArgs &r, Ana
         static const int vmap[12] = {0, 1, 2, 3, 16, 17, -1, -1, SYNV_COLS - 2, SYNV_COLS - 1, -1, -1};
         for (int k = 0; k < 20; ++k) a.colmap[k] = k < 4 * a.nf ? vmap[k] : -1;
     }
-    r.nslot_f = nslot;
     // with composition the ring also takes grad C (fields 4, 5) and forms
     // -u.grad C (compute_composition_nonlinear!, compositional.jl:219-260)
-    // as a fourth product; GB records of 12 slots, 16 with it
-    r.nfield = s->comp ? 6 : 4;
-    r.nslot_g = 8;                    // the force (products 0, 1)
-    r.np1 = 2;
-    r.nslot_g2 = s->comp ? 8 : 4;     // -u.grad T (and -u.grad C)
-    static const int fn[6] = {0, 2, 8, 10, 16, 18}, fsou[6] = {4, 6, 12, 14, 20, 22};
-    for (int F = 0; F < r.nfield; ++F) {
-        r.fn_off[F] = fn[F];
-        r.fs_off[F] = fsou[F];
-    }
+    // as a fourth product
+    if (s->comp) ring_slots(s, a, r, 6, 4, 2);
+    else ring_slots(s, a, r, 4, 3, 2);
     *mode = s->comp ? RING_STEP_TANG_C : RING_STEP_TANG;
     // force -> (pol, tor) of velocity nl (velocity.jl:331); the magnetic nl
     // is u x B = 0 here and its planes stay zero
     gv = g;
-    gv.nslot_g = r.nslot_g;
     gv.nf = 1;
-    gv.gslot0 = 0;
     gv.tab0 = gd_sht_tab(p, 1);
     gv.tab1 = gd_sht_tab(p, 2);
     gv.out[0] = nl_out + 2 * fs; // S(adv) -> u_pol
@@ -282,15 +291,14 @@ static void tang_args(gd_step *s, double *nl_out, SynthArgs &a, RingArgs &r, Ana
     gv.scale[0] = 0;
     gv.scale[1] = 0;
     gs = g;
-    gs.gb = s->gb2.p;
-    gs.nslot_g = r.nslot_g2;
-    gs.gslot0 = 0;
+    gs.gb = scalar_products(s, r.goff[2]);
+    gs.plane = g.plane / 2;
     gs.nf = 1;
     gs.tab0 = gd_sht_tab(p, 0);
     gs.tab1 = nullptr;
     gs.out[0] = nl_out + 8 * fs; // -u.grad T -> T
     gs.scale[0] = 1;
-    if (s->comp) { // and -u.grad C -> the composition's nl (GB slots 12..15)
+    if (s->comp) { // and -u.grad C -> the composition's nl
         gs.nf = 2;
         gs.out[1] = s->cnl[s->step & 1].as<double>() + 8 * fs;
         gs.scale[1] = 1;
@@ -347,7 +355,9 @@ template <typename T> static int nonlinear_T(gd_step *s, double *nl_out, hipEven
     base_args(s, a, r, g);
     {
         // vector fields u, omega, B, j (S,T) and grad T (S only)
-        a.nslot = 60;
+        // FB: the five vector fields, then u_r, omega_r, B_r, j_r, dT/dr; GB: the
+        // force, u x B, then -u.grad T
+        ring_slots(s, a, r, 15, 5, 4);
         a.nf = 5;
         static const int vmap[20] = {0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16, 17, -1, -1};
         for (int k = 0; k < 20; ++k) a.colmap[k] = vmap[k];
@@ -360,36 +370,20 @@ template <typename T> static int nonlinear_T(gd_step *s, double *nl_out, hipEven
         if (s->d.radials) {
             a.nf = 5;
             for (int k = 0; k < 20; ++k) a.colmap[k] = k < 10 ? k : -1;
-            a.slot0 = 40;
         } else {
             // the radial components are identically zero (their FB slots were
             // cleared at creation and are never written): only dT/dr is synthesised
             a.nf = 1;
             for (int k = 0; k < 20; ++k) a.colmap[k] = k < 2 ? 8 + k : -1;
-            a.slot0 = 56;
         }
+        a.out = s->fb.as<T>() + r.foff[s->d.radials ? 10 : 14];
+        a.plane = 4;
         GD_TRY(gd_launch_synth_scal<T>(st, a));
         GD_MARK(3);
-        r.nslot_f = 60;
-        r.nslot_g = 16;                   // the force and u x B (products 0..3)
-        r.np1 = 4;
-        r.nslot_g2 = 4;                   // -u.grad T
-        r.nfield = 15;
-        for (int F = 0; F < 10; ++F) {
-            const int f = F / 2, c = F % 2;
-            r.fn_off[F] = 8 * f + 2 * c;
-            r.fs_off[F] = 8 * f + 4 + 2 * c;
-        }
-        for (int F = 10; F < 15; ++F) {
-            r.fn_off[F] = 40 + 4 * (F - 10);
-            r.fs_off[F] = 40 + 4 * (F - 10) + 2;
-        }
         GD_TRY(gd_launch_ring<T>(st, RING_STEP, r));
         GD_MARK(4);
         // force -> (pol, tor) of velocity nl (velocity.jl:331); u x B -> curl (magnetic.jl:437-440)
-        g.nslot_g = 16;
         g.nf = 2;
-        g.gslot0 = 0;
         g.tab0 = gd_sht_tab(p, 1);
         g.tab1 = gd_sht_tab(p, 2);
         g.out[0] = nl_out + 2 * fs; // S(adv)   -> u_pol
@@ -402,9 +396,7 @@ template <typename T> static int nonlinear_T(gd_step *s, double *nl_out, hipEven
         g.scale[3] = 2;
         GD_TRY(gd_launch_ana<T>(st, g, true, maxgroup));
         GD_MARK(5);
-        g.gb = s->gb2.p;
-        g.nslot_g = r.nslot_g2;
-        g.gslot0 = 0;
+        g.gb = scalar_products(s, r.goff[4]);
     }
     g.nf = 1;
     g.tab0 = gd_sht_tab(p, 0);
@@ -603,7 +595,7 @@ static int step_release(gd_step *s)
     gd_adj_work_release(s);
     DevBuf *bufs[] = {&s->state[0], &s->state[1], &s->nlbuf[0], &s->nlbuf[1], &s->Lt, &s->LUt, &s->ULt, &s->rdiag2, &s->Rint, &s->nuLap, &s->nus,
                       &s->D1, &s->D2, &s->rtab, &s->synV,
-                      &s->synS, &s->fb, &s->gb, &s->gb2, &s->part, &s->eout, &s->scratch, &s->status, &s->zrow, &s->rdiag};
+                      &s->synS, &s->fb, &s->gb, &s->part, &s->eout, &s->scratch, &s->status, &s->zrow, &s->rdiag};
     for (DevBuf *b : bufs) b->release();
     for (hipEvent_t *e : {&s->ev_fork, &s->ev_ring, &s->ev_join})
         if (*e) (void)hipEventDestroy(*e);
@@ -731,9 +723,9 @@ static int step_build(gd_ctx *ctx, const gd_step_desc *d, gd_step *s)
     GD_TRY(s->nlbuf[1].ensure(sizeof(double) * s->fs * 10));
     GD_TRY(s->synV.ensure(esz * s->fs * SYNV_COLS));
     GD_TRY(s->synS.ensure(esz * s->fs * 10));
-    GD_TRY(s->fb.ensure(esz * (size_t)s->sht.nlat2 * nr * nm * 60));
-    GD_TRY(s->gb.ensure(esz * (size_t)nm * s->sht.nlat2 * nr * 16));
-    GD_TRY(s->gb2.ensure(esz * (size_t)nm * s->sht.nlat2 * nr * 8));
+    const size_t recs = (size_t)nm * nr * s->sht.nlat2;
+    GD_TRY(s->fb.ensure(esz * recs * 60));
+    GD_TRY(s->gb.ensure(esz * recs * 20));
     GD_TRY(s->part.ensure(sizeof(double) * 3 * 512));
     GD_TRY(s->eout.ensure(sizeof(double) * 4));
     GD_TRY(s->zrow.ensure(sizeof(double) * s->nlm));
@@ -745,7 +737,7 @@ static int step_build(gd_ctx *ctx, const gd_step_desc *d, gd_step *s)
     GD_HIP(hipMemsetAsync(s->nlbuf[0].p, 0, sizeof(double) * s->fs * 10, ctx->stream));
     GD_HIP(hipMemsetAsync(s->nlbuf[1].p, 0, sizeof(double) * s->fs * 10, ctx->stream));
     GD_HIP(hipMemsetAsync(s->synS.p, 0, esz * s->fs * 10, ctx->stream));
-    GD_HIP(hipMemsetAsync(s->fb.p, 0, esz * (size_t)s->sht.nlat2 * nr * nm * 60, ctx->stream));
+    GD_HIP(hipMemsetAsync(s->fb.p, 0, esz * recs * 60, ctx->stream));
     GD_HIP(hipStreamSynchronize(ctx->stream));
     s->step = 0;
     s->chain = gd_cnab2_chain_supported(nr, bw) != 0;
@@ -1431,6 +1423,7 @@ static bool fused_args(gd_step *s, int parity, ShellArgs &x)
         g->k0 = 0;
         g->nk = x.a.nlat2;
         g->accum = 0;
+        gd_ana_plan(*g, g == &x.gv, (s->sht.lmax + 2) / 2);
     }
     if (x.fm.lds_lane > 64 * 1024 || (x.fm.twist && x.fm.lds_twist > 64 * 1024)) return false;
     if (gd_synth_tang_batchable(x.a) != GD_OK || gd_ring_tang_batchable(x.r, x.fp64) != GD_OK) return false;
@@ -1504,8 +1497,8 @@ static int fused_build(gd_batch *b, int parity)
         switch (g.kind) {
         case BK_SYNTH: return gd_synth_tang_blocks(x.a, g.key);
         case BK_RING: return x.r.nlat2 * x.r.nr;
-        case BK_ANAV: return gd_ana_blocks(x.gv);
-        case BK_ANAS: return gd_ana_blocks(x.gs);
+        case BK_ANAV: return gd_ana_blocks(x.gv, true);
+        case BK_ANAS: return gd_ana_blocks(x.gs, false);
         default: return gd_cnab2_chain_blocks(x.c);
         }
     };

@@ -15,7 +15,6 @@ struct gd_step {
     DevBuf nuLap, nus;             // [nu][W*nr] nu * Laplacian band; the three diffusivities
     DevBuf D1, D2, rtab;
     DevBuf synV, synS, fb, gb;
-    DevBuf gb2;                    // the scalar analysis's Fourier records (-u.grad T, -u.grad C)
     DevBuf part, eout, scratch;
     DevBuf status;
     DevBuf zrow;                   // nlm zeros

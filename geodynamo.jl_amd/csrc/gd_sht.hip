@@ -439,26 +439,29 @@ static void launch_synth(hipStream_t st, const SynthArgs &a)
 template <typename T> int gd_launch_synth_vec(hipStream_t st, const SynthArgs &a)
 {
     GD_CHECK(!a.mm || sizeof(T) == 4, GD_ERR_ARG, "synth_vec: the BF16x3 contraction takes FP32 operands");
+    GD_CHECK((a.ng == 0 && (a.nf == 1 || a.nf == 2 || a.nf == 3 || a.nf == 5)) || (a.nf == 1 && (a.ng == 1 || a.ng == 2)) ||
+                 (a.nf == 2 && a.ng == 1),
+             GD_ERR_ARG, "synth_vec: nf=%d ng=%d", a.nf, a.ng);
+    if (gd_launch_synth_reg<T>(st, a, true)) return gd_check_launch("synth_reg_kernel<vec>");
     // one full field with 1 or 2 gradient fields: 6 columns per level (two
     // levels per 12-column group, 3 waves = 8 levels) or 8 (4 waves = 8 levels)
     if (a.ng == 1 && a.nf == 1) launch_synth<T, true, 1, 3, 16, 1>(st, a);
     else if (a.ng == 2 && a.nf == 1) launch_synth<T, true, 1, 4, 16, 2>(st, a);
     else if (a.ng == 1 && a.nf == 2) launch_synth<T, true, 2, 5, 16, 1>(st, a); // 10 columns, 5 waves = 8 levels
-    else if (a.ng != 0) GD_CHECK(false, GD_ERR_ARG, "synth_vec: nf=%d ng=%d", a.nf, a.ng);
     else if (a.nf == 5) launch_synth<T, true, 5, 5, 16>(st, a);
     else if (a.nf == 3) launch_synth<T, true, 3, 3, 16>(st, a); // 12 columns per level, 3 waves = 4 levels
     else if (a.nf == 2) launch_synth<T, true, 2, 4, 16>(st, a);
-    else if (a.nf == 1) launch_synth<T, true, 1, 1, 16>(st, a);
-    else GD_CHECK(false, GD_ERR_ARG, "synth_vec: nf=%d (1, 2, 3 or 5)", a.nf);
+    else launch_synth<T, true, 1, 1, 16>(st, a);
     return gd_check_launch("synth_kernel<vec>");
 }
 
 template <typename T> int gd_launch_synth_scal(hipStream_t st, const SynthArgs &a)
 {
     GD_CHECK(!a.mm || sizeof(T) == 4, GD_ERR_ARG, "synth_scal: the BF16x3 contraction takes FP32 operands");
+    GD_CHECK(a.nf == 1 || a.nf == 5, GD_ERR_ARG, "synth_scal: nf=%d (1 or 5)", a.nf);
+    if (gd_launch_synth_reg<T>(st, a, false)) return gd_check_launch("synth_reg_kernel<scal>");
     if (a.nf == 5) launch_synth<T, false, 5, 5, 16>(st, a);
-    else if (a.nf == 1) launch_synth<T, false, 1, 1, 16>(st, a);
-    else GD_CHECK(false, GD_ERR_ARG, "synth_scal: nf=%d (1 or 5)", a.nf);
+    else launch_synth<T, false, 1, 1, 16>(st, a);
     return gd_check_launch("synth_kernel<scal>");
 }
 

@@ -135,6 +135,8 @@ int gd_launch_plm(hipStream_t st, const double *x, const int *moff, int lmax, in
                   float *tab32, int nlm);
 template <typename T> int gd_launch_synth_vec(hipStream_t st, const SynthArgs &a);
 template <typename T> int gd_launch_synth_scal(hipStream_t st, const SynthArgs &a);
+// either synthesis with the spectral columns in registers; false beyond its degrees
+template <typename T> bool gd_launch_synth_reg(hipStream_t st, const SynthArgs &a, bool vec);
 template <typename T> int gd_launch_ana(hipStream_t st, const AnaArgs &a, bool vec, int maxgroup);
 template <typename T> int gd_launch_ring(hipStream_t st, int mode, const RingArgs &a);
 // ring lengths with a compiled FFT plan (gd_fft.hpp): every 2^a 3^b from 48 to 768

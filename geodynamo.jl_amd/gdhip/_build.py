@@ -10,7 +10,7 @@ CSRC = os.path.join(os.path.dirname(PKG), "csrc")
 INCLUDE = os.path.join(ROOT, "include")
 OBJDIR = os.path.join(os.path.dirname(PKG), "_build")
 LIB = os.path.join(PKG, "libgdhip.so")
-SOURCES = ["gd_chain.hip", "gd_core.hip", "gd_etd.hip", "gd_radial.hip", "gd_sht.hip", "gd_ana.hip", "gd_ring.hip",
+SOURCES = ["gd_chain.hip", "gd_core.hip", "gd_etd.hip", "gd_radial.hip", "gd_sht.hip", "gd_synth.hip", "gd_ana.hip", "gd_ring.hip",
            "gd_ring_io_f32.hip", "gd_ring_io_f64.hip", "gd_ring_step_f32.hip", "gd_ring_step_f64.hip", "gd_plan.hip",
            "gd_step.hip",
            "gd_restart.hip", "gd_bc.hip", "gd_adjoint.hip"]

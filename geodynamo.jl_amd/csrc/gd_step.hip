@@ -189,7 +189,7 @@ static int ensure_syn(gd_step *s)
 
 // The transform arguments common to both step forms: the synthesis a (the
 // vector columns synV into FB), the ring pass r (FB into GB, the scalar
-// analysis's products into GB2) and the analysis g (GB into nl_out).
+// analysis's products into arrays of their own) and the analysis g (GB into nl_out).
 static void base_args(gd_step *s, SynthArgs &a, RingArgs &r, AnaArgs &g)
 {
     gd_sht_plan *p = &s->sht;

@@ -283,8 +283,9 @@ __device__ __forceinline__ void fft_rows_stage(C2<T> *buf, const C2<T> *tws)
 // First stage of an inverse transform: butterfly j's inputs from the Fourier
 // slots of one component, order m's at rec + m * mstr (T elements), packed as
 // Z = X + iY of the north (X) and south (Y) rings: X_m + i Y_m at m, and
-// conj(X_m) + i conj(Y_m) at n - m (the imaginary parts of order 0 are not
-// read).  Unused orders read order 0.
+// conj(X_m) + i conj(Y_m) at n - m.  The imaginary parts of order 0 do not
+// enter, whatever they hold (they are selected away, not multiplied by 0).
+// Unused orders read order 0.
 template <typename T, int N, bool DEAL>
 __device__ __forceinline__ void fft_pack_stage(const T *rec, unsigned mstr, int nm, int j, C2<T> *v)
 {
@@ -304,18 +305,23 @@ __device__ __forceinline__ void fft_pack_stage(const T *rec, unsigned mstr, int 
         if (part == PART_NONE) continue;
         const bool low = part == PART_LOW || (part == PART_BOTH && 2 * k < N);
         const int m = low ? k : N - k;
-        const T s = r == 0 && j == 0 ? T(0) : low ? T(1) : T(-1);
-        if (m < nm) v[r] = C2<T>{z[r].v[0] - s * z[r].v[3], s * z[r].v[1] + z[r].v[2]};
+        const bool real = r == 0 && j == 0;
+        const T s = low ? T(1) : T(-1), xi = real ? T(0) : z[r].v[1], yi = real ? T(0) : z[r].v[3];
+        if (m < nm) v[r] = C2<T>{z[r].v[0] - s * yi, s * xi + z[r].v[2]};
     }
     dft<R, 1>(v);
 }
 
-// The Fourier slots of order m from a transform's natural-order row: split Z
-// into north X and south Y, G+- = (X +- Y) c
-template <typename T> __device__ __forceinline__ RingRec<T> fft_split(const C2<T> *b, int n, int m, T c)
+// The Fourier slots of order m from a transform's results Z at m and Zc at
+// n - m: split into north X and south Y, G+- = (X +- Y) c.  Order 0 of the real
+// rings is real: its imaginary parts are 0 also where Z is not finite.
+template <typename T> __device__ __forceinline__ RingRec<T> fft_split(C2<T> Z, C2<T> Zc, int m, T c)
 {
-    const C2<T> Z = b[m], Zc = b[m ? n - m : 0];
-    const C2<T> X = C2<T>{T(0.5) * (Z.x + Zc.x), T(0.5) * (Z.y - Zc.y)};
-    const C2<T> Y = C2<T>{T(0.5) * (Z.y + Zc.y), T(0.5) * (Zc.x - Z.x)};
+    C2<T> X = C2<T>{T(0.5) * (Z.x + Zc.x), T(0.5) * (Z.y - Zc.y)};
+    C2<T> Y = C2<T>{T(0.5) * (Z.y + Zc.y), T(0.5) * (Zc.x - Z.x)};
+    if (m == 0) {
+        X = C2<T>{Z.x, T(0)};
+        Y = C2<T>{Z.y, T(0)};
+    }
     return RingRec<T>{{(X.x + Y.x) * c, (X.y + Y.y) * c, (X.x - Y.x) * c, (X.y - Y.y) * c}};
 }

@@ -479,12 +479,9 @@ template <typename T, int MODE, int NC, class AT> __device__ __forceinline__ voi
     const int NPn = NPC ? NPC : NP;
     for (int e = tid; e < NPn * nm; e += nthr) {
         const int P = e % NPn, m = e / NPn;
-        const C2<T> Z = buf[P * ld + sk(m)], Zc = buf[P * ld + sk(m ? n - m : 0)];
-        const C2<T> X = C2<T>{T(0.5) * (Z.x + Zc.x), T(0.5) * (Z.y - Zc.y)};
-        const C2<T> Y = C2<T>{T(0.5) * (Z.y + Zc.y), T(0.5) * (Zc.x - Z.x)};
         const size_t rec = m * a.gdim.m + r * a.gdim.l + i * a.gdim.i;
         *reinterpret_cast<RingRec<T> *>(gb + a.goff[P] + rec * a.gstr[P]) =
-            RingRec<T>{{(X.x + Y.x) * c, (X.y + Y.y) * c, (X.x - Y.x) * c, (X.y - Y.y) * c}};
+            fft_split<T>(buf[P * ld + sk(m)], buf[P * ld + sk(m ? n - m : 0)], m, c);
     }
 }
 

@@ -112,8 +112,9 @@ __global__ void __launch_bounds__((RingIoShape<T, N, NF>::nthr)) ring_plan_kerne
             if (q >= nq) continue;
             T *rec = static_cast<T *>(a.gb) + (F ? a.goff[1] : a.goff[0]) +
                      (lev * a.gdim.l + (i0 + q) * a.gdim.i) * a.gstr[0];
+            const C2<T> *x = buf + (q * NF + F) * LD;
             *reinterpret_cast<RingRec<T> *>(rec + (unsigned)m * (unsigned)(a.gdim.m * a.gstr[0])) =
-                fft_split<T>(buf + (q * NF + F) * LD, N, m, static_cast<const T *>(a.wq)[i0 + q]);
+                fft_split<T>(x[m], x[m ? N - m : 0], m, static_cast<const T *>(a.wq)[i0 + q]);
         }
     }
 }

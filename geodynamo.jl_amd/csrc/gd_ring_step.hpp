@@ -194,7 +194,7 @@ __device__ __forceinline__ void ring_step_body(const AT &a, int L)
         const int P = e % M::NP, m = e / M::NP, str = gd_comp_str(P, M::NPV);
         T *rec = gb + gd_comp_off(P, M::NPV, recs) + rec0 * str;
         *reinterpret_cast<RingRec<T> *>(rec + (unsigned)m * ((unsigned)a.gdim.m * str)) =
-            fft_split<T>(buf + P * LD, N, m, c);
+            fft_split<T>(buf[P * LD + m], buf[P * LD + (m ? N - m : 0)], m, c);
     }
 }
 

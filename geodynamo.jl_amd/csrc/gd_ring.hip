@@ -692,10 +692,13 @@ int gd_ring_tang_batchable(const RingArgs &a, bool fp64)
     GD_TRY(ring_check(RING_STEP_TANG, a, &nf));
     GD_CHECK((fp64 ? 16 : 8) * ((size_t)ring_ld(a.nlon) * nf + a.nlon) <= 160 * 1024, GD_ERR_ARG,
              "ring batch: nlon=%d needs too much LDS", a.nlon);
-    // the batched compiled plan takes dealiased grids (others run their own step)
-    GD_CHECK(ring_short(a.nlon) || !gd_ring_compiled(a.nlon) || (3 * (a.mmax + 1) <= a.nlon && gd_offsets_fit(a)),
-             GD_ERR_ARG, "ring batch: nlon=%d mmax=%d", a.nlon, a.mmax);
     return GD_OK;
+}
+
+int gd_ring_tang_form(const RingArgs &a)
+{
+    if (ring_short(a.nlon) || !gd_ring_compiled(a.nlon) || !gd_offsets_fit(a)) return 0;
+    return gd_ring_deal(a) ? 1 : 2;
 }
 
 // ring pairs per block of the boundary passes of lengths without a compiled
@@ -781,18 +784,20 @@ template <typename T> int gd_launch_ring(hipStream_t st, int mode, const RingArg
 }
 
 // The tangential step's ring pass in one grid over several shells of one
-// ring length
+// ring length and form
 template <typename T, int NC>
 static void ring_batch_launch(hipStream_t st, const BatchRef<RingArgs> &b, int nblocks, size_t lds)
 {
     hipLaunchKernelGGL((ring_batch_kernel<T, RING_STEP_TANG, NC>), dim3(nblocks), dim3(RING_THREADS), lds, st, b);
 }
 
-template <typename T> int gd_launch_ring_tang_batch(hipStream_t st, const BatchRef<RingArgs> &b, int nblocks, int nlon)
+template <typename T> int gd_launch_ring_tang_batch(hipStream_t st, const BatchRef<RingArgs> &b, int nblocks, int nlon, int form)
 {
     if (nblocks <= 0) return GD_OK;
-    if (!ring_short(nlon) && gd_launch_ring_tang_batch_plan<T>(st, b, nblocks, nlon))
+    if (form) {
+        GD_CHECK(gd_launch_ring_tang_batch_plan<T>(st, b, nblocks, nlon, form == 1), GD_ERR_ARG, "ring batch: no plan of nlon=%d", nlon);
         return gd_check_launch("ring_step_batch_kernel");
+    }
     const size_t lds = sizeof(C2<T>) * ((size_t)ring_ld(nlon) * 4 + nlon);
     GD_CHECK(lds <= 160 * 1024, GD_ERR_ARG, "ring batch: LDS %zu too large", lds);
     switch (nlon) {
@@ -806,8 +811,8 @@ template <typename T> int gd_launch_ring_tang_batch(hipStream_t st, const BatchR
     }
     return gd_check_launch("ring_batch_kernel");
 }
-template int gd_launch_ring_tang_batch<float>(hipStream_t, const BatchRef<RingArgs> &, int, int);
-template int gd_launch_ring_tang_batch<double>(hipStream_t, const BatchRef<RingArgs> &, int, int);
+template int gd_launch_ring_tang_batch<float>(hipStream_t, const BatchRef<RingArgs> &, int, int, int);
+template int gd_launch_ring_tang_batch<double>(hipStream_t, const BatchRef<RingArgs> &, int, int, int);
 
 template int gd_launch_ring<float>(hipStream_t, int, const RingArgs &);
 template int gd_launch_ring<double>(hipStream_t, int, const RingArgs &);

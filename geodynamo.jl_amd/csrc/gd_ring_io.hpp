@@ -123,7 +123,7 @@ template <typename T, int MODE, int N, int NF> void ring_plan_launch(hipStream_t
 {
     using SH = RingIoShape<T, N, NF>;
     const dim3 grid((a.nlat2 + SH::RG - 1) / SH::RG, a.nr), block(SH::nthr);
-    if (3 * (a.mmax + 1) <= N) hipLaunchKernelGGL((ring_plan_kernel<T, MODE, N, NF, true>), grid, block, SH::lds, st, a);
+    if (gd_ring_deal(a)) hipLaunchKernelGGL((ring_plan_kernel<T, MODE, N, NF, true>), grid, block, SH::lds, st, a);
     else hipLaunchKernelGGL((ring_plan_kernel<T, MODE, N, NF, false>), grid, block, SH::lds, st, a);
 }
 

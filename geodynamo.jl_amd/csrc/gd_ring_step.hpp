@@ -205,13 +205,14 @@ __global__ void __launch_bounds__((RingStepShape<T, MODE, N>::nthr)) ring_step_p
     ring_step_body<T, MODE, N, DEAL>(a, xcd_logical(blockIdx.x, gridDim.x));
 }
 
-// one grid over the ring passes of several shells (every one dealiased)
-template <typename T, int MODE, int N>
+// one grid over the ring passes of several shells, dealiased ones or any (their
+// own launches' instance, so that each shell gets its own bits)
+template <typename T, int MODE, int N, bool DEAL>
 __global__ void __launch_bounds__((RingStepShape<T, MODE, N>::nthr)) ring_step_batch_kernel(BatchRef<RingArgs> b)
 {
     const int sh = b.shell_of_block[blockIdx.x];
     if (sh == BATCH_PAD) return;
-    ring_step_body<T, MODE, N, true>(batch_args(b, sh), xcd_logical(blockIdx.x - b.block_off[sh], b.block_cnt[sh]));
+    ring_step_body<T, MODE, N, DEAL>(batch_args(b, sh), xcd_logical(blockIdx.x - b.block_off[sh], b.block_cnt[sh]));
 }
 
 template <typename T, int MODE, int N> bool ring_step_launch(hipStream_t st, const RingArgs &a)
@@ -221,7 +222,7 @@ template <typename T, int MODE, int N> bool ring_step_launch(hipStream_t st, con
         return false;
     } else {
         const dim3 grid(a.nlat2 * a.nr), block(SH::nthr);
-        if (3 * (a.mmax + 1) <= N) hipLaunchKernelGGL((ring_step_plan_kernel<T, MODE, N, true>), grid, block, SH::lds, st, a);
+        if (gd_ring_deal(a)) hipLaunchKernelGGL((ring_step_plan_kernel<T, MODE, N, true>), grid, block, SH::lds, st, a);
         else hipLaunchKernelGGL((ring_step_plan_kernel<T, MODE, N, false>), grid, block, SH::lds, st, a);
         return true;
     }
@@ -238,17 +239,19 @@ template <typename T, int MODE> bool ring_step_mode(hipStream_t st, const RingAr
     }
 }
 
-template <typename T, int N> bool ring_step_batch_launch(hipStream_t st, const BatchRef<RingArgs> &b, int nblocks)
+template <typename T, int N> bool ring_step_batch_launch(hipStream_t st, const BatchRef<RingArgs> &b, int nblocks, bool deal)
 {
     using SH = RingStepShape<T, RING_STEP_TANG, N>;
-    hipLaunchKernelGGL((ring_step_batch_kernel<T, RING_STEP_TANG, N>), dim3(nblocks), dim3(SH::nthr), SH::lds, st, b);
+    const dim3 grid(nblocks), block(SH::nthr);
+    if (deal) hipLaunchKernelGGL((ring_step_batch_kernel<T, RING_STEP_TANG, N, true>), grid, block, SH::lds, st, b);
+    else hipLaunchKernelGGL((ring_step_batch_kernel<T, RING_STEP_TANG, N, false>), grid, block, SH::lds, st, b);
     return true;
 }
 
-template <typename T> bool ring_step_batch(hipStream_t st, const BatchRef<RingArgs> &b, int nblocks, int nlon)
+template <typename T> bool ring_step_batch(hipStream_t st, const BatchRef<RingArgs> &b, int nblocks, int nlon, bool deal)
 {
     switch (nlon) {
-#define GD_RING_LEN(N) case N: return ring_step_batch_launch<T, N>(st, b, nblocks);
+#define GD_RING_LEN(N) case N: return ring_step_batch_launch<T, N>(st, b, nblocks, deal);
         GD_RING_LENGTHS
 #undef GD_RING_LEN
     default: return false;

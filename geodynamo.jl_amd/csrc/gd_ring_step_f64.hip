@@ -12,7 +12,7 @@ template <> bool gd_launch_ring_step_plan<double>(hipStream_t st, int mode, cons
     }
 }
 
-template <> bool gd_launch_ring_tang_batch_plan<double>(hipStream_t st, const BatchRef<RingArgs> &b, int nblocks, int nlon)
+template <> bool gd_launch_ring_tang_batch_plan<double>(hipStream_t st, const BatchRef<RingArgs> &b, int nblocks, int nlon, bool deal)
 {
-    return ring_step_batch<double>(st, b, nblocks, nlon);
+    return ring_step_batch<double>(st, b, nblocks, nlon, deal);
 }

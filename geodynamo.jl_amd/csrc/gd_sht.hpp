@@ -152,6 +152,9 @@ inline bool gd_offsets_fit(const RingArgs &a)
     const size_t lim = (size_t)1 << 31, nm = a.mmax + 1;
     return nm * a.fdim.m * a.fstr < lim && nm * a.gdim.m * 8 < lim;
 }
+// a dealiased grid (the middle third of the orders is unused): instances of
+// the compiled plans of their own
+inline bool gd_ring_deal(const RingArgs &a) { return 3 * (a.mmax + 1) <= a.nlon; }
 // stage twiddles of the compiled plan of nlon, e^{-i angle} as (re, im) pairs
 void gd_ring_stage_twiddles(int nlon, std::vector<double> &tw);
 // a boundary pass (RING_SYNTH, RING_ANALYSIS; 1 or 2 fields) by the compiled
@@ -164,9 +167,9 @@ template <> bool gd_launch_ring_plan<double>(hipStream_t st, int mode, const Rin
 template <typename T> bool gd_launch_ring_step_plan(hipStream_t st, int mode, const RingArgs &a);
 template <> bool gd_launch_ring_step_plan<float>(hipStream_t st, int mode, const RingArgs &a);
 template <> bool gd_launch_ring_step_plan<double>(hipStream_t st, int mode, const RingArgs &a);
-template <typename T> bool gd_launch_ring_tang_batch_plan(hipStream_t st, const BatchRef<RingArgs> &b, int nblocks, int nlon);
-template <> bool gd_launch_ring_tang_batch_plan<float>(hipStream_t st, const BatchRef<RingArgs> &b, int nblocks, int nlon);
-template <> bool gd_launch_ring_tang_batch_plan<double>(hipStream_t st, const BatchRef<RingArgs> &b, int nblocks, int nlon);
+template <typename T> bool gd_launch_ring_tang_batch_plan(hipStream_t st, const BatchRef<RingArgs> &b, int nblocks, int nlon, bool deal);
+template <> bool gd_launch_ring_tang_batch_plan<float>(hipStream_t st, const BatchRef<RingArgs> &b, int nblocks, int nlon, bool deal);
+template <> bool gd_launch_ring_tang_batch_plan<double>(hipStream_t st, const BatchRef<RingArgs> &b, int nblocks, int nlon, bool deal);
 // up to LM_MAXPLANES planes between the l-major layout of the interface
 // (level stride nlm) and the m-major device layout, one launch for all:
 // to_m writes element type T with dst_ls elements from level to level (nlm for
@@ -197,9 +200,12 @@ bool gd_synth_tile_ok(int tile, bool fp64);
 template <typename T>
 int gd_launch_synth_tang_batch(hipStream_t st, const BatchRef<SynthArgs> &b, int nblocks, int tile, int mm);
 template <typename T> int gd_launch_synth_tang_tile(hipStream_t st, const SynthArgs &a, int tile);
-template <typename T> int gd_launch_ring_tang_batch(hipStream_t st, const BatchRef<RingArgs> &b, int nblocks, int nlon);
+template <typename T> int gd_launch_ring_tang_batch(hipStream_t st, const BatchRef<RingArgs> &b, int nblocks, int nlon, int form);
 int gd_synth_tang_batchable(const SynthArgs &a);
 int gd_ring_tang_batchable(const RingArgs &a, bool fp64);
+// the instance of a shell's tangential ring pass, which a batched launch shares:
+// 0 ring_kernel's plans, 1 a compiled register plan on a dealiased grid, 2 on any
+int gd_ring_tang_form(const RingArgs &a);
 int gd_ana_kn(int nlat2, bool fp64);
 void gd_ana_plan(AnaArgs &a, bool vec, int maxgroup);
 int gd_ana_blocks(const AnaArgs &a, bool vec);

@@ -1281,7 +1281,7 @@ enum { BK_SYNTH = 0, BK_RING, BK_ANAV, BK_ANAS, BK_CHAIN, BK_NKIND };
 
 struct BatchGroup {
     int lane = 0;
-    int kind = 0, fp64 = 0, mm = 0, key = 0; // key: synthesis tile, ring length, node tile or band width
+    int kind = 0, fp64 = 0, mm = 0, key = 0; // key: synthesis tile, 4 ring length + form, node tile or band width
     ChainForm fm{};
     size_t lds = 0;
     int nblocks = 0;
@@ -1485,7 +1485,7 @@ static int fused_build(gd_batch *b, int parity)
         cur_lane = lane_of[i];
         GD_CHECK(gd_synth_tile_ok(t, x.fp64), GD_ERR_ARG, "gd_batch: shell %d: synthesis tile %d not available", i, t);
         find(BK_SYNTH, x.fp64, x.a.mm, t, nullptr).shells.push_back(i);
-        find(BK_RING, x.fp64, 0, x.r.nlon, nullptr).shells.push_back(i);
+        find(BK_RING, x.fp64, 0, 4 * x.r.nlon + gd_ring_tang_form(x.r), nullptr).shells.push_back(i);
         find(BK_ANAV, x.fp64, x.gv.mm, x.kn, nullptr).shells.push_back(i);
         find(BK_ANAS, x.fp64, x.gs.mm, x.kn, nullptr).shells.push_back(i);
         BatchGroup &gc = find(BK_CHAIN, x.fp64, 0, x.c.bw, &x.fm);
@@ -1584,7 +1584,7 @@ template <typename T> static int launch_group(gd_batch *b, int parity, const Bat
 {
     switch (g.kind) {
     case BK_SYNTH: return gd_launch_synth_tang_batch<T>(st, group_ref<SynthArgs>(b, parity, g), g.nblocks, g.key, g.mm);
-    case BK_RING: return gd_launch_ring_tang_batch<T>(st, group_ref<RingArgs>(b, parity, g), g.nblocks, g.key);
+    case BK_RING: return gd_launch_ring_tang_batch<T>(st, group_ref<RingArgs>(b, parity, g), g.nblocks, g.key / 4, g.key % 4);
     case BK_ANAV:
     case BK_ANAS:
         return gd_launch_ana_batch<T>(st, group_ref<AnaArgs>(b, parity, g), g.nblocks, g.kind == BK_ANAV, g.key, g.mm);

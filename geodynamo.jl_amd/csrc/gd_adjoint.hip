@@ -337,7 +337,7 @@ static int nonlinear_adjoint_T(gd_step *s, const double *xs, const double *mu, d
     a.in = w->syn.p;
     a.cin = ADJ_COLS;
     const size_t nm = p->mmax + 1, recs = nm * nr * p->nlat2;
-    a.dim = RecDim{1, nm, nm * nr}; // as the step: FB[i][level][m], GB[m][i][level]
+    a.dim = gd_step_fb_dim((int)nm, nr);
     a.plane = 8;
     a.rstr = ADJ_NSLOT;
     // u and the force cotangent as full fields, grad T as a gradient field
@@ -359,14 +359,6 @@ static int nonlinear_adjoint_T(gd_step *s, const double *xs, const double *mu, d
     r.fb = w->fb.p;
     r.gb = w->gb.p;
     r.nfield = 7;
-    r.fdim = a.dim;
-    r.gdim = RecDim{(size_t)p->nlat2 * nr, 1, (size_t)nr};
-    r.fstr = ADJ_NSLOT;
-    for (int F = 0; F < 7; ++F) r.foff[F] = 4 * F;
-    for (int P = 0; P < 4; ++P) {
-        r.goff[P] = gd_comp_off(P, 4, recs);
-        r.gstr[P] = gd_comp_str(P, 4);
-    }
     r.ro = s->d.Pm / s->d.E;
     r.coriolis_index = s->d.coriolis_index;
     GD_TRY(gd_launch_ring<T>(st, RING_ADJ_TANG, r));
@@ -374,7 +366,7 @@ static int nonlinear_adjoint_T(gd_step *s, const double *xs, const double *mu, d
     g.mm = p->prec == GD_PREC_BF16X3;
     g.gb = w->gb.p;
     g.plane = 8 * recs;
-    g.dim = r.gdim;
+    g.dim = gd_step_gb_dim(p->nlat2, nr);
     g.nf = 2;
     g.moff = p->d_moff.as<int>();
     g.ne = p->d_ne.as<int>();
@@ -781,8 +773,7 @@ extern "C" int gd_adjoint_misfit(gd_adjoint *a, int kind, int level, const doubl
     gd_sht_fill_ring(p, rg, 1);
     rg.fb = p->fb.p;
     rg.nfield = 1;
-    rg.fstr = 4;
-    rg.fdim = dim;
+    rg.dim = dim;
     rg.phys_out[0] = a->mgrid.as<double>();
     GD_TRY(gd_launch_ring<double>(st, RING_SYNTH, rg));
     GD_TRY(gd_from_device(s->ctx, a->hgrid.data(), a->mgrid.p, sizeof(double) * nlat * nlon));
@@ -807,8 +798,7 @@ extern "C" int gd_adjoint_misfit(gd_adjoint *a, int kind, int level, const doubl
     gd_sht_fill_ring(p, ra, 1);
     ra.wq = a->ones.p;
     ra.gb = p->gb.p;
-    ra.gstr[0] = 4;
-    ra.gdim = dim;
+    ra.dim = dim;
     ra.nfield = 1;
     ra.phys_in[0] = a->mgrid.as<double>();
     GD_TRY(gd_launch_ring<double>(st, RING_ANALYSIS, ra));

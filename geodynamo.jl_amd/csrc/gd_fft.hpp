@@ -105,6 +105,25 @@ template <int R, int DIR, typename T> __device__ __forceinline__ void dft(C2<T> 
     }
 }
 
+// the step modes' fields, tangential components among them, products,
+// tangential among them
+template <int MODE> struct StepMode { static constexpr int NF = 0, NFV = 0, NP = 0, NPV = 0; };
+template <> struct StepMode<RING_STEP_TANG> { static constexpr int NF = 4, NFV = 4, NP = 3, NPV = 2; };
+template <> struct StepMode<RING_STEP_TANG_C> { static constexpr int NF = 6, NFV = 6, NP = 4, NPV = 2; };
+template <> struct StepMode<RING_ADJ_TANG> { static constexpr int NF = 7, NFV = 6, NP = 4, NPV = 4; };
+template <> struct StepMode<RING_STEP> { static constexpr int NF = 15, NFV = 10, NP = 5, NPV = 4; };
+
+// Block order of a step mode's pass over nodes (fastest) and levels: block b of
+// the launch goes to XCD b % 8, and a node's consecutive levels write pieces of
+// the same lines of GB.  Where the nodes are a multiple of 8 they meet on one XCD
+// in the launch order; else the blocks are renumbered so that each XCD takes a
+// contiguous range.  Measured, launch order against renumbered (us): 192 nodes,
+// 33 levels, rings of 768, FP32 tangential 87 / 106, with composition 137 / 162;
+// 96 nodes, 65 levels, rings of 384 FP32 36.8 / 38.6, 15 fields 119 / 125, FP64
+// 70.7 / 71.7; 54 nodes, rings of 216 FP32 20.0 / 19.1; 81 nodes, rings of 324,
+// with composition 56.8 / 55.1.
+__device__ __forceinline__ int ring_step_block(int b, int nblk, int nlat2) { return nlat2 % 8 ? xcd_logical(b, nblk) : b; }
+
 // ---- compiled plans: two stages where both radices are at most 18 (the least
 // largest radix), else three of at most 12
 struct FftStages {

@@ -140,6 +140,8 @@ void gd_sht_fill_ring(const gd_sht_plan *p, RingArgs &a, int nr)
 {
     a.tw = p->tw.p;
     a.tws = p->tws.p;
+    a.foff[0] = 0;
+    a.foff[1] = 4;
     a.sinth = p->sinth.p;
     a.costh = p->costh.p;
     a.wq = p->wq.p;
@@ -308,9 +310,7 @@ static int run_synth(gd_sht_plan *p, bool vec, const double *a_re, const double 
     gd_sht_fill_ring(p, r, nr);
     r.fb = p->fb.p;
     r.nfield = vec ? 2 : 1;
-    for (int F = 0; F < r.nfield; ++F) r.foff[F] = 4 * F;
-    r.fstr = nslot;
-    r.fdim = dim;
+    r.dim = dim;
     r.phys_out[0] = o0;
     r.phys_out[1] = o1;
     GD_TRY(gd_launch_ring<T>(st, RING_SYNTH, r));
@@ -341,11 +341,7 @@ static int run_analysis(gd_sht_plan *p, bool vec, const double *f0, const double
     gd_sht_fill_ring(p, r, nr);
     r.gb = p->gb.p;
     r.nfield = vec ? 2 : 1;
-    for (int F = 0; F < r.nfield; ++F) {
-        r.goff[F] = 4 * F;
-        r.gstr[F] = nslot;
-    }
-    r.gdim = dim;
+    r.dim = dim;
     r.phys_in[0] = f0;
     r.phys_in[1] = f1;
     if (adj) r.wq = p->wone.p;

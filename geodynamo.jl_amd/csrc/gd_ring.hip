@@ -252,6 +252,20 @@ __device__ __forceinline__ void fft_ct(C2<T> *buf, const C2<T> *tw, int nfft)
     }
 }
 
+// A record of the step's FB, which this pass reads once and nothing reads again:
+// a non-temporal load, so that FB does not push the products out of the
+// last-level cache before the analyses read them.  96 nodes, 65 levels, rings of
+// 384, whole step (us): FP64 tangential 259 -> 245, with composition 390 -> 350;
+// FP32 with composition 235 -> 226, 15 fields 456 -> 434 (its vector analysis 62
+// -> 44).  The register plans, whose lanes read pieces of several
+// orders, lose 5 % of a step that way and keep the ordinary load.
+template <typename T> __device__ __forceinline__ RingRec<T> fb_load(const T *p)
+{
+    typedef T V4 __attribute__((ext_vector_type(4)));
+    const V4 q = __builtin_nontemporal_load(reinterpret_cast<const V4 *>(p));
+    return RingRec<T>{{q[0], q[1], q[2], q[3]}};
+}
+
 // One block per (northern node i, level r) (the launch's own grid, or its share
 // of a batched launch).  NC > 0: the ring length is the compile-time constant
 // NC (nlon); NC = 0 uses the runtime plan.
@@ -263,20 +277,15 @@ template <typename T, int MODE, int NC, class AT> __device__ __forceinline__ voi
     C2<T> *tw = reinterpret_cast<C2<T> *>(smem_raw);
     C2<T> *buf = tw + n;
     __shared__ int srad[12];
-    __shared__ size_t sfo[16];
     const int tid = threadIdx.x;
     constexpr int nthr = RING_THREADS;
     const int is = a.nlat - 1 - i; // southern mirror
     const C2<T> *twg = static_cast<const C2<T> *>(a.tw);
     for (int k = tid; k < n; k += nthr) tw[k] = twg[k];
     if (tid < 12) srad[tid] = a.radix[tid];
-    if (tid < 16) sfo[tid] = a.foff[tid];
     __syncthreads();
-    // fields in / products out: compile-time for the step modes
-    constexpr int NFC = MODE == RING_STEP ? 15 : MODE == RING_STEP_TANG ? 4 : MODE == RING_STEP_TANG_C ? 6
-                      : MODE == RING_ADJ_TANG ? 7 : 0;
-    constexpr int NPC = MODE == RING_STEP ? 5 : MODE == RING_STEP_TANG ? 3 : MODE == RING_STEP_TANG_C ? 4
-                      : MODE == RING_ADJ_TANG ? 4 : 0;
+    // fields in / products out: compile-time for the step modes (0: a boundary pass)
+    constexpr int NFC = StepMode<MODE>::NF, NPC = StepMode<MODE>::NP, NPV = StepMode<MODE>::NPV;
     const int NF = NFC ? NFC : a.nfield;
 
     if (MODE != RING_ANALYSIS) {
@@ -291,7 +300,9 @@ template <typename T, int MODE, int NC, class AT> __device__ __forceinline__ voi
         constexpr int MAXU0 = (NC > 0 && NFC > 0) ? (NFC * (NC / 3) + nthr - 1) / nthr : 0;
         constexpr int MAXU = MAXU0 < MAXI ? MAXU0 : MAXI;
         const int ne = NF * nm;
-        const size_t rec0 = r * a.fdim.l + i * a.fdim.i;
+        // a step mode's slots of one ring are contiguous, orders outermost
+        const size_t rec0 = NFC ? ((size_t)i * a.nr + r) * nm : r * a.dim.l + i * a.dim.i;
+        const T *src = static_cast<const T *>(a.fb) + rec0 * (4 * NF);
         RingRec<T> z[MAXI];
 #pragma unroll
         for (int it = 0; it < MAXI; ++it) {
@@ -299,8 +310,8 @@ template <typename T, int MODE, int NC, class AT> __device__ __forceinline__ voi
             if (it < MAXU || e0 < ne) {
                 const int e = e0 < ne ? e0 : ne - 1;
                 const int F = e % NF, m = e / NF;
-                z[it] = *reinterpret_cast<const RingRec<T> *>(static_cast<const T *>(a.fb) + sfo[F] +
-                                                              (m * a.fdim.m + rec0) * a.fstr);
+                if constexpr (NFC > 0) z[it] = fb_load(src + 4 * e);
+                else z[it] = *reinterpret_cast<const RingRec<T> *>(src + m * a.dim.m * (4 * NF) + 4 * F);
             }
         }
 #pragma unroll
@@ -477,20 +488,27 @@ template <typename T, int MODE, int NC, class AT> __device__ __forceinline__ voi
     const T c = static_cast<const T *>(a.wq)[i];
     T *gb = static_cast<T *>(a.gb);
     const int NPn = NPC ? NPC : NP;
+    const unsigned ms = (unsigned)(a.nlat2 * a.nr); // a step mode's records of one order
+    const size_t rec0 = (size_t)i * a.nr + r;
     for (int e = tid; e < NPn * nm; e += nthr) {
         const int P = e % NPn, m = e / NPn;
-        const size_t rec = m * a.gdim.m + r * a.gdim.l + i * a.gdim.i;
-        *reinterpret_cast<RingRec<T> *>(gb + a.goff[P] + rec * a.gstr[P]) =
+        T *d;
+        if constexpr (NFC > 0)
+            d = gb + gd_comp_off(P, NPV, (size_t)nm * ms) + ((size_t)m * ms + rec0) * gd_comp_str(P, NPV);
+        else
+            d = gb + (m * a.dim.m + r * a.dim.l + i * a.dim.i) * (4 * NF) + 4 * P;
+        *reinterpret_cast<RingRec<T> *>(d) =
             fft_split<T>(buf[P * ld + sk(m)], buf[P * ld + sk(m ? n - m : 0)], m, c);
     }
 }
 
-// consecutive nodes of one level on one XCD: their slots, and in the boundary
-// layouts their grid values, share cache lines
+// a boundary pass takes consecutive nodes of one level on one XCD (their grid
+// values share cache lines)
 template <typename T, int MODE, int NC> __global__ void __launch_bounds__(256) ring_kernel(RingArgs a)
 {
-    const int L = xcd_logical(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
-    ring_body<T, MODE, NC>(a, L % gridDim.x, L / gridDim.x);
+    const int b = blockIdx.x + gridDim.x * blockIdx.y, nblk = gridDim.x * gridDim.y;
+    const int L = StepMode<MODE>::NF > 0 ? ring_step_block(b, nblk, a.nlat2) : xcd_logical(b, nblk);
+    ring_body<T, MODE, NC>(a, L % a.nlat2, L / a.nlat2);
 }
 
 // The boundary passes (RING_SYNTH: Fourier -> physical rings, RING_ANALYSIS:
@@ -512,7 +530,6 @@ __device__ __forceinline__ void ring_io_body(const RingArgs &a, int g, int r)
     C2<T> *tw = reinterpret_cast<C2<T> *>(smem_raw);
     C2<T> *buf = tw + n;
     __shared__ int srad[12];
-    __shared__ size_t sfo[16];
     const int tid = threadIdx.x;
     constexpr int nthr = RING_THREADS;
     const int NF = a.nfield;
@@ -521,7 +538,6 @@ __device__ __forceinline__ void ring_io_body(const RingArgs &a, int g, int r)
     const C2<T> *twg = static_cast<const C2<T> *>(a.tw);
     for (int k = tid; k < n; k += nthr) tw[k] = twg[k];
     if (tid < 12) srad[tid] = a.radix[tid];
-    if (tid < 16) sfo[tid] = a.foff[tid];
     __syncthreads();
     if (MODE == RING_SYNTH) {
         // Hermitian spectra of the north (X) and south (Y) rings packed as Z = X + iY
@@ -535,7 +551,7 @@ __device__ __forceinline__ void ring_io_body(const RingArgs &a, int g, int r)
                 const int e = min(e0 + tid + it * nthr, NT * nm - 1);
                 const int F = e % NF, q = (e / NF) % nq, m = e / NT;
                 const C2<T> *p = reinterpret_cast<const C2<T> *>(
-                    static_cast<const T *>(a.fb) + sfo[F] + (m * a.fdim.m + r * a.fdim.l + (i0 + q) * a.fdim.i) * a.fstr);
+                    static_cast<const T *>(a.fb) + 4 * F + (m * a.dim.m + r * a.dim.l + (i0 + q) * a.dim.i) * (4 * NF));
                 xn[it] = p[0];
                 xs[it] = p[1];
             }
@@ -615,8 +631,7 @@ __device__ __forceinline__ void ring_io_body(const RingArgs &a, int g, int r)
             X = C2<T>{T(0.5) * (Z.x + Zc.x), T(0.5) * (Z.y - Zc.y)};
             Y = C2<T>{T(0.5) * (Z.y + Zc.y), T(0.5) * (Zc.x - Z.x)};
         }
-        const size_t rec = m * a.gdim.m + r * a.gdim.l + i * a.gdim.i;
-        T *d = gb + a.goff[F] + rec * a.gstr[F];
+        T *d = gb + (m * a.dim.m + r * a.dim.l + i * a.dim.i) * (4 * NF) + 4 * F;
         d[0] = (X.x + Y.x) * c;
         d[1] = (X.y + Y.y) * c;
         d[2] = (X.x - Y.x) * c;
@@ -638,7 +653,7 @@ template <typename T, int MODE, int NC> __global__ void __launch_bounds__(256) r
     const int sh = b.shell_of_block[blockIdx.x];
     if (sh == BATCH_PAD) return;
     const auto &a = batch_args(b, sh);
-    const int L = xcd_logical(blockIdx.x - b.block_off[sh], b.block_cnt[sh]);
+    const int L = ring_step_block(blockIdx.x - b.block_off[sh], b.block_cnt[sh], a.nlat2);
     ring_body<T, MODE, NC>(a, L % a.nlat2, L / a.nlat2);
 }
 } // namespace
@@ -648,11 +663,38 @@ template <typename T, int MODE, int NC> static void ring_launch(hipStream_t st, 
     hipLaunchKernelGGL((ring_kernel<T, MODE, NC>), grid, dim3(RING_THREADS), lds, st, a);
 }
 
-// lengths whose tangential modes run ring_kernel's own compiled plan (the
-// measured choice: gd_ring_step.hpp)
-static bool ring_short(int nlon)
+// Lengths whose tangential modes run ring_kernel's own compiled plan, not the
+// register plans: its blocks of 256 threads hold more waves.  us at 65 levels,
+// against the register plan: FP32 rings of 48 / 96 / 144 / 192 / 288 / 384 4.6
+// against 6.9, 6.7 - 8.6, 11.3 - 12.9, 14.4 - 17.2, 29.8 - 32.7, 36.8 - 39.0; FP64
+// 5.2 against 7.7, 11.0 - 11.6, 16.7 - 17.6, 24.0 - 30.4, 48.6 - 53.8, 70.7 - 69.4.
+// Beyond, at 33 levels (renumbered blocks): 432 FP32 33.2 against 31.4, FP64 56 -
+// 54, 576 FP32 55.7 - 51.6, FP64 103 - 99.5, 768 FP32 109 - 106, FP64 199 - 195.
+static bool ring_short(int nlon) { return nlon % 48 == 0 && nlon <= 384; }
+
+// The 15-field step keeps ring_kernel's plan where the register plan takes three
+// stages, ring_kernel no more, and three of its blocks fit a CU's LDS.  us at 65
+// levels, against the register plan: FP32 384 119 - 127 (fits); FP64 384 342 - 260
+// and, at 33 levels, FP32 512 89 - 72 (do not fit); FP32 243, five stages, 74 - 47
+template <typename T> constexpr bool ring_step_own(int n)
 {
-    return nlon == 48 || nlon == 96 || nlon == 144 || nlon == 192 || nlon == 288 || nlon == 384;
+    const size_t lds = sizeof(C2<T>) * ((size_t)ring_ld(n) * StepMode<RING_STEP>::NF + n);
+    return fft_stages(n).n == 3 && ct_nstages(n) <= 3 && 3 * lds <= 160 * 1024;
+}
+template <typename T> static bool ring_step_own_launch(hipStream_t st, dim3 grid, size_t lds, const RingArgs &a)
+{
+    switch (a.nlon) {
+#define GD_RING_LEN(N)                                          \
+    case N:                                                     \
+        if constexpr (ring_step_own<T>(N)) {                    \
+            ring_launch<T, RING_STEP, N>(st, grid, lds, a);     \
+            return true;                                        \
+        }                                                       \
+        return false;
+        GD_RING_LENGTHS
+#undef GD_RING_LEN
+    default: return false;
+    }
 }
 
 template <typename T, int MODE> static void ring_dispatch(hipStream_t st, dim3 grid, size_t lds, const RingArgs &a)
@@ -697,7 +739,7 @@ int gd_ring_tang_batchable(const RingArgs &a, bool fp64)
 
 int gd_ring_tang_form(const RingArgs &a)
 {
-    if (ring_short(a.nlon) || !gd_ring_compiled(a.nlon) || !gd_offsets_fit(a)) return 0;
+    if (ring_short(a.nlon) || !gd_ring_compiled(a.nlon) || !gd_step_offsets_fit(a)) return 0;
     return gd_ring_deal(a) ? 1 : 2;
 }
 
@@ -767,7 +809,8 @@ template <typename T> int gd_launch_ring(hipStream_t st, int mode, const RingArg
     size_t lds = sizeof(C2<T>) * ((size_t)ring_ld(a.nlon) * nf + a.nlon);
     GD_CHECK(lds <= 160 * 1024, GD_ERR_ARG, "ring: LDS %zu too large", lds);
     dim3 grid(a.nlat2, a.nr);
-    if ((!ring_short(a.nlon) || (mode == RING_STEP && !(sizeof(T) == 4 && a.nlon == 384))) && gd_launch_ring_step_plan<T>(st, mode, a))
+    if (mode == RING_STEP && ring_step_own_launch<T>(st, grid, lds, a)) return gd_check_launch("ring_kernel");
+    if ((mode == RING_STEP || !ring_short(a.nlon)) && gd_launch_ring_step_plan<T>(st, mode, a))
         return gd_check_launch("ring_step_plan_kernel");
     switch (mode) {
     case RING_SYNTH: ring_launch<T, RING_SYNTH, 0>(st, grid, lds, a); break;
@@ -775,10 +818,7 @@ template <typename T> int gd_launch_ring(hipStream_t st, int mode, const RingArg
     case RING_STEP_TANG: ring_dispatch<T, RING_STEP_TANG>(st, grid, lds, a); break;
     case RING_STEP_TANG_C: ring_dispatch<T, RING_STEP_TANG_C>(st, grid, lds, a); break;
     case RING_ADJ_TANG: ring_dispatch<T, RING_ADJ_TANG>(st, grid, lds, a); break;
-    default:
-        if (sizeof(T) == 4 && a.nlon == 384) ring_launch<float, RING_STEP, 384>(st, grid, lds, a);
-        else ring_launch<T, RING_STEP, 0>(st, grid, lds, a);
-        break;
+    default: ring_launch<T, RING_STEP, 0>(st, grid, lds, a); break;
     }
     return gd_check_launch("ring_kernel");
 }

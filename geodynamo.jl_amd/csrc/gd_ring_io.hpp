@@ -58,9 +58,9 @@ __global__ void __launch_bounds__((RingIoShape<T, N, NF>::nthr)) ring_plan_kerne
             const int g = tid + it * nthr, F = g % NF, q = g / NF % RG, j = g / SH::NT;
             if (total0 % nthr != 0 && g >= total0) continue;
             const T *rec = static_cast<const T *>(a.fb) + (F ? a.foff[1] : a.foff[0]) +
-                           (lev * a.fdim.l + (i0 + min(q, nq - 1)) * a.fdim.i) * a.fstr;
+                           (lev * a.dim.l + (i0 + min(q, nq - 1)) * a.dim.i) * (4 * NF);
             C2<T> v[R0];
-            fft_pack_stage<T, N, DEAL>(rec, (unsigned)(a.fdim.m * a.fstr), nm, j, v);
+            fft_pack_stage<T, N, DEAL>(rec, (unsigned)(a.dim.m * (4 * NF)), nm, j, v);
             fft_lds_put<T, N, 0, 1>(buf + (q * NF + F) * LD, j, v);
         }
         if constexpr (S == 2) fft_rows_stage<T, N, 1, 1, SH::NT, nthr, LD, false>(buf, tws);
@@ -110,10 +110,9 @@ __global__ void __launch_bounds__((RingIoShape<T, N, NF>::nthr)) ring_plan_kerne
         for (int e = tid; e < SH::NT * nm; e += nthr) {
             const int F = e % NF, q = e / NF % RG, m = e / SH::NT;
             if (q >= nq) continue;
-            T *rec = static_cast<T *>(a.gb) + (F ? a.goff[1] : a.goff[0]) +
-                     (lev * a.gdim.l + (i0 + q) * a.gdim.i) * a.gstr[0];
+            T *rec = static_cast<T *>(a.gb) + 4 * F + (lev * a.dim.l + (i0 + q) * a.dim.i) * (4 * NF);
             const C2<T> *x = buf + (q * NF + F) * LD;
-            *reinterpret_cast<RingRec<T> *>(rec + (unsigned)m * (unsigned)(a.gdim.m * a.gstr[0])) =
+            *reinterpret_cast<RingRec<T> *>(rec + (unsigned)m * (unsigned)(a.dim.m * (4 * NF))) =
                 fft_split<T>(x[m], x[m ? N - m : 0], m, static_cast<const T *>(a.wq)[i0 + q]);
         }
     }

@@ -14,23 +14,15 @@
 // slower (fewer resident waves).
 //
 // Measured at nr = 65 against ring_kernel's plan (us): 15 fields FP32 nlon 96 /
-// 192 / 288: 12.3 / 31.7 / 80.7 -> 9.6 / 26.4 / 61.8; FP64 192 / 384: 56 / 352 ->
-// 45 / 274.  The tangential modes at 48 .. 384 (multiples of 48) are as fast or
-// faster with ring_kernel's compiled plans (FP32 192: 15.8 against 17.8, FP64
-// 25.0 against 30.4) and keep them; so does the 15-field step in FP32 at 384,
-// whose plan has three stages (128 against 140).
+// 192 / 288: 12.2 / 31.9 / 79.5 -> 9.4 / 25.4 / 57.4; FP64 192 / 384: 55 / 336 ->
+// 44 / 260; against the runtime plan, tangential FP32 216 / 324: 79 / 165 -> 19 /
+// 42.  Some lengths keep ring_kernel's plan (gd_ring.hip: ring_short,
+// ring_step_own).
 #pragma once
 #include "gd_fft.hpp"
 #include "gd_sht.hpp"
 
 namespace {
-// fields, tangential components among them, products, tangential among them
-template <int MODE> struct StepMode;
-template <> struct StepMode<RING_STEP_TANG> { static constexpr int NF = 4, NFV = 4, NP = 3, NPV = 2; };
-template <> struct StepMode<RING_STEP_TANG_C> { static constexpr int NF = 6, NFV = 6, NP = 4, NPV = 2; };
-template <> struct StepMode<RING_ADJ_TANG> { static constexpr int NF = 7, NFV = 6, NP = 4, NPV = 4; };
-template <> struct StepMode<RING_STEP> { static constexpr int NF = 15, NFV = 10, NP = 5, NPV = 4; };
-
 // threads for `total` butterflies: as few rounds as `most` threads allow, evenly
 constexpr int ring_step_threads(int total, int most)
 {
@@ -140,13 +132,13 @@ __device__ __forceinline__ void ring_step_body(const AT &a, int L)
     {
         // lanes take the fields of one order first (contiguous slots)
         constexpr int R0 = fi.r[0], nb0 = N / R0, total = M::NF * nb0, IT = (total + nthr - 1) / nthr;
-        const T *rec = static_cast<const T *>(a.fb) + (lev * a.fdim.l + i * a.fdim.i) * a.fstr;
+        const T *rec = static_cast<const T *>(a.fb) + ((size_t)i * a.nr + lev) * nm * (4 * M::NF);
 #pragma unroll
         for (int it = 0; it < IT; ++it) {
             const int g = tid + it * nthr, F = g % M::NF, j = g / M::NF;
             if (total % nthr != 0 && g >= total) continue;
             C2<T> v[R0];
-            fft_pack_stage<T, N, DEAL>(rec + 4 * F, (unsigned)(a.fdim.m * a.fstr), nm, j, v);
+            fft_pack_stage<T, N, DEAL>(rec + 4 * F, 4u * M::NF, nm, j, v);
             fft_lds_put<T, N, 0, 1>(buf + F * LD, j, v);
         }
     }
@@ -189,11 +181,12 @@ __device__ __forceinline__ void ring_step_body(const AT &a, int L)
     __syncthreads();
     const T c = static_cast<const T *>(a.wq)[i];
     T *gb = static_cast<T *>(a.gb);
-    const size_t recs = nm * a.gdim.m, rec0 = lev * a.gdim.l + i * a.gdim.i;
+    const unsigned ms = (unsigned)(a.nlat2 * a.nr);
+    const size_t recs = (size_t)nm * ms, rec0 = (size_t)i * a.nr + lev;
     for (int e = tid; e < M::NP * nm; e += nthr) {
         const int P = e % M::NP, m = e / M::NP, str = gd_comp_str(P, M::NPV);
         T *rec = gb + gd_comp_off(P, M::NPV, recs) + rec0 * str;
-        *reinterpret_cast<RingRec<T> *>(rec + (unsigned)m * ((unsigned)a.gdim.m * str)) =
+        *reinterpret_cast<RingRec<T> *>(rec + (unsigned)m * (ms * str)) =
             fft_split<T>(buf[P * LD + m], buf[P * LD + (m ? N - m : 0)], m, c);
     }
 }
@@ -201,8 +194,7 @@ __device__ __forceinline__ void ring_step_body(const AT &a, int L)
 template <typename T, int MODE, int N, bool DEAL>
 __global__ void __launch_bounds__((RingStepShape<T, MODE, N>::nthr)) ring_step_plan_kernel(RingArgs a)
 {
-    // one level's nodes on one XCD: the pieces of GB's lines (consecutive levels) meet in one L2
-    ring_step_body<T, MODE, N, DEAL>(a, xcd_logical(blockIdx.x, gridDim.x));
+    ring_step_body<T, MODE, N, DEAL>(a, ring_step_block(blockIdx.x, gridDim.x, a.nlat2));
 }
 
 // one grid over the ring passes of several shells, dealiased ones or any (their
@@ -212,7 +204,8 @@ __global__ void __launch_bounds__((RingStepShape<T, MODE, N>::nthr)) ring_step_b
 {
     const int sh = b.shell_of_block[blockIdx.x];
     if (sh == BATCH_PAD) return;
-    ring_step_body<T, MODE, N, DEAL>(batch_args(b, sh), xcd_logical(blockIdx.x - b.block_off[sh], b.block_cnt[sh]));
+    const auto &a = batch_args(b, sh);
+    ring_step_body<T, MODE, N, DEAL>(a, ring_step_block(blockIdx.x - b.block_off[sh], b.block_cnt[sh], a.nlat2));
 }
 
 template <typename T, int MODE, int N> bool ring_step_launch(hipStream_t st, const RingArgs &a)
@@ -230,7 +223,7 @@ template <typename T, int MODE, int N> bool ring_step_launch(hipStream_t st, con
 
 template <typename T, int MODE> bool ring_step_mode(hipStream_t st, const RingArgs &a)
 {
-    if (!gd_offsets_fit(a)) return false;
+    if (!gd_step_offsets_fit(a)) return false;
     switch (a.nlon) {
 #define GD_RING_LEN(N) case N: return ring_step_launch<T, MODE, N>(st, a);
         GD_RING_LENGTHS

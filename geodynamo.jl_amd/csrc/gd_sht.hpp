@@ -43,6 +43,9 @@ inline RecDim gd_rec_dim(int nr, int nlat2, bool fp64)
     if (l / line % 2 == 0) l += line;
     return RecDim{nr * l + (nr % 2 ? 0 : line), l, 1};
 }
+// the step's record orders, of FB and of GB
+inline RecDim gd_step_fb_dim(int nm, int nr) { return RecDim{1, (size_t)nm, (size_t)nm * nr}; }
+inline RecDim gd_step_gb_dim(int nlat2, int nr) { return RecDim{(size_t)nlat2 * nr, 1, (size_t)nr}; }
 // planes of products: nv tangential components in pairs, one vector array of
 // recs records each, then the scalars
 __host__ __device__ inline size_t gd_comp_off(int c, int nv, size_t recs)
@@ -88,15 +91,20 @@ struct AnaArgs {
     int mm;               // 1: BF16x3 split-precision contraction (FP32 operands), 0: native MFMA
 };
 
+// A real field F's four slots of a record are at fb + 4 nfield index + 4 F.  The
+// boundary passes write (RING_ANALYSIS) gb likewise; a step mode's product P is
+// at gb + gd_comp_off(P) + gd_comp_str(P) index.  The step modes' records are in
+// the orders gd_step_fb_dim and gd_step_gb_dim.
 struct RingArgs {
     const void *fb;       // T*
     void *gb;             // T*
     int nfield;           // real fields to synthesise (SYNTH/STEP) or analyse (ANALYSIS)
-    // a real field's four slots of a record: fb + foff + index * fstr (16-byte
-    // aligned), a product's: gb + goff + index * gstr
-    size_t foff[16], goff[5];
-    RecDim fdim, gdim;
-    int fstr, gstr[5];
+    RecDim dim;           // record order of a boundary pass
+    // 4 F of a boundary synthesis' field F, an argument: with the constant the
+    // compiler holds the first stage in fewer registers and then orders the next
+    // stage's loads behind its LDS reads (FP32 vector 384 x 768, 97 levels: 160
+    // -> 167 us)
+    size_t foff[2];
     const double *phys_in[2];
     double *phys_out[2];
     const void *tw;       // T2[nlon], e^{-2 pi i k / nlon}
@@ -146,11 +154,12 @@ template <typename T> int gd_launch_ring(hipStream_t st, int mode, const RingArg
     GD_RING_LEN(243) GD_RING_LEN(256) GD_RING_LEN(288) GD_RING_LEN(324) GD_RING_LEN(384) GD_RING_LEN(432)        \
     GD_RING_LEN(486) GD_RING_LEN(512) GD_RING_LEN(576) GD_RING_LEN(648) GD_RING_LEN(729) GD_RING_LEN(768)
 bool gd_ring_compiled(int nlon);
-// offsets along m fit 32 bits (the compiled plans' addresses)
-inline bool gd_offsets_fit(const RingArgs &a)
+// offsets along m fit 32 bits (the compiled plans' addresses): of a boundary
+// pass, of a step mode
+inline bool gd_offsets_fit(const RingArgs &a) { return (a.mmax + 1) * a.dim.m * 8 < (size_t)1 << 31; }
+inline bool gd_step_offsets_fit(const RingArgs &a)
 {
-    const size_t lim = (size_t)1 << 31, nm = a.mmax + 1;
-    return nm * a.fdim.m * a.fstr < lim && nm * a.gdim.m * 8 < lim;
+    return (a.mmax + 1) * gd_step_gb_dim(a.nlat2, a.nr).m * 8 < (size_t)1 << 31;
 }
 // a dealiased grid (the middle third of the orders is unused): instances of
 // the compiled plans of their own

@@ -210,8 +210,7 @@ static void base_args(gd_step *s, SynthArgs &a, RingArgs &r, AnaArgs &g)
     r = RingArgs{};
     gd_sht_fill_ring(p, r, nr);
     const size_t nm = p->mmax + 1;
-    a.dim = r.fdim = RecDim{1, nm, nm * nr};             // FB[i][level][m]
-    r.gdim = RecDim{(size_t)p->nlat2 * nr, 1, (size_t)nr}; // GB[m][i][level]
+    a.dim = gd_step_fb_dim((int)nm, nr);
     a.plane = 8;
     r.fb = s->fb.p;
     r.gb = s->gb.p;
@@ -220,8 +219,8 @@ static void base_args(gd_step *s, SynthArgs &a, RingArgs &r, AnaArgs &g)
     g = AnaArgs{};
     g.mm = p->prec == GD_PREC_BF16X3;
     g.gb = s->gb.p;
-    g.plane = 8 * nm * r.gdim.m;
-    g.dim = r.gdim;
+    g.dim = gd_step_gb_dim(p->nlat2, nr);
+    g.plane = 8 * nm * g.dim.m;
     g.moff = p->d_moff.as<int>();
     g.ne = p->d_ne.as<int>();
     g.l_of_idx = p->d_l_of_idx.as<int>();
@@ -231,22 +230,13 @@ static void base_args(gd_step *s, SynthArgs &a, RingArgs &r, AnaArgs &g)
     g.mmax = p->mmax;
 }
 
-// The fields of a ring pass side by side in FB's records of 4 nf slots, and its
-// np products (npv of them tangential components): vector and scalar products
-// in arrays of their own so that neither analysis reads the other's slots
-static void ring_slots(gd_step *s, SynthArgs &a, RingArgs &r, int nf, int np, int npv)
+// The fields of a ring pass side by side in FB's records of 4 nf slots; its
+// products, vector and scalar ones in arrays of their own so that neither
+// analysis reads the other's slots: here the scalar ones, after npv tangential
+// components
+static const void *scalar_products(const gd_step *s, int npv)
 {
-    r.nfield = nf;
-    r.fstr = a.rstr = 4 * nf;
-    for (int F = 0; F < nf; ++F) r.foff[F] = 4 * F;
-    for (int P = 0; P < np; ++P) {
-        r.goff[P] = gd_comp_off(P, npv, (s->sht.mmax + 1) * r.gdim.m);
-        r.gstr[P] = gd_comp_str(P, npv);
-    }
-}
-
-static const void *scalar_products(const gd_step *s, size_t off)
-{
+    const size_t off = gd_comp_off(npv, npv, (size_t)(s->sht.mmax + 1) * s->sht.nlat2 * s->d.nr);
     if (s->d.prec == GD_PREC_FP64) return s->gb.as<double>() + off;
     return s->gb.as<float>() + off;
 }
@@ -277,8 +267,8 @@ static void tang_args(gd_step *s, double *nl_out, SynthArgs &a, RingArgs &r, Ana
     // with composition the ring also takes grad C (fields 4, 5) and forms
     // -u.grad C (compute_composition_nonlinear!, compositional.jl:219-260)
     // as a fourth product
-    if (s->comp) ring_slots(s, a, r, 6, 4, 2);
-    else ring_slots(s, a, r, 4, 3, 2);
+    r.nfield = s->comp ? 6 : 4;
+    a.rstr = 4 * r.nfield;
     *mode = s->comp ? RING_STEP_TANG_C : RING_STEP_TANG;
     // force -> (pol, tor) of velocity nl (velocity.jl:331); the magnetic nl
     // is u x B = 0 here and its planes stay zero
@@ -291,7 +281,7 @@ static void tang_args(gd_step *s, double *nl_out, SynthArgs &a, RingArgs &r, Ana
     gv.scale[0] = 0;
     gv.scale[1] = 0;
     gs = g;
-    gs.gb = scalar_products(s, r.goff[2]);
+    gs.gb = scalar_products(s, 2);
     gs.plane = g.plane / 2;
     gs.nf = 1;
     gs.tab0 = gd_sht_tab(p, 0);
@@ -357,7 +347,8 @@ template <typename T> static int nonlinear_T(gd_step *s, double *nl_out, hipEven
         // vector fields u, omega, B, j (S,T) and grad T (S only)
         // FB: the five vector fields, then u_r, omega_r, B_r, j_r, dT/dr; GB: the
         // force, u x B, then -u.grad T
-        ring_slots(s, a, r, 15, 5, 4);
+        r.nfield = 15;
+        a.rstr = 60;
         a.nf = 5;
         static const int vmap[20] = {0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16, 17, -1, -1};
         for (int k = 0; k < 20; ++k) a.colmap[k] = vmap[k];
@@ -376,7 +367,7 @@ template <typename T> static int nonlinear_T(gd_step *s, double *nl_out, hipEven
             a.nf = 1;
             for (int k = 0; k < 20; ++k) a.colmap[k] = k < 2 ? 8 + k : -1;
         }
-        a.out = s->fb.as<T>() + r.foff[s->d.radials ? 10 : 14];
+        a.out = s->fb.as<T>() + (s->d.radials ? 40 : 56);
         a.plane = 4;
         GD_TRY(gd_launch_synth_scal<T>(st, a));
         GD_MARK(3);
@@ -396,7 +387,7 @@ template <typename T> static int nonlinear_T(gd_step *s, double *nl_out, hipEven
         g.scale[3] = 2;
         GD_TRY(gd_launch_ana<T>(st, g, true, maxgroup));
         GD_MARK(5);
-        g.gb = scalar_products(s, r.goff[4]);
+        g.gb = scalar_products(s, 4);
     }
     g.nf = 1;
     g.tab0 = gd_sht_tab(p, 0);

@@ -273,15 +273,21 @@ template <typename T, bool VEC, int NF, int NW, int KC, int NG = 0> constexpr si
     return 128 + sizeof(T) * (pipe > tile ? pipe : tile);
 }
 
-// The block's output tile -- per plane and level the records of TM consecutive
-// nodes -- is staged in LDS and stored as 16-byte vectors of those runs.
+// The block's output tile is staged in LDS in the order of the records it is
+// stored to, as 16-byte vectors: the step's, the fields side by side in a record
+// (plane = PS), [node][level][slot]; with NODE (one field, nodes the records'
+// fastest index) [level][node][slot].  Every divisor of the store is a constant:
+// one loop for both orders, with the order read at run time, took 120 us where
+// this takes 111 (batched step, six shells of lmax 63, 65 levels, FP64), 71
+// against 64 (FP32, tile 1).
 // blk, nblk: the block's index and the block count of this synthesis (the
 // launch's own, or its share of a batched launch over several shells)
-template <typename T, bool VEC, int NF, int NW, int KC, bool VL, int NG, int MM, class AT>
+template <typename T, bool VEC, int NF, int NW, int KC, bool VL, int NG, int MM, bool NODE, class AT>
 __device__ __forceinline__ void synth_body(const AT &a, int blk, int nblk)
 {
     static_assert(!MM || sizeof(T) == 4, "the BF16x3 contraction takes FP32 operands");
     using TL = SynthTile<VEC, NF, NW, NG>;
+    static_assert(!NODE || TL::PL == 1, "node-fastest records hold one field");
     constexpr int NT = TL::NT, VC = TL::VC, LT = TL::LT, RS = TL::RS;
     extern __shared__ __align__(16) char smem_raw[];
     int *scol = reinterpret_cast<int *>(smem_raw);
@@ -307,8 +313,10 @@ __device__ __forceinline__ void synth_body(const AT &a, int blk, int nblk)
     synth_pipeline<T, VEC, NF, NW, KC, VL, NG, MM>(a, in, tab0, tab1, sA, scol, m, i0, r0, accE, accO);
     __syncthreads(); // the tile below reuses the pipeline's LDS
 
-    T *tile = sA; // [plane][level][node][slot]
-    auto rec = [&](int pl, int il, int lv_) { return tile + ((pl * LT + lv_) * TM + il) * TL::PS; };
+    T *tile = sA;
+    auto rec = [&](int pl, int il, int lv_) {
+        return tile + (NODE ? lv_ * TM + il : il * LT + lv_) * RS + pl * TL::PS;
+    };
     const int vcol = wave * 16 + (lane & 15);
     int lv, fv;
     TL::decode(vcol, lv, fv);
@@ -369,34 +377,20 @@ __device__ __forceinline__ void synth_body(const AT &a, int blk, int nblk)
     T *out = static_cast<T *>(a.out);
     for (int t = tid; t < NV; t += 64 * NW) {
         const int e = t * EV;
-        // lanes along the records' runs: consecutive nodes of a (field, level), or
-        // the fields and levels side by side
-        int pl, l2, il, so;
-        if (a.dim.i == 1) {
-            const int run = e / (TM * TL::PS), w = e - run * (TM * TL::PS);
-            pl = run / LT;
-            l2 = run - pl * LT;
-            il = w / TL::PS;
-            so = w - il * TL::PS;
-        } else {
-            const int run = e / RS, w = e - run * RS;
-            il = run / LT;
-            l2 = run - il * LT;
-            pl = w / TL::PS;
-            so = w - pl * TL::PS;
-        }
+        const int q = e / RS, so = e - q * RS;
+        const int il = NODE ? q % TM : q / LT, l2 = NODE ? q / TM : q % LT;
         const int i = i0 + il, r = r0 + l2;
         if (i < a.nlat2 && r < a.nr) {
-            T *dst = out + pl * a.plane + (m * a.dim.m + r * a.dim.l + i * a.dim.i) * a.rstr + so;
-            *reinterpret_cast<V *>(dst) = *reinterpret_cast<const V *>(rec(pl, il, l2) + so);
+            T *dst = out + (m * a.dim.m + r * a.dim.l + i * (NODE ? 1 : a.dim.i)) * a.rstr + so;
+            *reinterpret_cast<V *>(dst) = *reinterpret_cast<const V *>(tile + e);
         }
     }
 }
 
-template <typename T, bool VEC, int NF, int NW, int KC, bool VL, int NG = 0, int MM = 0>
+template <typename T, bool VEC, int NF, int NW, int KC, bool VL, int NG, int MM, bool NODE>
 __global__ void __launch_bounds__(64 * NW) synth_kernel(SynthArgs a)
 {
-    synth_body<T, VEC, NF, NW, KC, VL, NG, MM>(a, blockIdx.x, gridDim.x);
+    synth_body<T, VEC, NF, NW, KC, VL, NG, MM, NODE>(a, blockIdx.x, gridDim.x);
 }
 
 // one grid over the syntheses of several shells (a batched step)
@@ -405,22 +399,27 @@ __global__ void __launch_bounds__(64 * NW) synth_batch_kernel(BatchRef<SynthArgs
 {
     const int sh = b.shell_of_block[blockIdx.x];
     if (sh == BATCH_PAD) return;
-    synth_body<T, VEC, NF, NW, KC, VL, NG, MM>(batch_args(b, sh), blockIdx.x - b.block_off[sh], b.block_cnt[sh]);
+    synth_body<T, VEC, NF, NW, KC, VL, NG, MM, false>(batch_args(b, sh), blockIdx.x - b.block_off[sh], b.block_cnt[sh]);
 }
 
 } // namespace
 
-template <typename T, bool VEC, int NF, int NW, int KC, int NG, int MM>
+template <typename T, bool VEC, int NF, int NW, int KC, int NG, int MM, bool NODE = false>
 static void launch_synth_mm(hipStream_t st, const SynthArgs &a)
 {
+    if constexpr (!NODE && NF == 1 && NG == 0)
+        if (a.dim.i == 1) {
+            launch_synth_mm<T, VEC, NF, NW, KC, NG, MM, true>(st, a);
+            return;
+        }
     using TL = SynthTile<VEC, NF, NW, NG>;
     dim3 grid(((a.nlat2 + TM - 1) / TM) * ((a.nr + TL::LT - 1) / TL::LT) * (a.mmax + 1));
     constexpr size_t lds = synth_lds_bytes<T, VEC, NF, NW, KC, NG>();
     // 16-byte table loads need every node row and tile start 16-byte aligned
     if (a.nlat2 % 4 == 0 && ((uintptr_t)a.tab0 % 16) == 0 && ((uintptr_t)a.tab1 % 16) == 0)
-        hipLaunchKernelGGL((synth_kernel<T, VEC, NF, NW, KC, true, NG, MM>), grid, dim3(64 * NW), lds, st, a);
+        hipLaunchKernelGGL((synth_kernel<T, VEC, NF, NW, KC, true, NG, MM, NODE>), grid, dim3(64 * NW), lds, st, a);
     else
-        hipLaunchKernelGGL((synth_kernel<T, VEC, NF, NW, KC, false, NG, MM>), grid, dim3(64 * NW), lds, st, a);
+        hipLaunchKernelGGL((synth_kernel<T, VEC, NF, NW, KC, false, NG, MM, NODE>), grid, dim3(64 * NW), lds, st, a);
 }
 
 // a.mm = 1: the BF16x3 contraction (FP32 operands only)
@@ -442,6 +441,7 @@ template <typename T> int gd_launch_synth_vec(hipStream_t st, const SynthArgs &a
     GD_CHECK((a.ng == 0 && (a.nf == 1 || a.nf == 2 || a.nf == 3 || a.nf == 5)) || (a.nf == 1 && (a.ng == 1 || a.ng == 2)) ||
                  (a.nf == 2 && a.ng == 1),
              GD_ERR_ARG, "synth_vec: nf=%d ng=%d", a.nf, a.ng);
+    GD_CHECK(a.nf + a.ng == 1 || a.plane == 8, GD_ERR_ARG, "synth_vec: fields %zu elements apart, not side by side", a.plane);
     if (gd_launch_synth_reg<T>(st, a, true)) return gd_check_launch("synth_reg_kernel<vec>");
     // one full field with 1 or 2 gradient fields: 6 columns per level (two
     // levels per 12-column group, 3 waves = 8 levels) or 8 (4 waves = 8 levels)
@@ -458,7 +458,7 @@ template <typename T> int gd_launch_synth_vec(hipStream_t st, const SynthArgs &a
 template <typename T> int gd_launch_synth_scal(hipStream_t st, const SynthArgs &a)
 {
     GD_CHECK(!a.mm || sizeof(T) == 4, GD_ERR_ARG, "synth_scal: the BF16x3 contraction takes FP32 operands");
-    GD_CHECK(a.nf == 1 || a.nf == 5, GD_ERR_ARG, "synth_scal: nf=%d (1 or 5)", a.nf);
+    GD_CHECK(a.nf == 1 || (a.nf == 5 && a.plane == 4), GD_ERR_ARG, "synth_scal: nf=%d (1 or 5, side by side)", a.nf);
     if (gd_launch_synth_reg<T>(st, a, false)) return gd_check_launch("synth_reg_kernel<scal>");
     if (a.nf == 5) launch_synth<T, false, 5, 5, 16>(st, a);
     else launch_synth<T, false, 1, 1, 16>(st, a);
@@ -518,7 +518,7 @@ template int gd_launch_synth_tang_batch<double>(hipStream_t, const BatchRef<Synt
 template <typename T> int gd_launch_synth_tang_tile(hipStream_t st, const SynthArgs &a, int tile)
 {
     GD_CHECK(gd_synth_tile_ok(tile, sizeof(T) == 8), GD_ERR_ARG, "synth: tile %d", tile);
-    GD_CHECK(a.nf == 1 && a.ng == 1, GD_ERR_ARG, "synth tile: the tangential form (nf=1, ng=1)");
+    GD_CHECK(a.nf == 1 && a.ng == 1 && a.plane == 8, GD_ERR_ARG, "synth tile: the tangential form (nf=1, ng=1)");
     if (tile == 0) launch_synth<T, true, 1, 3, 16, 1>(st, a);
     else if (tile == 1) launch_synth<T, true, 1, 3, 32, 1>(st, a);
     else if constexpr (sizeof(T) == 4) launch_synth<T, true, 1, 6, 16, 1>(st, a);
@@ -531,7 +531,7 @@ template int gd_launch_synth_tang_tile<double>(hipStream_t, const SynthArgs &, i
 // its own launch, and the 16-byte table form (VL) that the batched kernel has
 int gd_synth_tang_batchable(const SynthArgs &a)
 {
-    GD_CHECK(a.nf == 1 && a.ng == 1, GD_ERR_ARG, "synth batch: nf=%d ng=%d", a.nf, a.ng);
+    GD_CHECK(a.nf == 1 && a.ng == 1 && a.plane == 8, GD_ERR_ARG, "synth batch: nf=%d ng=%d", a.nf, a.ng);
     GD_CHECK(a.nlat2 % 4 == 0 && (uintptr_t)a.tab0 % 16 == 0 && (uintptr_t)a.tab1 % 16 == 0, GD_ERR_ARG,
              "synth batch: nlat/2=%d needs 16-byte table rows", a.nlat2);
     return GD_OK;

@@ -293,7 +293,12 @@ int node_tile(int nk) { return nk <= 32 ? 32 : nk <= 48 ? 48 : nk <= 64 ? 64 : n
 template <typename T, bool VEC> void launch_ana(hipStream_t st, const AnaArgs &a, int blocks)
 {
     if (a.accum) {
-        launch_kn<T, VEC, ANA_MAX, true>(st, a, blocks);
+        // the last chunk's remainder seldom needs all ANA_MAX nodes.  Both chunks,
+        // us, the second with 192 against 96: scalar, 288 nodes, lmax 383, 9 levels
+        // FP32 107 - 86, FP64 130 - 101; vector, 33 levels FP32 351 - 288, FP64 554 -
+        // 436 (chunks of 96 throughout, with the tables in LDS: 90, 164, 425, 1024)
+        if (a.nk <= 96) launch_kn<T, VEC, 96, true>(st, a, blocks);
+        else launch_kn<T, VEC, ANA_MAX, true>(st, a, blocks);
         return;
     }
     switch (node_tile(a.nk)) {

@@ -249,7 +249,10 @@ template <typename T> bool gd_launch_synth_reg(hipStream_t st, const SynthArgs &
     // Columns of more than 128 degrees per parity (8 groups of re and im) do not
     // fit the registers of two FP32 waves or one FP64 wave per SIMD, a column's
     // last loads need four values, and FP64 scalars of more than 64 degrees per
-    // parity are as fast in the LDS form (lmax 255: 140 us against 142).
+    // parity are faster in the LDS form (us, against this one: lmax 150, 65 levels
+    // 34 - 37; lmax 190, 17 / 33 / 66 levels 24 - 31, 33 - 38, 51 - 61; lmax 222,
+    // 34 levels 48 - 56; lmax 255, 33 / 97 levels 58 - 61, 150 - 153; below, lmax
+    // 130, 33 levels 20.5 - 20.0).
     // degrees of order 0: nlm = sum over m of (lmax + 1 - m)
     const int nm = a.mmax + 1, k0 = (a.nlm + a.mmax * nm / 2) / nm, ng = ((k0 + 1) / 2 + 15) / 16;
     if (ng > 8 || a.nlm < 4 || (sizeof(T) == 8 && !vec && ng > 4)) return false;

@@ -1,6 +1,6 @@
 """The step's nonlinear terms and the transposed ones over ring lengths with
 and without a compiled plan, with orders up to the Nyquist limit, against the
-FP64 oracle: tangential, full, and with composition.
+FP64 oracle: tangential and full (with composition: test_gpu_ring_step_composition.py).
 
 Tolerances, relative to each field's largest value: those of the step's own
 parity tests, 1e-10 in FP64 and 1e-4 in FP32 (products of fields whose curls

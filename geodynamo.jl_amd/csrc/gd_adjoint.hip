@@ -370,7 +370,6 @@ static int nonlinear_adjoint_T(gd_step *s, const double *xs, const double *mu, d
     g.nf = 2;
     g.moff = p->d_moff.as<int>();
     g.ne = p->d_ne.as<int>();
-    g.l_of_idx = p->d_l_of_idx.as<int>();
     g.nlat2 = p->nlat2;
     g.nr = nr;
     g.nlm = nlm;
@@ -808,7 +807,6 @@ extern "C" int gd_adjoint_misfit(gd_adjoint *a, int kind, int level, const doubl
     g.nf = 1;
     g.moff = p->d_moff.as<int>();
     g.ne = p->d_ne.as<int>();
-    g.l_of_idx = p->d_l_of_idx.as<int>();
     g.nlat2 = p->nlat2;
     g.nr = 1;
     g.nlm = nlm;

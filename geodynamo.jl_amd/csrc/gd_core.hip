@@ -169,7 +169,6 @@ void LmMaps::build(int lmax_, int mmax_)
     moff.assign(mmax + 2, 0);
     ne.assign(mmax + 1, 0);
     lmaj_of_idx.assign(nlm, 0);
-    idx_of_lmaj.assign(nlm, 0);
     l_of_idx.assign(nlm, 0);
     m_of_idx.assign(nlm, 0);
     // l-major offsets (shtnskit_transforms.jl:177-188)
@@ -184,7 +183,6 @@ void LmMaps::build(int lmax_, int mmax_)
             for (int l = m + par; l <= lmax; l += 2) {
                 int lm = loff[l] + m;
                 lmaj_of_idx[idx] = lm;
-                idx_of_lmaj[lm] = idx;
                 l_of_idx[idx] = l;
                 m_of_idx[idx] = m;
                 ++idx;

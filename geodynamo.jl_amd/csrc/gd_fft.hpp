@@ -344,3 +344,60 @@ template <typename T> __device__ __forceinline__ RingRec<T> fft_split(C2<T> Z, C
     }
     return RingRec<T>{{(X.x + Y.x) * c, (X.y + Y.y) * c, (X.x - Y.x) * c, (X.y - Y.y) * c}};
 }
+
+// ---- which plan a step mode's pass runs
+constexpr int MAXC = 32; // complex values a thread holds across one stage's barrier
+constexpr int RING_THREADS = 256; // ring_kernel block size
+__host__ __device__ constexpr int ring_ld(int n) { return n + (n >> 4) + 1; } // per-transform LDS stride
+
+// ---- compile-time plans: every divisor and twiddle stride is a constant
+constexpr int ct_next_radix(int n)
+{
+    return n % 8 == 0 ? 8 : n % 4 == 0 ? 4 : n % 6 == 0 ? 6 : n % 3 == 0 ? 3 : n % 2 == 0 ? 2 : 0;
+}
+constexpr int ct_nstages(int n)
+{
+    int s = 0;
+    while (n > 1) {
+        n /= ct_next_radix(n);
+        ++s;
+    }
+    return s;
+}
+constexpr int ct_radix(int n, int stage)
+{
+    for (int s = 0; s < stage; ++s) n /= ct_next_radix(n);
+    return ct_next_radix(n);
+}
+
+// Lengths whose tangential modes run ring_kernel's own compiled plan, not the
+// register plans: its blocks of 256 threads hold more waves.  us at 65 levels,
+// against the register plan: FP32 rings of 48 / 96 / 144 / 192 / 288 / 384 4.6
+// against 6.9, 6.7 - 8.6, 11.3 - 12.9, 14.4 - 17.2, 29.8 - 32.7, 36.8 - 39.0; FP64
+// 5.2 against 7.7, 11.0 - 11.6, 16.7 - 17.6, 24.0 - 30.4, 48.6 - 53.8, 70.7 - 69.4.
+// Beyond, at 33 levels (renumbered blocks): 432 FP32 33.2 against 31.4, FP64 56 -
+// 54, 576 FP32 55.7 - 51.6, FP64 103 - 99.5, 768 FP32 109 - 106, FP64 199 - 195.
+constexpr bool ring_short(int nlon) { return nlon % 48 == 0 && nlon <= 384; }
+
+// The 15-field step keeps ring_kernel's plan where the register plan takes three
+// stages, ring_kernel no more, and three of its blocks fit a CU's LDS.  us at 65
+// levels, against the register plan: FP32 384 119 - 127 (fits); FP64 384 342 - 260
+// and, at 33 levels, FP32 512 89 - 72 (do not fit); FP32 243, five stages, 74 - 47
+template <typename T> constexpr bool ring_step_own(int n)
+{
+    const size_t lds = sizeof(C2<T>) * ((size_t)ring_ld(n) * StepMode<RING_STEP>::NF + n);
+    return fft_stages(n).n == 3 && ct_nstages(n) <= 3 && 3 * lds <= 160 * 1024;
+}
+
+// what ring_check refuses of nf fields of n points, whichever plan would run:
+// more butterflies of a stage of ring_kernel's plan than its threads hold, or
+// more than ring_most_orders orders
+constexpr bool ring_fits(int nf, int n)
+{
+    for (int s = 0; s < ct_nstages(n); ++s) {
+        const int r = ct_radix(n, s);
+        if ((nf * (n / r) + RING_THREADS - 1) / RING_THREADS * r > MAXC) return false;
+    }
+    return true;
+}
+constexpr int ring_most_orders(int nf) { return 8 * RING_THREADS / nf; }

@@ -66,7 +66,6 @@ struct LmMaps {
     int lmax = 0, mmax = 0, nlm = 0;
     std::vector<int> moff, ne;          // mmax+2, mmax+1
     std::vector<int> lmaj_of_idx;       // device idx -> l-major lm
-    std::vector<int> idx_of_lmaj;       // l-major lm -> device idx
     std::vector<int> l_of_idx, m_of_idx;
     void build(int lmax_, int mmax_);
 };

@@ -354,7 +354,6 @@ static int run_analysis(gd_sht_plan *p, bool vec, const double *f0, const double
     a.nf = 1;
     a.moff = p->d_moff.as<int>();
     a.ne = p->d_ne.as<int>();
-    a.l_of_idx = p->d_l_of_idx.as<int>();
     a.nlat2 = p->nlat2;
     a.nr = nr;
     a.nlm = nlm;

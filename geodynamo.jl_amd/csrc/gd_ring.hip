@@ -82,12 +82,9 @@ template <int R, typename T> __device__ __forceinline__ void dftR(C2<T> *v, int 
     }
 }
 
-constexpr int MAXC = 32; // complex values a thread holds across one stage's barrier
-
 // LDS index skew: one pad slot per 16 complex values, so the stride-R writes
 // of the early Stockham stages (and stride-Ns groups later) spread over banks.
 __device__ __forceinline__ int sk(int e) { return e + (e >> 4); }
-__host__ __device__ constexpr int ring_ld(int n) { return n + (n >> 4) + 1; } // per-transform LDS stride
 
 // One Stockham stage over nfft transforms of length n (stride ld in buf); in
 // place, with every butterfly read before any is written.  Runtime radix plan.
@@ -147,28 +144,6 @@ __device__ void fft_batch(C2<T> *buf, const C2<T> *tw, int nfft, int n, int ld, 
         Ns *= R;
     }
 }
-
-// ---- compile-time plans: every divisor and twiddle stride is a constant
-constexpr int ct_next_radix(int n)
-{
-    return n % 8 == 0 ? 8 : n % 4 == 0 ? 4 : n % 6 == 0 ? 6 : n % 3 == 0 ? 3 : n % 2 == 0 ? 2 : 0;
-}
-constexpr int ct_nstages(int n)
-{
-    int s = 0;
-    while (n > 1) {
-        n /= ct_next_radix(n);
-        ++s;
-    }
-    return s;
-}
-constexpr int ct_radix(int n, int stage)
-{
-    for (int s = 0; s < stage; ++s) n /= ct_next_radix(n);
-    return ct_next_radix(n);
-}
-
-constexpr int RING_THREADS = 256; // ring_kernel block size
 
 // The Stockham write of a butterfly goes to idxD + r NS with idxD = q NS R + k,
 // k < NS.  sk(idxD + r NS) - sk(idxD) = r NS + [(idxD + r NS) / 16 - idxD / 16]
@@ -663,24 +638,6 @@ template <typename T, int MODE, int NC> static void ring_launch(hipStream_t st, 
     hipLaunchKernelGGL((ring_kernel<T, MODE, NC>), grid, dim3(RING_THREADS), lds, st, a);
 }
 
-// Lengths whose tangential modes run ring_kernel's own compiled plan, not the
-// register plans: its blocks of 256 threads hold more waves.  us at 65 levels,
-// against the register plan: FP32 rings of 48 / 96 / 144 / 192 / 288 / 384 4.6
-// against 6.9, 6.7 - 8.6, 11.3 - 12.9, 14.4 - 17.2, 29.8 - 32.7, 36.8 - 39.0; FP64
-// 5.2 against 7.7, 11.0 - 11.6, 16.7 - 17.6, 24.0 - 30.4, 48.6 - 53.8, 70.7 - 69.4.
-// Beyond, at 33 levels (renumbered blocks): 432 FP32 33.2 against 31.4, FP64 56 -
-// 54, 576 FP32 55.7 - 51.6, FP64 103 - 99.5, 768 FP32 109 - 106, FP64 199 - 195.
-static bool ring_short(int nlon) { return nlon % 48 == 0 && nlon <= 384; }
-
-// The 15-field step keeps ring_kernel's plan where the register plan takes three
-// stages, ring_kernel no more, and three of its blocks fit a CU's LDS.  us at 65
-// levels, against the register plan: FP32 384 119 - 127 (fits); FP64 384 342 - 260
-// and, at 33 levels, FP32 512 89 - 72 (do not fit); FP32 243, five stages, 74 - 47
-template <typename T> constexpr bool ring_step_own(int n)
-{
-    const size_t lds = sizeof(C2<T>) * ((size_t)ring_ld(n) * StepMode<RING_STEP>::NF + n);
-    return fft_stages(n).n == 3 && ct_nstages(n) <= 3 && 3 * lds <= 160 * 1024;
-}
 template <typename T> static bool ring_step_own_launch(hipStream_t st, dim3 grid, size_t lds, const RingArgs &a)
 {
     switch (a.nlon) {
@@ -716,7 +673,7 @@ static int ring_check(int mode, const RingArgs &a, int *nf_out)
     int nf = (mode == RING_STEP) ? 15 : (mode == RING_STEP_TANG) ? 4 : (mode == RING_STEP_TANG_C) ? 6
            : (mode == RING_ADJ_TANG) ? 7 : a.nfield;
     GD_CHECK(nf >= 1 && nf <= 15, GD_ERR_ARG, "ring: nfield=%d", nf);
-    GD_CHECK((long)nf * (a.mmax + 1) <= 8L * nthr, GD_ERR_ARG, "ring: %d fields x %d orders exceed one load batch",
+    GD_CHECK(a.mmax + 1 <= ring_most_orders(nf), GD_ERR_ARG, "ring: %d fields x %d orders exceed one load batch",
              nf, a.mmax + 1);
     for (int s = 0; s < a.nstages; ++s) {
         int R = a.radix[s];

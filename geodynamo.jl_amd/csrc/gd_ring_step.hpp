@@ -34,7 +34,11 @@ template <typename T, int MODE, int N> struct RingStepShape {
     using M = StepMode<MODE>;
     static constexpr int LD = FftRow<T, N>::ld(1);
     static constexpr size_t lds = sizeof(C2<T>) * LD * M::NF;
-    static constexpr bool ok = lds <= 160 * 1024;
+    // launched for this length and mode: its rings fit LDS, no plan of ring_kernel
+    // is preferred, and the 15 fields are not refused
+    static constexpr bool ok = lds <= 160 * 1024 &&
+        (MODE == RING_STEP ? ring_fits(M::NF, N) && !ring_step_own<T>(N) : !ring_short(N));
+    static constexpr bool deal_only = 3 * ring_most_orders(M::NF) <= N; // no more orders than a dealiased grid's
     static constexpr FftStages f = fft_stages(N);
     static constexpr int nthr = ring_step_threads(M::NF * (N / f.r[f.n - 1]), 512);
 };
@@ -216,7 +220,8 @@ template <typename T, int MODE, int N> bool ring_step_launch(hipStream_t st, con
     } else {
         const dim3 grid(a.nlat2 * a.nr), block(SH::nthr);
         if (gd_ring_deal(a)) hipLaunchKernelGGL((ring_step_plan_kernel<T, MODE, N, true>), grid, block, SH::lds, st, a);
-        else hipLaunchKernelGGL((ring_step_plan_kernel<T, MODE, N, false>), grid, block, SH::lds, st, a);
+        else if constexpr (!SH::deal_only) hipLaunchKernelGGL((ring_step_plan_kernel<T, MODE, N, false>), grid, block, SH::lds, st, a);
+        else return false;
         return true;
     }
 }
@@ -235,10 +240,14 @@ template <typename T, int MODE> bool ring_step_mode(hipStream_t st, const RingAr
 template <typename T, int N> bool ring_step_batch_launch(hipStream_t st, const BatchRef<RingArgs> &b, int nblocks, bool deal)
 {
     using SH = RingStepShape<T, RING_STEP_TANG, N>;
-    const dim3 grid(nblocks), block(SH::nthr);
-    if (deal) hipLaunchKernelGGL((ring_step_batch_kernel<T, RING_STEP_TANG, N, true>), grid, block, SH::lds, st, b);
-    else hipLaunchKernelGGL((ring_step_batch_kernel<T, RING_STEP_TANG, N, false>), grid, block, SH::lds, st, b);
-    return true;
+    if constexpr (!SH::ok) {
+        return false;
+    } else {
+        const dim3 grid(nblocks), block(SH::nthr);
+        if (deal) hipLaunchKernelGGL((ring_step_batch_kernel<T, RING_STEP_TANG, N, true>), grid, block, SH::lds, st, b);
+        else hipLaunchKernelGGL((ring_step_batch_kernel<T, RING_STEP_TANG, N, false>), grid, block, SH::lds, st, b);
+        return true;
+    }
 }
 
 template <typename T> bool ring_step_batch(hipStream_t st, const BatchRef<RingArgs> &b, int nblocks, int nlon, bool deal)

@@ -78,7 +78,7 @@ struct AnaArgs {
     RecDim dim;
     int nf;               // vector fields (components 2V, 2V+1) or scalar fields
     const void *tab0, *tab1;
-    const int *moff, *ne, *l_of_idx;
+    const int *moff, *ne;
     int nlat2, nr, nlm, mmax;
     int maxgroup;         // largest parity group, ceil((lmax+1)/2); set by gd_ana_plan
     // outputs, FP64 m-major [reim][level][idx]; vector field V: out[2V] gets S, out[2V+1] gets T

@@ -223,7 +223,6 @@ static void base_args(gd_step *s, SynthArgs &a, RingArgs &r, AnaArgs &g)
     g.plane = 8 * nm * g.dim.m;
     g.moff = p->d_moff.as<int>();
     g.ne = p->d_ne.as<int>();
-    g.l_of_idx = p->d_l_of_idx.as<int>();
     g.nlat2 = p->nlat2;
     g.nr = nr;
     g.nlm = nlm;

@@ -92,16 +92,22 @@ def kernel_costs(prec_bytes, tangential=True):
 
 
 # kernel of each class on the headline (tangential) path, as rocprofv3 names it
-# (synthesis: u and grad T as gradient fields, or, with GD_SYNTH_GRAD=0, as
-# full fields; CNAB2: one lane per column on the FP64 path, the twisted form
-# on the FP32-synthesis path, re and im columns paired in a lane by default)
-TANG_KERNELS = {"spectral_pre": "spectral_pre_kernel<{T}>",
-                "synth_vector": ("synth_kernel<{T}, true, 1, 3, 16, true, 1, 0>",
-                                 "synth_kernel<{T}, true, 2, 4, 16, true, 0, 0>"),
-                "ring_fft_products": "ring_kernel<{T}, 3, 384>", "analysis_vector": "ana_res_kernel<{T}, true, 1, 96, 0>",
-                "analysis_scalar": "ana_res_kernel<{T}, false, 1, 96, 0>",
+# (CNAB2: the twisted form with re and im columns paired in a lane by default,
+# the unpaired and the one-lane forms by switch)
+TANG_KERNELS = {"spectral_pre": ("spectral_pre_kernel<{T}>",),
+                "synth_vector": ("synth_reg_kernel<{T}, true, 4, 0>",),
+                "ring_fft_products": ("ring_kernel<{T}, 3, 384>",),
+                "analysis_vector": ("ana_kernel<{T}, true, 96, 0, false>",),
+                "analysis_scalar": ("ana_kernel<{T}, false, 96, 0, false>",),
                 "cnab2_solve": ("cnab2_chain_kernel<3, 4, {T}, true,", "cnab2_twist_kernel<3, 2, {T}, 2>",
                                 "cnab2_twist_kernel<3, 4, {T}, 1>")}
+
+
+def is_tang_kernel(cls, fp64, kernel):
+    """whether kernel (a rocprofv3 name) is one that the class launches"""
+    return any(p.format(T="double" if fp64 else "float") in kernel for p in TANG_KERNELS[cls])
+
+
 TRAFFIC_JSON = os.path.join(ROOT, "profiles", "pmc_step_lmax127_nr65.json")
 COPY_PROBE_BYTES = 268435456
 
@@ -111,7 +117,8 @@ def derive_traffic(prof_dir):
     of `bench.py --no-full --copy-probe 268435456` (FETCH_SIZE in
     prof_dir/fetch, WRITE_SIZE in prof_dir/write; KiB per dispatch), each
     scaled by what the counter reads for copy_kernel moving a known number of
-    bytes.  Writes TRAFFIC_JSON."""
+    bytes.  Writes TRAFFIC_JSON; every class must have its one kernel in both
+    runs."""
     import collections
     import csv
 
@@ -127,12 +134,12 @@ def derive_traffic(prof_dir):
     wscale = COPY_PROBE_BYTES / val["write"][copy]
     out = {"fetch_scale": round(fscale, 4), "write_scale": round(wscale, 4), "fp32": {}, "fp64": {}}
     for prec, T in (("fp32", "float"), ("fp64", "double")):
-        for cls, pat in TANG_KERNELS.items():
-            pats = pat if isinstance(pat, tuple) else (pat,)
-            ks = [k for k in val["fetch"] if any(p.format(T=T) in k for p in pats)]
-            if not ks:
-                continue
-            rd, wr = val["fetch"][ks[0]] * fscale, val["write"].get(ks[0], 0.0) * wscale
+        for cls in TANG_KERNELS:
+            ks = [k for k in val["fetch"] if is_tang_kernel(cls, prec == "fp64", k)]
+            if len(ks) != 1 or ks[0] not in val["write"]:
+                raise RuntimeError("%s %s: %d kernels of the counter runs match %s" % (
+                    prec, cls, len(ks), [p.format(T=T) for p in TANG_KERNELS[cls]]))
+            rd, wr = val["fetch"][ks[0]] * fscale, val["write"][ks[0]] * wscale
             out[prec][cls] = {"kernel": ks[0], "read_bytes": round(rd), "write_bytes": round(wr),
                               "hbm_bytes_per_launch": round(rd + wr)}
     with open(TRAFFIC_JSON, "w") as f:
@@ -155,6 +162,9 @@ def summarize_trace(prof_dir):
         for prec in ("fp32", "fp64"):
             for cls, rec in tj.get(prec, {}).items():
                 traffic[rec["kernel"]] = (cls, rec)
+    missing = sorted(set(traffic) - {r["Name"] for r in rows})
+    if missing:
+        raise RuntimeError("kernels of %s that the trace does not have: %s" % (TRAFFIC_JSON, missing))
     lines = ["| kernel | calls | avg us | min us | max us | class | HBM read MB | HBM write MB |",
              "|---|---|---|---|---|---|---|---|"]
     for r in sorted(rows, key=lambda r: -float(r["TotalDurationNs"])):
@@ -197,13 +207,14 @@ def roofline(prof_ms, prec):
     ridge = peak_f * 1e12 / (PEAK["hbm"] * 1e9)
     mfma = c["flops"] > 0 and c["flops"] / c["bytes"] > ridge
     # HBM bytes per launch from the committed rocprofv3 FETCH_SIZE / WRITE_SIZE
-    # runs (scaled by a copy kernel of known size), when they cover this kernel
+    # runs (scaled by a copy kernel of known size), when they are of the kernel
+    # that runs
     traffic = None
     pmc = TRAFFIC_JSON
     if os.path.exists(pmc):
         with open(pmc) as f:
             rec = json.load(f).get(prec, {}).get(name)
-        if rec:
+        if rec and is_tang_kernel(name, prec == "fp64", rec["kernel"]):
             traffic = round(rec["hbm_bytes_per_launch"])
     if mfma:
         ach = c["flops"] / t / 1e12

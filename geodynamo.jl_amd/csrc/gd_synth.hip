@@ -173,13 +173,13 @@ template <typename T, bool VEC, int MM> struct SynthWave {
 // 4 kq + j, and table rows are permuted so that register v of lane group g
 // holds node 4 g + v.
 //
-// Against blocks that staged tables and output tiles in LDS, 16 degrees and a
-// barrier at a time (us): 1691 vector instructions per 79 MFMA became 238 per
-// 60, and the step's u and grad T at lmax 127, 65 levels went FP32 45 -> 38,
-// FP64 82 -> 75 (MFMA 22); lmax 63 17.2 -> 12.6; all fields of the full step 119
-// -> 98 and 65 -> 57; FP32 vector lmax 255 231 -> 166; FP64 vector lmax 107 39 ->
-// 26.  Bound by the start of a wave and by
-// loads that wait behind a tile's stores, which the counter keeps in order.
+// Against blocks that stage tables and output tiles in LDS, 16 degrees and a
+// barrier at a time (us): the step's u and grad T at lmax 127, 65 levels FP32 45
+// -> 41, FP64 78 -> 71 (MFMA 22), lmax 63 16.4 -> 12.6 and 27 -> 19, lmax 15 7.2 ->
+// 4.8; u and grad T, C 56 -> 55 and 104 -> 107; all vector fields of the full step
+// 119 -> 103 and 244 -> 189; FP32 vector lmax 255, 97 levels 272 -> 167; FP64
+// vector lmax 107, 41 levels 37 -> 27.  Bound by the start of a wave and by loads
+// that wait behind a tile's stores, which the counter keeps in order.
 template <typename T, bool VEC, int KG, int MM>
 __global__ void __launch_bounds__(64, (sizeof(T) == 4 || KG <= 4 ? 2 : 1)) synth_reg_kernel(SynthArgs a, int ny, int tw)
 {
@@ -254,8 +254,12 @@ template <typename T> bool gd_launch_synth_reg(hipStream_t st, const SynthArgs &
     // 34 levels 48 - 56; lmax 255, 33 / 97 levels 58 - 61, 150 - 153; below, lmax
     // 130, 33 levels 20.5 - 20.0).
     // degrees of order 0: nlm = sum over m of (lmax + 1 - m)
+    // So are several FP64 scalars side by side in the step's records beyond 16
+    // degrees per parity: the LDS form stores their slots as one run, a lane here
+    // 32 bytes of it (five fields, 65 levels, lmax 47 / 95 / 127: 15.3 - 16.2, 58 -
+    // 60, 92 - 105; lmax 15: 6.0 - 5.2)
     const int nm = a.mmax + 1, k0 = (a.nlm + a.mmax * nm / 2) / nm, ng = ((k0 + 1) / 2 + 15) / 16;
-    if (ng > 8 || a.nlm < 4 || (sizeof(T) == 8 && !vec && ng > 4)) return false;
+    if (ng > 8 || a.nlm < 4 || (sizeof(T) == 8 && !vec && (ng > 4 || (ng > 1 && a.nf > 1)))) return false;
     // node tiles per wave: the runs that bring the grid nearest to 8192 waves
     // (order 0 has many times the degrees of the last ones, and a CU's first
     // waves wait for their columns).  Against 2048 waves, us: FP32 vector lmax

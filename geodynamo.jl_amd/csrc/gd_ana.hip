@@ -42,10 +42,10 @@ template <typename T> constexpr int ana_occ(int kn) { return sizeof(T) == 4 || k
 // blocks of one order are neighbours on one XCD (their records meet in its L2).
 //
 // Against a block of four waves with the tables in LDS, one slot per lane and
-// load, and node chunks of 96 (us): FP64 at lmax 127, 65 levels, vector 71 ->
-// 45 (MFMA floor with the tiles' padding 15); FP32 lmax 255, 97 levels, vector
-// 388 -> 218, of which 75 are MFMA; FP64 scalar there 236 -> 168 (40 MFMA); FP64
-// lmax 107, 41 levels, vector 55 -> 31.  What is left is the lanes' gather from
+// load, and node chunks of 96 (us): FP64 at lmax 127, 65 levels, vector 74 ->
+// 43 (MFMA floor with the tiles' padding 15); FP32 lmax 255, 97 levels, vector
+// 388 -> 216, of which 75 are MFMA; FP64 scalar there 236 -> 168 (40 MFMA); FP64
+// lmax 107, 41 levels, vector 46 -> 30.  What is left is the lanes' gather from
 // L1 (lanes of one level per 16- or 32-byte piece) and the start of a wave.
 template <typename T, bool VEC, int KN, int MM, bool ADD, class AT>
 __device__ __forceinline__ void ana_body(const AT &a, int blk, int nblk)

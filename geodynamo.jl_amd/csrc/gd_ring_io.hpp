@@ -5,9 +5,11 @@
 //
 // One block takes RG consecutive ring pairs (a northern ring and its southern
 // mirror, one complex transform each) of one level and NF fields.  The first
-// stage's butterflies load their inputs from global memory and the last
-// stage's store their results to it, so a point passes LDS only between
-// stages (one exchange for n <= 324, two beyond).  The grid arrays are
+// stage's butterflies load their inputs from global memory, and the synthesis'
+// last ones store the grid values to it, so a point crosses LDS only between
+// stages: once in plans of two stages (n <= 324, except 243), twice in plans of
+// three.  The analysis crosses once more: order m's slots need the results at m
+// and n - m.  The grid arrays are
 // colatitude-fastest: on their side lanes take the rings of one longitude
 // first, on the record side consecutive orders.  RG = 4 (32-byte runs of
 // colatitudes) where two blocks fit a CU's LDS, else 2.

@@ -371,7 +371,7 @@ constexpr int ct_radix(int n, int stage)
 }
 
 // Lengths whose tangential modes run ring_kernel's own compiled plan, not the
-// register plans: its blocks of 256 threads hold more waves.  us at 65 levels,
+// register plans.  us at 65 levels,
 // against the register plan: FP32 rings of 48 / 96 / 144 / 192 / 288 / 384 4.6
 // against 6.9, 6.7 - 8.6, 11.3 - 12.9, 14.4 - 17.2, 29.8 - 32.7, 36.8 - 39.0; FP64
 // 5.2 against 7.7, 11.0 - 11.6, 16.7 - 17.6, 24.0 - 30.4, 48.6 - 53.8, 70.7 - 69.4.
